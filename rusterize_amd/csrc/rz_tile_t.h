@@ -1246,14 +1246,20 @@ __global__ __launch_bounds__(256) void k_tile_heavy(TileArgs a) {
   uint64_t* mk = s_mk[wave];
   ItemDesc* ds = s_ds[wave];
   unsigned long long burns = 0;
-  uint32_t u = 0, u_end = 0;
+  // A wave's first units are its own share (no atomic), and the counter hands
+  // out those past every wave's share.  One atomic per wave to learn that no
+  // unit is left took 95 us a launch on its own (8,192 waves on one word,
+  // about 11.6 ns each); most launches have fewer units than waves.
+  const uint32_t first = gridDim.x * 4u * grab;
+  uint32_t u = min(units, (blockIdx.x * 4u + (uint32_t)wave) * grab), u_end = min(units, u + grab);
   for (;;) {
     if (u == u_end) {
+      if (first >= units) break;
       uint32_t g = 0;
       if (lane == 0) g = atomicAdd(a.heavy_ctr, grab);
-      u = (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
-      u_end = min(u + grab, units);
+      u = first + (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
       if (u >= units) break;
+      u_end = min(u + grab, units);
     }
     const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.heavy_list[h0 + (u >> 2)]);
     const int32_t strip = (int32_t)(u & 3u);
