@@ -9,6 +9,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "rz_kernels.h"
 
 namespace rzk {
@@ -46,6 +48,60 @@ __device__ inline double x86_nan(double r, double a, double b) {
 __device__ inline double crossing(const PolyEdge& e, int32_t r) {
   return e.x0 + (((double)r + 0.5) - e.y0) * e.dxdy;
 }
+
+// PolyEdge of the ring segment (x0, y0) -> (x1, y1) in pixel coordinates
+// (extract_ring + PolyEdge::new, edges.rs:27-46, 90-110), rows clamped to
+// nrows; true when the edge crosses a row.  xb is its lower end's x.  `odd`
+// is set when some row may end with an odd crossing count.  With `slope`
+// false the slope of an edge of finite ends is left 0 (edge_slope sets it).
+__device__ inline double edge_slope(double xt, double yt, double xb, double yb) {
+  // (yb - yt is neither NaN nor zero here)
+  const double dx = x86_nan(xb - xt, xb, xt);
+  return x86_nan(dx / (yb - yt), dx, 0.0);
+}
+__device__ inline bool ring_edge(double x0, double y0, double x1, double y1, int32_t nrows, bool slope, PolyEdge& e,
+                                 double& xb, double& yb, bool& odd) {
+  e = PolyEdge{0.0, 0.0, 0.0, 0, 0};
+  if (!(fabs(y0 - y1) >= 2.220446049250313e-16)) {  // edges.rs:100
+    // a skipped segment whose end points straddle a pixel-centre row (or are
+    // not numbers) leaves rows with an odd crossing count
+    if (isnan(y0) || isnan(y1) || ceil(fmin(y0, y1) - 0.5) != ceil(fmax(y0, y1) - 0.5)) odd = true;
+    return false;
+  }
+  if (!(fmin(y0, y1) < (double)nrows && fmax(y0, y1) >= 0.0)) return false;  // edges.rs:105
+  const bool down = y0 < y1;
+  e.x0 = down ? x0 : x1;
+  e.y0 = down ? y0 : y1;
+  xb = down ? x1 : x0;
+  yb = down ? y1 : y0;
+  e.ystart = sat_usize_cap(ceil(e.y0 - 0.5), nrows);
+  e.yend = sat_usize_cap(ceil(yb - 0.5), nrows);
+  const double inf = __builtin_inf();
+  const bool finite = fabs(e.x0) < inf && fabs(xb) < inf && fabs(e.y0) < inf && fabs(yb) < inf;
+  if (slope || !finite) {
+    e.dxdy = edge_slope(e.x0, e.y0, xb, yb);
+    // With a NaN x0 or slope, every crossing of the edge is NaN with that
+    // NaN's sign (x0's when both are NaN).  The reference sorts a positive
+    // NaN crossing last, where it closes an empty span or is the odd one out:
+    // as if it were absent, so the edge is emptied.  A negative one sorts
+    // first and spans from column 0, like -inf: the edge is pinned there.
+    if (isnan(e.x0) || isnan(e.dxdy)) {
+      if (signbit(isnan(e.x0) ? e.x0 : e.dxdy)) {
+        e.x0 = -inf;
+        e.y0 = 0.0;
+        e.dxdy = 0.0;
+      } else {
+        if (e.ystart < e.yend) odd = true;  // its rows lose one crossing each
+        e.ystart = e.yend = 0;
+      }
+    }
+  }
+  return e.ystart < e.yend;
+}
+
+// The wave's index in its workgroup, as a scalar (the compiler takes
+// threadIdx.x >> 6 for a value per lane, and all addresses made of it too).
+__device__ inline int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 // Orders a wave's LDS accesses around this point (wave-private buffers need
 // no workgroup barrier).
@@ -215,6 +271,41 @@ template <typename T> __device__ inline T from_bits(uint64_t b) {
 }
 
 
+// The new value of a pixel written once (the transitions of fold, k = 1).
+template <typename T, int FUN>
+__device__ inline T fold_value(T p, T v, T bg) {
+  return fold_select<T, FUN>(p, v, bg, true);
+}
+
+// ~0 when bit r (a constant) of x is set, else 0.  (In asm: written out, the
+// compiler turns the extract and the select below into a compare and a
+// conditional move.)
+__device__ __attribute__((always_inline)) inline int32_t bit_mask(uint32_t x, int r) {
+  int32_t m;
+  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(x), "n"(r));
+  return m;
+}
+
+// p where mask is 0, n where it is ~0 (bit select, no compare).
+template <typename T>
+__device__ inline T bit_select(int32_t mask, T n, T p) {
+  if constexpr (sizeof(T) == 8) {
+    uint2 a, b;
+    __builtin_memcpy(&a, &n, 8);
+    __builtin_memcpy(&b, &p, 8);
+    b.x = (a.x & (uint32_t)mask) | (b.x & ~(uint32_t)mask);
+    b.y = (a.y & (uint32_t)mask) | (b.y & ~(uint32_t)mask);
+    __builtin_memcpy(&p, &b, 8);
+  } else {
+    uint32_t a, b;
+    __builtin_memcpy(&a, &n, 4);
+    __builtin_memcpy(&b, &p, 4);
+    b = (a & (uint32_t)mask) | (b & ~(uint32_t)mask);
+    __builtin_memcpy(&p, &b, 4);
+  }
+  return p;
+}
+
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // XOR-combine a value across the four lanes of a quad with DPP quad
@@ -230,6 +321,26 @@ __device__ inline uint64_t quad_xor_all64(uint64_t x) {
 __device__ inline int32_t quad_max_all(int32_t x) {
   x = max(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));
   x = max(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));
+  return x;
+}
+
+// A workgroup barrier that orders LDS accesses only: global loads and stores
+// stay in flight across it (__syncthreads waits for all of them).
+__device__ inline void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Inclusive prefix sum over the wave with DPP row shifts and broadcasts
+// (VALU only: a shuffle of this chain waits on LDS at every step).
+__device__ inline uint32_t wave_prefix_sum(uint32_t x) {
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);   // row_shr:1
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);   // row_shr:2
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);   // row_shr:4
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);   // row_shr:8
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
   return x;
 }
 
@@ -270,9 +381,8 @@ __device__ inline uint32_t xcd_unit_lo(uint32_t x, uint32_t n) {
 template <int NWORD>
 __device__ inline uint64_t strip_coverage(const PolyEdge* ebase, uint32_t n_e, int32_t Rw,
                                           int32_t strip_r1, int32_t C0, double ncols_f,
-                                          PolyEdge* stage, int lane, int wq = -1) {
+                                          PolyEdge* stage, int lane) {
   const int rl = lane >> 2, q = lane & 3;
-  if (wq < 0) wq = q;  // the window word this lane returns (window from C0, NWORD words)
   const int32_t r = Rw + rl;
   const bool row_ok = r < strip_r1;
   uint64_t tog[NWORD];
@@ -314,16 +424,7 @@ __device__ inline uint64_t strip_coverage(const PolyEdge* ebase, uint32_t n_e, i
   amax = quad_max_all(amax);
 #pragma unroll
   for (int w = 0; w < NWORD; ++w) tog[w] = quad_xor_all64(tog[w]);
-  return wq < NWORD ? row_coverage_word<NWORD>(tog, lp, amax, C0, wq) : 0ull;
-}
-
-// Largest value of v (0..16) over the lanes of the wave, from five ballots.
-__device__ inline int32_t wave_max16(int32_t v) {
-  int32_t m = 0;
-#pragma unroll
-  for (int step = 16; step >= 1; step >>= 1)
-    if (__any(v >= m + step)) m += step;
-  return m;
+  return q < NWORD ? row_coverage_word<NWORD>(tog, lp, amax, C0, q) : 0ull;
 }
 
 }  // namespace rzk

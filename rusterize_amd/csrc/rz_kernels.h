@@ -1,20 +1,27 @@
 // rz_kernels.h -- gfx950 kernels of the rasteriser.
 //
 // Pipeline of one rasterise call or batch of calls (all on one HIP stream):
-//   k_prep        one thread per vertex: world->pixel transform, polygon edge
-//                 records (rust/src/geo/edges.rs:27-46, 90-110), line / point
-//                 pixel coordinates (edges.rs:79-88, 112-134) and a per-item
-//                 pixel bounding box (segmented wave reduction + atomics).
+//   k_prep        one thread per vertex: world->pixel transform, line / point
+//                 pixel coordinates (rust/src/geo/edges.rs:79-88, 112-134) and
+//                 a per-item pixel bounding box (segmented wave reduction +
+//                 atomics); polygon edge records (edges.rs:27-46, 90-110) only
+//                 where an item may end up without masks.
 //   k_item_desc   one thread per item: its descriptor (field value, band)
 //                 and tile count.
 //   scan / k_bin_emit / stable radix sort / k_tile_offsets / k_gather_desc
 //                 sort-middle binning of items into 64-row tiles, keeping
 //                 geometry order inside every tile.
+//   k_cover       the coverage masks of every polygon item, one bit per pixel
+//                 of its box, each edge's crossings computed once.
+//   (k_items      k_prep, k_item_desc and most of k_cover in one launch, for
+//                 calls of few polygons)
 //   k_tile        persistent work-queue kernel over 16-row tile strips: the
 //                 background fill of RasterInfo::build_raster
 //                 (rust/src/geo/raster.rs:23-28) and every burn of every item
 //                 of the strip, folded in geometry order in registers, then
-//                 written to HBM exactly once.
+//                 written to HBM exactly once; k_tile_block does the same with
+//                 a workgroup per tile for groups of few tiles, k_tile_lp with
+//                 the pixels in LDS for groups with lines or points.
 //
 // Exactness: all f64 arithmetic is compiled with -ffp-contract=off, divisions
 // and floor/ceil are IEEE exact, so every crossing and every pixel-centre
@@ -27,6 +34,21 @@
 
 namespace rzk {
 
+// Launches of polygon groups of at most this many tiles take a workgroup per
+// tile (k_tile_block), larger ones a wave per strip (k_tile): calls of 1,024
+// tiles took 36 us against 50, 4,096 tiles 131 against 138, 8,281 tiles 175
+// against 196 (float64), 11,900 tiles 207 against 231 (int32); 15,750 tiles
+// 299 against 273 where rows do not start on 64-byte lines (k_tile writes
+// whole lines), and 24,700 byte tiles 2012 against 1618.
+constexpr uint32_t kBlockTiles = 12288;
+// A call of at most this many polygons and vertices gets no masks either: the
+// few strips that meet an item compute its coverage from its edges, which
+// saves the mask kernels (32 convex polygons on 500 x 500: 18 us against 28;
+// 256 on 1000 x 1000: 22 against 30; 512 stars on 2000 x 2000: 31 against 30;
+// 300 polygons among 3,000 lines and 12,000 points: 309 against 339;
+// only where all of them meet the same few tiles are masks ahead, 25 against
+// 33 for 32 stars on 100 x 200).
+constexpr int64_t kBareItems = 512, kBareVerts = 4096;
 constexpr int TILE_H = 64;       // rows per tile (4 waves x 16 rows)
 constexpr int WAVE_ROWS = 16;    // rows per wave strip
 constexpr int NUM_XCD = 8;       // MI355X: 8 XCDs, workgroups dispatched round-robin
@@ -144,11 +166,10 @@ struct PrepArgs {
   const int64_t* job_vend;  // [n_jobs] prefix ends of the vertex ranges
   int n_jobs;
   int64_t n_vertices;       // batch total
-  PolyEdge* edges;          // [n_vertices]
+  PolyEdge* edges;          // [n_vertices], or null: every polygon has masks (k_cover reads xy)
   uint4* lseg;              // [n_vertices] segment / cell records of line and point vertices
   ItemBox* item_box;        // [n_items]
-  unsigned long long* item_last;  // [n_items] lines: last kept segment + 1 (global; 0: none);
-                                  // polygons: the sum over edges of the rows each crosses
+  unsigned long long* item_last;  // [n_items] lines: last kept segment + 1 (global; 0: none)
   unsigned long long* item_win;   // [8 n_items] all-touched sum / count polygons (or null): the f64
                                   // box of their kept outline segments (min x, min y, max x, max y as
                                   // ordered keys), then that of all their vertices (a NaN widens it
@@ -224,17 +245,15 @@ struct __align__(64) ItemDesc {
   uint64_t value;           // field value bits (dtype of the call)
   uint64_t last;            // lines: last kept segment + 1 (0: none; kItemFarBit masked off)
   uint32_t job;
-  uint32_t band;            // banded polygon or line item: first band entry + 1 (0: not banded)
+  uint32_t band;            // banded line item: first band entry + 1 (0: not banded)
   uint32_t flags;           // kItem* bits
-  uint32_t wide;            // kItemWide: first word of the item's row masks / 16
+  uint32_t mask;            // kItemMask: first word of the item's coverage masks / 16
 };
 
-// ItemDesc::flags.  kItemWide: the polygon's coverage is precomputed once
-// per 16-row strip over its whole column range (k_wide_cover) instead of in
-// every output tile it meets: for items several tiles wide with many edges
-// per strip, and for items of many short edges (which the pre-pass visits
-// edge by edge).
-constexpr uint32_t kItemWide = 1u;
+// ItemDesc::flags.  kItemMask: the polygon's coverage masks are precomputed
+// (k_cover); without it (a capacity was reached, or the allocation-free entry
+// point) the tile kernel computes the item's coverage strip by strip.
+constexpr uint32_t kItemMask = 1u;
 // kItemOddRows: some row of the polygon may have an odd crossing count (an
 // edge emptied for a positive-NaN slope or origin, or a segment skipped as
 // horizontal that straddles a pixel-centre row).  Only then does a row's
@@ -251,31 +270,25 @@ constexpr unsigned long long kItemOddBit = 1ull << 63;
 // ... and line items with a kLsFar segment in bit 62 (they are never banded).
 constexpr unsigned long long kItemFarBit = 1ull << 62;
 
-// Row masks of a kItemWide item: strip k (rows from (r0 / 16 + k) * 16) holds
-// 16 rows of nw = (c1 - 1) / 64 - c0 / 64 + 1 words each (word w covers
-// columns (c0 / 64 + w) * 64 .. + 63), at wide_masks[wide * 16 + (16 k + row)
-// * nw + w].  A unit of k_wide_cover is one strip of one item and at most
-// kWideWords words of it (a window).
-constexpr int kWideWords = 32;
+// Coverage masks of a kItemMask item: strip k (rows from (r0 / 16 + k) * 16)
+// and word w (columns (c0 / 64 + w) * 64 .. + 63) hold one block of 128 bytes
+// at masks[(mask + k * nw + w) * 16], nw = (c1 - 1) / 64 - c0 / 64 + 1: for
+// each column the bits of its 16 rows, column c at 16-bit element
+// mask_element(c).  A wave whose lanes stand for columns reads a block with
+// one 2-byte load per lane.
+__host__ __device__ inline int32_t mask_element(int32_t c) { return (c & 15) * 4 + (c >> 4); }
+__host__ __device__ inline int32_t mask_row_words(int32_t c0, int32_t c1) { return ((c1 - 1) >> 6) - (c0 >> 6) + 1; }
+__host__ __device__ inline int32_t mask_strip_count(int32_t r0, int32_t r1) { return (r1 - 1) / 16 - r0 / 16 + 1; }
 
-__host__ __device__ inline int32_t wide_row_words(int32_t c0, int32_t c1) { return ((c1 - 1) >> 6) - (c0 >> 6) + 1; }
-__host__ __device__ inline int32_t wide_strip_count(int32_t r0, int32_t r1) { return (r1 - 1) / 16 - r0 / 16 + 1; }
-
-// Edge bands: a polygon item with more than kBandMinEdges edges that spans
-// two or more 16-row strips gets its edges binned by strip (an edge goes to
-// every strip its rows [ystart, yend) meet), so a strip visits only its own
-// edges instead of the whole ring set.  Band entry
-// band - 1 + (Rw / kBandRows - r0 / kBandRows) of such an item holds the
-// edges of the strip starting at row Rw in
-// band_edges[band_off[e] .. band_off[e + 1]) (any order: the crossing
-// toggles and the maximum commute).
-// Line items with more than kLineBandMinSegs segments over two or more
-// strips (and no kLsFar segment) are banded the same way: a segment goes to
-// every strip the rows of its cells [min(iy0, iy1), max(iy0, iy1)] meet, as
-// a 16-byte segment record in band_segs[band_off[e] ..) whose flag marks the
-// end cell (any order: a line's writes all carry one value, so only their
-// number per pixel matters).
-constexpr int kBandMinEdges = 128;
+// Edge bands: a line item with more than kLineBandMinSegs segments over two
+// or more 16-row strips (and no kLsFar segment) gets its segments binned by
+// strip (a segment goes to every strip the rows of its cells
+// [min(iy0, iy1), max(iy0, iy1)] meet), so a strip visits only its own.  Band
+// entry band - 1 + (Rw / kBandRows - r0 / kBandRows) of such an item holds
+// the strip starting at row Rw as 16-byte segment records in
+// band_segs[band_off[e] .. band_off[e + 1]) whose flag marks the end cell
+// (any order: a line's writes all carry one value, so only their number per
+// pixel matters).
 constexpr int kLineBandMinSegs = 32;
 constexpr int kBandRows = WAVE_ROWS;
 
@@ -304,19 +317,66 @@ struct InitArgs {
   }
 };
 
+// k_cover's work, listed by k_item_desc.  A unit keeps the toggle words of
+// its rows in LDS (a row's words padded to an odd count against bank
+// conflicts, one more for the rightmost crossing of a kItemOddRows item):
+//   small  items of at most 64 vertices whose words fit kCoverWave, as many
+//          to a wave as fit together;
+//   wave   items of at most kCoverBlockNv vertices (a few chunks of 64, so
+//          reading them once per window costs little): windows of kCoverWave
+//          words, each a wave's work;
+//   block  all others: windows of kCoverBlock words, each a workgroup's work
+//          (a window reads all the item's edges: larger windows, fewer times).
+// A window is a run of whole strips by at most (words / 16 - 2) mask words.
+// Masks and list entries are handed out by counters, one atomic of each per
+// workgroup; their order does not matter.
+constexpr int kCoverWave = 448, kCoverBlock = 3840;
+constexpr int kCoverRun = 16;  // small items a wave takes at once
+constexpr int kCoverBlockNv = 320;
+struct CoverWindows {
+  int32_t ww, stride, strips;  // mask words, padded words and strips of a window
+  int32_t ncw, n;              // windows across, windows in all
+};
+__host__ __device__ inline CoverWindows cover_windows(int32_t ns, int32_t nw, bool odd, int32_t words) {
+  CoverWindows c;
+  c.ww = nw < words / 16 - 2 ? nw : words / 16 - 2;
+  c.stride = (c.ww + (odd ? 1 : 0)) | 1;
+  if (c.ww == nw && (int64_t)16 * c.stride * ns <= words) {  // (no divisions)
+    c.strips = ns;
+    c.ncw = c.n = 1;
+    return c;
+  }
+  c.strips = words / (16 * c.stride);
+  if (c.strips > ns) c.strips = ns;
+  c.ncw = (nw + c.ww - 1) / c.ww;
+  c.n = c.ncw * ((ns + c.strips - 1) / c.strips);
+  return c;
+}
+constexpr int kDescBlock = 512;  // threads of a k_item_desc workgroup
+struct CoverCounters {
+  unsigned long long mask_units;  // 16-word units of masks handed out
+  uint32_t n_small, n_wave, n_block, pad[11];
+};
+struct CoverLists {
+  CoverCounters* ctr;   // zero at launch
+  uint64_t mask_cap;    // 16-word units; items past a capacity get no masks
+  uint32_t unit_cap;    // entries of wave and of block
+  uint32_t* small;      // [n_items]
+  uint2* wave;          // [unit_cap] item, window
+  uint2* block;         // [unit_cap]
+};
+
 struct DescArgs {
   const JobDev* jobs;
   const int64_t* job_iend;  // [n_jobs] prefix ends of the item ranges
   int n_jobs;
   int64_t n_items;
   const ItemBox* item_box;
-  const unsigned long long* item_last;  // lines: last kept segment + 1; polygons: rows their edges cross
+  const unsigned long long* item_last;  // lines: last kept segment + 1
   ItemDesc* desc;           // [n_items]
   uint32_t* counts;         // [n_items] tiles per item, or null (no binned job)
-  uint32_t* band_n;         // [n_items] tile rows of a banded polygon item (0: not banded)
-  int wide_mode;            // wide pre-pass: 0 chosen per item, 1 never, 2 every polygon item
-  uint32_t* wide_units;     // [n_items] k_wide_cover units of a wide item (0: not wide), or null
-  uint32_t* wide_words;     // [n_items] row-mask words of a wide item
+  uint32_t* band_n;         // [n_items] strips of a banded line item (0: not banded)
+  CoverLists cover;         // the polygon items' masks and work lists (ctr null: no masks)
   uint32_t* status;         // bit 4 set when a geometry's layer index is >= the job's n_layers
   const unsigned long long* item_win;  // all-touched polygons' outline boxes (null: none)
   uint2* scan_box;          // [n_items] boxes of items of scan_compact jobs (or null), see ScanBox
@@ -337,39 +397,24 @@ struct AtCacheArgs {
   uint32_t* status;         // bit 64: a walk did not end
 };
 
-// Wide items within the capacities get their flag, mask base and unit list.
-struct WideAssignArgs {
-  ItemDesc* desc;
-  int64_t n_items;
-  const uint32_t* wide_units;
-  const uint64_t* unit_base;  // [n_items + 1] exclusive scan of wide_units
-  const uint64_t* word_base;  // [n_items + 1] exclusive scan of wide_words
-  uint64_t unit_cap, word_cap;
-  uint32_t* unit_item;        // [unit_cap] item of every unit
+// Arguments of k_items: k_item_desc's (no line or all-touched items), edge
+// records to write (or null) and the masks.
+constexpr int kItemsWaves = 8;
+constexpr int kCoverOwn = 4;          // wave windows of an item that its wave covers itself
+constexpr int64_t kItemsMax = 6144;   // items of a call that takes k_items: the waves that fit the
+                                      // chip (3 workgroups to a CU)
+struct ItemsArgs {
+  DescArgs d;
+  PolyEdge* edges;
+  uint64_t* masks;
 };
 
-struct WideCoverArgs {
+// Arguments of k_cover.
+struct CoverArgs {
   const JobDev* jobs;
-  const ItemDesc* desc;       // [n_items], wide fields assigned
-  int64_t n_items;
-  const uint32_t* unit_item;  // [units]
-  const uint64_t* unit_base;  // [n_items + 1]
-  const uint64_t* n_units;    // unit total (device side), clamped to unit_cap
-  uint64_t unit_cap;
-  const PolyEdge* edges;
-  const uint64_t* band_off;
-  const PolyEdge* band_edges;
-  uint64_t* wide_masks;
-  int cov_mode;               // layout per chunk of edges: 0 the cheaper, 1 row-major, 2 edge-major
-  // heavy tiles (null heavy_cnt: none): their items' masks also go to the
-  // heavy slots (see TileArgs), at the item's place in the tile's pair list
-  const uint32_t* heavy_cnt;  // [n_tiles] items of a heavy tile, 0 otherwise
-  const uint64_t* heavy_base;
-  const uint64_t* pair_off;   // [n_items + 1] an item's first pair in emission order
-  uint64_t pair_cap;          // pairs emitted at most (an item past it has none)
-  const uint32_t* wide_j;     // [pair_cap] by emission index: a wide item's place in a heavy tile
+  const ItemDesc* desc;  // [n_items], masks and lists assigned
+  CoverLists cover;
   uint64_t* masks;
-  uint32_t slot_words;
 };
 
 // Per-item edge-band build: one wave per item (grid-stride), counters of
@@ -381,12 +426,10 @@ struct BandArgs {
   const uint32_t* band_n;   // [n_items] strips of a banded item
   const uint32_t* items;    // [*n_list] the banded items with assigned entries
   const uint32_t* n_list;
-  const PolyEdge* edges;    // [n_vertices]
   const uint4* lseg;        // [n_vertices] line segment records
   uint32_t* band_cnt;       // [n_bands] edges per band entry (count pass)
   const uint64_t* band_off; // [n_bands + 1] exclusive scan of band_cnt (scatter pass)
-  PolyEdge* band_edges;     // [edge_cap] polygon entries (scatter pass), or null
-  uint4* band_segs;         // [edge_cap] line entries (scatter pass), or null
+  uint4* band_segs;         // [edge_cap] (scatter pass)
   uint64_t edge_cap;
   uint32_t* status;         // bit 3 set when the banded edges exceed edge_cap
 };
@@ -433,27 +476,12 @@ struct TileArgs {
   const uint32_t* tile_off;  // [n_tiles + 1], or null when no job is binned
   const ItemDesc* pair_desc;  // descriptors in pair order
   const uint2* scan_box;      // [n_items] compact boxes of scan_compact jobs' items
-  const uint64_t* band_off;   // edge bands of banded polygon and line items
-  const PolyEdge* band_edges;
+  const uint64_t* band_off;   // edge bands of banded line items
   const uint4* band_segs;
-  // heavy tiles: heavy_base[t] .. heavy_base[t + 1] index the tile's items in
-  // the pre-pass masks (null: no heavy tiles); slot_words u64 per strip mask,
-  // item j of tile t, strip s at slot heavy_base[t] * 4 + s * (items of t) + j
-  const uint64_t* heavy_base;
-  const uint64_t* masks;
-  uint32_t slot_words;
-  uint32_t heavy_min;       // items from which a tile is heavy
-  const uint64_t* wide_masks;  // row masks of kItemWide items (null: none)
-  // heavy tiles of polygon-only groups go to k_tile_heavy (heavy_split = 1):
-  // the heavy tiles in tile order, each tile's rank in that list, and the
-  // launch's work counter
-  int heavy_split;
-  const uint32_t* heavy_list;
-  const uint32_t* heavy_rank;  // [n_tiles + 1]
-  uint32_t* heavy_ctr;
+  const uint64_t* masks;      // coverage masks of kItemMask items
   // scan jobs: every item of the job is tested against the tile
   const ItemDesc* desc;
-  const PolyEdge* edges;
+  const PolyEdge* edges;    // read for polygon items without masks only
   const uint4* lseg;        // line / point vertex records (kLs*)
   // all-touched polygons with sum / count: outline boxes (PixelCache
   // windows) and, for those whose fill reaches beyond them, the PixelCache
@@ -467,28 +495,6 @@ struct TileArgs {
 };
 
 constexpr int kBurnSlots = 1024;
-
-// Items per tile from which a tile's polygon coverage is precomputed by the
-// k_cover pre-pass (see rz_tile.hip).
-constexpr uint32_t kHeavyItems = 32;
-
-struct CoverArgs {
-  const JobDev* jobs;
-  const int64_t* job_tend;
-  int n_jobs;
-  const uint32_t* pair_tile;    // [n_pairs] tile of every pair (sorted keys)
-  const ItemDesc* pair_desc;    // [n_pairs]
-  const uint64_t* heavy_base;   // [n_tiles + 1]
-  const uint32_t* cover_list;   // [*cover_count] pair indices of heavy polygon pairs
-  const uint32_t* cover_count;
-  uint32_t n_tiles;
-  const PolyEdge* edges;
-  const uint64_t* band_off;
-  const PolyEdge* band_edges;
-  const uint32_t* tile_off;     // [n_tiles + 1]
-  uint64_t* masks;              // [4 x heavy pairs][slot_words], strip-major per tile
-  uint32_t slot_words;
-};
 
 // ------------------------------------------------ polygon row coverage --
 //

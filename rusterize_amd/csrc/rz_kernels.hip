@@ -87,36 +87,47 @@ __global__ void k_fill_keys(uint32_t* keys, const uint64_t* n_pairs, uint64_t ca
 
 // ------------------------------------------------------------------ prep --
 
+// One step of a segmented scan: the box of the lane DPP control C reads is
+// merged if it belongs to the same item.
+template <int C, int R>
+__device__ inline void merge_box(int it, ItemBox& b) {
+  const bool same = __builtin_amdgcn_update_dpp(it, it, C, R, 0xF, false) == it;
+  const int r0 = __builtin_amdgcn_update_dpp(b.r0, b.r0, C, R, 0xF, false);
+  const int r1 = __builtin_amdgcn_update_dpp(b.r1, b.r1, C, R, 0xF, false);
+  const int c0 = __builtin_amdgcn_update_dpp(b.c0, b.c0, C, R, 0xF, false);
+  const int c1 = __builtin_amdgcn_update_dpp(b.c1, b.c1, C, R, 0xF, false);
+  if (same) {
+    b.r0 = min(b.r0, r0);
+    b.r1 = max(b.r1, r1);
+    b.c0 = min(b.c0, c0);
+    b.c1 = max(b.c1, c1);
+  }
+}
+
 // Segmented (by item) min/max reduction across the wave, then one set of
 // atomics per item segment.  Items own contiguous vertex ranges, so lanes of
-// one item are contiguous.  `stat` is item_last's contribution: polygon
-// lanes add the rows their edge crosses (saturating: a ranking statistic
-// only), line lanes take the maximum of (kept segment + 1).  An item has one
-// kind, so every segment combines with one of the two.
-__device__ inline void reduce_box(int64_t item, ItemBox b, uint64_t stat, bool line, ItemBox* out,
+// one item are contiguous.  `stat` is a line lane's kept segment + 1 (v + 1; 0: none
+// kept, and for polygon and point lanes), whose maximum goes to item_last.
+__device__ inline void reduce_box(int64_t v, int64_t item, ItemBox b, uint64_t stat, ItemBox* out,
                                   unsigned long long* last_out, bool active) {
   const int lane = threadIdx.x & 63;
-  int64_t it = active ? item : -1;
-  // polygon row sums saturate below 2^31: 32-bit shuffles unless a line
-  // vertex (a 64-bit vertex index) is in the wave
-  const bool any_line = __ballot(line) != 0;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int64_t oit = __shfl_up(it, off, 64);
-    int32_t r0 = __shfl_up(b.r0, off, 64), r1 = __shfl_up(b.r1, off, 64);
-    int32_t c0 = __shfl_up(b.c0, off, 64), c1 = __shfl_up(b.c1, off, 64);
-    const uint64_t ostat = any_line ? (uint64_t)__shfl_up(stat, off, 64)
-                                    : (uint64_t)(uint32_t)__shfl_up((int)(uint32_t)stat, off, 64);
-    if (lane >= off && oit == it) {
-      b.r0 = min(b.r0, r0);
-      b.r1 = max(b.r1, r1);
-      b.c0 = min(b.c0, c0);
-      b.c1 = max(b.c1, c1);
-      stat = line ? max(stat, ostat) : min(stat + ostat, (uint64_t)0x7FFFFFFFu);
-    }
+  // (items of one wave are neighbours, so their low halves tell them apart)
+  const int it = active ? (int)(uint32_t)(uint64_t)item : -1;
+  const uint64_t kept = __ballot(stat != 0);
+  merge_box<0x111, 0xF>(it, b);  // row_shr:1, 2, 4, 8
+  merge_box<0x112, 0xF>(it, b);
+  merge_box<0x114, 0xF>(it, b);
+  merge_box<0x118, 0xF>(it, b);
+  merge_box<0x142, 0xA>(it, b);  // lane 15 of a row into the next one
+  merge_box<0x143, 0xC>(it, b);  // lane 31 into the upper half
+  const bool head = lane == 0 || __builtin_amdgcn_update_dpp(0, it, 0x138, 0xF, 0xF, false) != it;  // wave_shr:1
+  const uint64_t heads = __ballot(head);
+  const bool tail = lane == 63 || ((heads >> 1) >> lane & 1ull);
+  if (kept && tail) {  // the item's last kept segment in this wave
+    const uint64_t upto = ~0ull >> (63 - lane);
+    const uint64_t mine = kept & upto & (~0ull << (63 - __builtin_clzll(heads & upto)));
+    stat = mine ? (uint64_t)(v - lane + 64 - __builtin_clzll(mine)) : 0ull;
   }
-  int64_t nit = __shfl_down(it, 1, 64);
-  bool tail = (lane == 63) || (nit != it);
   // A segment's box is merged whenever some edge set it, even when its own
   // column range is empty: a polygon edge left or right of the raster
   // clamps to an empty range, and the item's other edges, possibly in
@@ -127,9 +138,35 @@ __device__ inline void reduce_box(int64_t item, ItemBox b, uint64_t stat, bool l
     atomicMin(&out[item].c0, b.c0);
     atomicMax(&out[item].c1, b.c1);
   }
-  if (active && tail && stat) {
-    if (line) atomicMax(&last_out[item], (unsigned long long)stat);
-    else atomicAdd(&last_out[item], (unsigned long long)stat);
+  if (active && tail && stat) atomicMax(&last_out[item], (unsigned long long)stat);
+}
+
+// The edge (pixel coordinates x0, y0 to x1, y1) that starts at a polygon
+// vertex: its record (its slope only if asked for), the box of its crossings
+// and whether rows may be left with an odd crossing count.
+__device__ inline void polygon_edge(uint64_t vi, double x0, double y0, double x1, double y1, const RZ_CONST JobDev& J,
+                                    bool slope, PolyEdge& e, ItemBox& box, bool& odd) {
+  e = PolyEdge{0.0, 0.0, 0.0, 0, 0};
+  // a ring left open by the caller (its last coordinate is not its
+  // first) can leave rows with an odd crossing count
+  if ((vi & VI_RING_START) && !(vi & VI_CLOSED)) odd = true;
+  double xb, yb;
+  if ((vi & VI_HAS_NEXT) && ring_edge(x0, y0, x1, y1, J.nrows, slope, e, xb, yb, odd)) {
+    box.r0 = e.ystart;
+    box.r1 = e.yend;
+    // Crossings of this edge lie between its end points up to a few
+    // ulps, so their span columns are within one pixel of these.
+    const double ax = fabs(e.x0), bx = fabs(xb);
+    if (!(ax <= 1.0e12 && bx <= 1.0e12)) {
+      box.c0 = 0;
+      box.c1 = J.ncols;
+    } else {
+      const double cols = (double)J.ncols;
+      const double lo = floor(fmin(e.x0, xb) + 0.5) - 1.0;
+      const double hi = floor(fmax(e.x0, xb) + 0.5) + 1.0;
+      box.c0 = (int32_t)fmin(fmax(lo, 0.0), cols);
+      box.c1 = (int32_t)fmin(fmax(hi, 0.0), cols);
+    }
   }
 }
 
@@ -142,8 +179,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   const bool active = v < a.n_vertices;
   int64_t item = -1;
   ItemBox box{INT_MAX, INT_MIN, INT_MAX, INT_MIN};
-  uint64_t stat = 0;  // polygon edges: rows [ystart, yend) crossed; lines: kept segment + 1
-  bool line = false;
+  uint64_t stat = 0;  // lines: kept segment + 1
   bool odd = false;   // polygon edges: some row may end with an odd crossing count
   bool far = false;   // line segments: a floored coordinate beyond +-2^30
   auto vertex = [&](const RZ_CONST JobDev& J) {
@@ -168,67 +204,9 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
     const double x0 = px_x(X0);
     const double y0 = px_y(Y0);
     if (kind == 0) {  // polygon rings: extract_ring + PolyEdge::new
-      PolyEdge e{0.0, 0.0, 0.0, 0, 0};
-      // a ring left open by the caller (its last coordinate is not its
-      // first) can leave rows with an odd crossing count
-      if ((vi & VI_RING_START) && !closed) odd = true;
-      if (has_next) {
-        const double x1 = px_x(X1);
-        const double y1 = px_y(Y1);
-        if (!(fabs(y0 - y1) >= 2.220446049250313e-16)) {
-          // a skipped segment whose end points straddle a pixel-centre row
-          // (or are not numbers) leaves rows with an odd crossing count
-          if (isnan(y0) || isnan(y1) || ceil(fmin(y0, y1) - 0.5) != ceil(fmax(y0, y1) - 0.5)) odd = true;
-        } else {  // edges.rs:100
-          const double min_y = fmin(y0, y1), max_y = fmax(y0, y1);
-          if (min_y < rows && max_y >= 0.0) {  // edges.rs:105
-            double xt, yt, xb, yb;
-            if (y0 < y1) { xt = x0; yt = y0; xb = x1; yb = y1; }
-            else { xt = x1; yt = y1; xb = x0; yb = y0; }
-            e.ystart = sat_usize_cap(ceil(yt - 0.5), J.nrows);
-            e.yend = sat_usize_cap(ceil(yb - 0.5), J.nrows);
-            // (yb - yt is neither NaN nor zero here)
-            const double dx = x86_nan(xb - xt, xb, xt);
-            e.dxdy = x86_nan(dx / (yb - yt), dx, 0.0);
-            e.x0 = xt;
-            e.y0 = yt;
-            // With a NaN x0 or slope, every crossing of the edge is NaN with
-            // that NaN's sign (x0's when both are NaN).  The reference sorts a
-            // positive NaN crossing last, where it closes an empty span or is
-            // the odd one out: as if it were absent, so the edge is emptied.
-            // A negative one sorts first and spans from column 0, like -inf:
-            // the edge is pinned there.
-            if (isnan(xt) || isnan(e.dxdy)) {
-              if (signbit(isnan(xt) ? xt : e.dxdy)) {
-                e.x0 = -__builtin_inf();
-                e.y0 = 0.0;
-                e.dxdy = 0.0;
-              } else {
-                if (e.ystart < e.yend) odd = true;  // its rows lose one crossing each
-                e.ystart = e.yend = 0;
-              }
-            }
-            if (e.ystart < e.yend) {
-              box.r0 = e.ystart;
-              box.r1 = e.yend;
-              stat = (uint64_t)(e.yend - e.ystart);
-              // Crossings of this edge lie between its end points up to a few
-              // ulps, so their span columns are within one pixel of these.
-              const double ax = fabs(xt), bx = fabs(xb);
-              if (isnan(xt) || isnan(xb) || ax > 1.0e12 || bx > 1.0e12) {
-                box.c0 = 0;
-                box.c1 = J.ncols;
-              } else {
-                const double lo = floor(fmin(xt, xb) + 0.5) - 1.0;
-                const double hi = floor(fmax(xt, xb) + 0.5) + 1.0;
-                box.c0 = (int32_t)fmin(fmax(lo, 0.0), cols);
-                box.c1 = (int32_t)fmin(fmax(hi, 0.0), cols);
-              }
-            }
-          }
-        }
-      }
-      a.edges[v] = e;
+      PolyEdge e;
+      polygon_edge(vi, x0, y0, px_x(X1), px_y(Y1), J, a.edges != nullptr, e, box, odd);
+      if (a.edges) a.edges[v] = e;
       const bool at_cache = a.item_win && (J.fun == 0 || J.fun == 5);
       if (J.all_touched && at_cache) {
         // the box of every vertex, which bounds the fill (a NaN coordinate
@@ -272,7 +250,6 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
         }
       }
     } else if (kind == 1) {  // line rings: extract_line
-      line = true;
       uint4 rec = make_uint4(kLsNone, 0u, 0u, 0u);
       if (has_next) {
         const double x1 = px_x(X1);
@@ -323,7 +300,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   } else if (active) {
     vertex(as_const(a.jobs)[find_job(a.job_vend, a.n_jobs, v)]);
   }
-  reduce_box(item, box, stat, line, a.item_box, a.item_last, active);
+  reduce_box(v, item, box, stat, a.item_box, a.item_last, active);
   if (odd) atomicOr(&a.item_last[item], kItemOddBit);
   if (far) atomicOr(&a.item_last[item], kItemFarBit);
 }
@@ -340,16 +317,90 @@ __device__ inline bool tile_rect(int32_t r0, int32_t r1, int32_t c0, int32_t c1,
   return true;
 }
 
+// Hands out masks and k_cover list entries for the polygon items of a
+// workgroup (every thread calls it; `poly` says the thread has one with a
+// box).  One atomic per counter and workgroup, as one per wave contended
+// measurably on millions of items.  Returns whether the item got its masks
+// and sets their first 16-word unit.
+// NWV: the workgroup's waves.  LIST: every item is entered in a list; else
+// the calling wave covers the items with `small` (of the small list's kind)
+// and those with `own` (at most kCoverOwn wave windows) itself.
+template <int NWV, bool LIST>
+__device__ inline bool assign_cover(const CoverLists& c, bool poly, const ItemDesc& d, int64_t i, uint32_t& mask,
+                                    bool& small, bool& own) {
+  __shared__ unsigned long long s_m[NWV + 1];
+  __shared__ uint32_t s_n[3][NWV + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t mu = 0;              // 16-word units of masks
+  uint32_t n[3] = {0, 0, 0};    // entries of small, wave, block
+  small = false;
+  if (poly) {
+    const int32_t ns = mask_strip_count(d.r0, d.r1), nw = mask_row_words(d.c0, d.c1);
+    const bool odd = (d.flags & kItemOddRows) != 0;
+    mu = (uint64_t)ns * (uint64_t)nw;
+    if (d.nv <= 64 && !odd && (uint64_t)ns * 16u * (uint64_t)(nw | 1) <= (uint64_t)kCoverWave) small = true;
+    else if (d.nv <= kCoverBlockNv) n[1] = (uint32_t)cover_windows(ns, nw, odd, kCoverWave).n;
+    else n[2] = (uint32_t)cover_windows(ns, nw, odd, kCoverBlock).n;
+  }
+  if (LIST) n[0] = small ? 1u : 0u;
+  own = !LIST && n[1] && n[1] <= (uint32_t)kCoverOwn;
+  if (own) n[1] = 0u;
+  // inclusive sums inside the wave (mu < 2^52: summed in halves of 26 bits)
+  const uint64_t xm = (uint64_t)wave_prefix_sum((uint32_t)mu & 0x3FFFFFFu) +
+                      ((uint64_t)wave_prefix_sum((uint32_t)(mu >> 26)) << 26);
+  uint32_t x[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) x[k] = wave_prefix_sum(n[k]);
+  if (lane == 63) {
+    s_m[wave] = xm;
+    for (int k = 0; k < 3; ++k) s_n[k][wave] = x[k];
+  }
+  lds_barrier();
+  if (threadIdx.x < 4) {  // thread 0: masks; 1-3: small, wave, block
+    const int k = (int)threadIdx.x - 1;
+    unsigned long long sum = 0;
+    for (int w = 0; w < NWV; ++w) {
+      const unsigned long long t = k < 0 ? s_m[w] : s_n[k][w];
+      if (k < 0) s_m[w] = sum;
+      else s_n[k][w] = (uint32_t)sum;
+      sum += t;
+    }
+    if (k < 0) s_m[NWV] = sum ? atomicAdd(&c.ctr->mask_units, sum) : 0ull;
+    else s_n[k][NWV] = sum ? atomicAdd(&(&c.ctr->n_small)[k], (uint32_t)sum) : 0u;
+  }
+  lds_barrier();
+  const uint64_t mb = s_m[NWV] + s_m[wave] + xm - mu;
+  uint32_t at[3];
+  for (int k = 0; k < 3; ++k) at[k] = s_n[k][NWV] + s_n[k][wave] + x[k] - n[k];
+  const bool ok = poly && mb + mu <= c.mask_cap && (!n[1] || at[1] + n[1] <= c.unit_cap) &&
+                  (!n[2] || at[2] + n[2] <= c.unit_cap);
+  mask = (uint32_t)mb;
+  // (an entry of an item without masks stays a gap: k_cover checks the flag)
+  if (n[0]) c.small[at[0]] = (uint32_t)i;
+  // windows: the wave writes one item's entries together
+  for (int k = 1; k < 3; ++k) {
+    uint2* list = k == 1 ? c.wave : c.block;
+    for (uint64_t m = __ballot(n[k] != 0u); m; m &= m - 1ull) {
+      const int b = __builtin_ctzll(m);
+      const uint32_t nb = (uint32_t)__builtin_amdgcn_readlane((int)n[k], b);
+      const uint32_t ab = (uint32_t)__builtin_amdgcn_readlane((int)at[k], b);
+      const uint32_t ib = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)i, b);
+      for (uint32_t t = (uint32_t)lane; t < nb; t += 64u)
+        if (ab + t < c.unit_cap) list[ab + t] = make_uint2(ib, t);
+    }
+  }
+  return ok;
+}
+
 // One thread per item: resolve the field value and band of the owning
-// geometry (rust/src/rasterize.rs:169-179) into the item's descriptor and,
-// for binned jobs, count the tiles its box covers.
-__global__ void k_item_desc(DescArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n_items) return;
+// geometry (rust/src/rasterize.rs:169-179) into the item's descriptor, hand
+// out its masks (polygons) and, for binned jobs, count the tiles its box
+// covers.
+// (b: its box; stat: its item_last word)
+__device__ inline ItemDesc make_desc(const DescArgs& a, int64_t i, ItemBox b, uint64_t stat) {
   const int j = find_job_wave(a.job_iend, a.n_jobs, i);
   const RZ_CONST JobDev& J = as_const(a.jobs)[j];
   const int64_t li = i - J.i_base;
-  ItemBox b = a.item_box[i];
   const int32_t g = J.item_geom[li];
   uint32_t layer = J.layer_of_geom ? J.layer_of_geom[g] : 0u;
   if (layer >= J.n_layers) {
@@ -375,12 +426,7 @@ __global__ void k_item_desc(DescArgs a) {
   }
   d.value = v;
   const int32_t kind = J.item_kind[li];
-  const uint64_t S_raw = a.item_last[i];
-  const bool tall = d.r0 < d.r1 && (d.r1 - 1) / kBandRows > d.r0 / kBandRows;
-  const bool banded = a.band_n && tall &&
-                      ((kind == 0 && d.nv > kBandMinEdges) ||
-                       (kind == 1 && d.nv > kLineBandMinSegs && !(S_raw & kItemFarBit) && !J.all_touched));
-  d.last = kind == 1 ? (S_raw & ~kItemFarBit) : 0ull;
+  d.last = kind == 1 ? (stat & ~kItemFarBit) : 0ull;
   if (kind == 0 && J.all_touched) d.last = (uint64_t)i;  // (its outline box is found by item)
   if (a.at_words) {
     // sum / count dedup (prelude.rs:116-118): the fill skips pixels in the
@@ -413,43 +459,15 @@ __global__ void k_item_desc(DescArgs a) {
   d.job = (uint32_t)j;
   d.band = 0;
   d.flags = 0;
-  d.wide = 0;
+  d.mask = 0;
   if (a.scan_box && J.scan_compact) a.scan_box[i] = scan_box_of(d.r0, d.r1, d.c0, d.c1, J.tile_w);
-  if (kind == 0 && (S_raw & kItemOddBit)) d.flags |= kItemOddRows;
+  if (kind == 0 && (stat & kItemOddBit)) d.flags |= kItemOddRows;
   if (a.at_words && a.at_words[i]) d.flags |= kItemAtCache;
-  a.desc[i] = d;
-  if (a.wide_units) {
-    // Work of one strip, from the rows the edges cross (S) over the item's
-    // height (H): an edge crossing s rows meets about (s + 15) / H of the
-    // item's strips, so a strip sees n ~ (S + 15 nv) / H edges.  In steps of
-    // 64 crossing tests: in a tile, row-major coverage takes n / 4 steps,
-    // repeated in each of the tw tiles of the item's width.  The wide
-    // pre-pass does the strip once, in n / 4 steps or, edge-major, in the
-    // longest crossing run of each chunk of 64 loaded edges (all nv, or the n
-    // of the strip's band; taken as 2 S / nv + 1 rows, at most 16), plus
-    // about 16 steps of set-up and mask stores, and the tiles then read one
-    // mask word each (about half a step).  Wide when that is at least a
-    // quarter cheaper.
-    uint32_t units = 0, words = 0;
-    if (kind == 0 && d.nv > 0 && d.r0 < d.r1 && d.c0 < d.c1 && a.wide_mode != 1) {
-      const float S = (float)(S_raw & ~kItemOddBit), nv = (float)d.nv, H = (float)(d.r1 - d.r0);
-      const float n = fminf(nv, (S + 15.0f * nv) / H);
-      const float chunks = ceilf((banded ? n : nv) / 64.0f);
-      const float run = fminf(16.0f, 2.0f * S / nv + 1.0f);
-      const float tw = (float)((d.c1 - 1) / J.tile_w - d.c0 / J.tile_w + 1);
-      const float in_tile = tw * fmaxf(1.0f, n / 4.0f);
-      const float wide = fminf(n / 4.0f, chunks * run) + 16.0f + 0.5f * tw;
-      if (a.wide_mode == 2 || in_tile > 1.25f * wide) {
-        const int32_t ns = wide_strip_count(d.r0, d.r1), nw = wide_row_words(d.c0, d.c1);
-        units = (uint32_t)ns * (uint32_t)((nw + kWideWords - 1) / kWideWords);
-        words = (uint32_t)ns * 16u * (uint32_t)nw;
-      }
-    }
-    a.wide_units[i] = units;
-    a.wide_words[i] = words;
-  }
-  if (a.band_n)
+  if (a.band_n) {
+    const bool banded = kind == 1 && d.nv > kLineBandMinSegs && !(stat & kItemFarBit) && !J.all_touched &&
+                        d.r0 < d.r1 && (d.r1 - 1) / kBandRows > d.r0 / kBandRows;
     a.band_n[i] = banded ? (uint32_t)((d.r1 - 1) / kBandRows - d.r0 / kBandRows + 1) : 0u;
+  }
   if (a.counts) {
     int32_t tx0, tx1, ty0, ty1;
     uint32_t c = 0;
@@ -457,12 +475,31 @@ __global__ void k_item_desc(DescArgs a) {
       c = (uint32_t)(tx1 - tx0 + 1) * (uint32_t)(ty1 - ty0 + 1);
     a.counts[i] = c;
   }
+  return d;
+}
+
+__global__ __launch_bounds__(kDescBlock) void k_item_desc(DescArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * kDescBlock + threadIdx.x;
+  const bool item = i < a.n_items;
+  ItemDesc d;
+  __builtin_memset(&d, 0, sizeof(d));
+  if (item) d = make_desc(a, i, a.item_box[i], a.item_last[i]);
+  if (a.cover.ctr) {
+    const bool poly = item && (d.kind_layer & 3u) == 0u && d.nv > 0 && d.r0 < d.r1 && d.c0 < d.c1;
+    uint32_t mask;
+    bool small, own;
+    if (assign_cover<kDescBlock / 64, true>(a.cover, poly, d, i, mask, small, own)) {
+      d.flags |= kItemMask;
+      d.mask = mask;
+    }
+  }
+  if (item) a.desc[i] = d;
 }
 
 // ------------------------------------------------------------ edge bands --
 
 // Items whose band entries would pass the capacity stay unbanded (their
-// strips then scan the whole edge list: slower, same result).
+// strips then read all their segments: slower, same result).
 // Assigned items are also appended to the list the band passes walk (any
 // order: every item owns its entries), one atomic per block (one per wave
 // contended measurably on millions of items).
@@ -488,21 +525,6 @@ __global__ __launch_bounds__(kBandAssignBlock) void k_band_assign(ItemDesc* desc
   uint32_t base = s_base;
   for (int w = 0; w < wave; ++w) base += s_n[w];
   if (ok) items[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)i;
-}
-
-// Wide items whose units and mask words fit the capacities (every item
-// below them in the scans does too) take the wide pre-pass: flag, mask base
-// and one unit-list entry per (strip, window) unit.
-__global__ void k_wide_assign(WideAssignArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n_items) return;
-  const uint32_t nu = a.wide_units[i];
-  if (!nu) return;
-  const uint64_t ub = a.unit_base[i], wb = a.word_base[i];
-  if (ub + nu > a.unit_cap || a.word_base[i + 1] > a.word_cap) return;  // stays per tile
-  a.desc[i].flags |= kItemWide;
-  a.desc[i].wide = (uint32_t)(wb >> 4);  // every item's words are a multiple of 16
-  for (uint32_t k = 0; k < nu; ++k) a.unit_item[ub + k] = (uint32_t)i;
 }
 
 // ------------------------------------------------- all-touched PixelCache --
@@ -539,12 +561,12 @@ __global__ __launch_bounds__(256) void k_at_cache(AtCacheArgs a) {
 }
 
 // Count pass, one wave per banded item (of the list k_band_assign built): band_cnt of each of its strips,
-// from a difference array in LDS (+1 at an edge's first strip, -1 after its
-// last) and a running sum, so an edge costs two LDS atomics however many
+// from a difference array in LDS (+1 at a segment's first strip, -1 after its
+// last) and a running sum, so a segment costs two LDS atomics however many
 // strips it meets.  Plain stores: every item owns its band entries.
 __global__ __launch_bounds__(256) void k_band_count(BandArgs a) {
   __shared__ uint32_t s_cnt[4][kBandLds + 1];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = wave_index(), lane = threadIdx.x & 63;
   uint32_t* cnt = s_cnt[wave];
   const uint32_t n_list = *a.n_list;
   for (uint32_t li = blockIdx.x * 4u + (uint32_t)wave; li < n_list; li += gridDim.x * 4u) {
@@ -552,17 +574,13 @@ __global__ __launch_bounds__(256) void k_band_count(BandArgs a) {
     const uint32_t ns = as_const(a.band_n)[i];
     const RZ_CONST ItemDesc& d = as_const(a.desc)[i];
     const int32_t sr0 = d.r0 / kBandRows, sr1 = (d.r1 - 1) / kBandRows;
-    const PolyEdge* eb = a.edges + d.vbeg;
     for (uint32_t s0 = 0; s0 < ns; s0 += kBandLds) {
       const uint32_t L = min((uint32_t)kBandLds, ns - s0);
       for (uint32_t k = lane; k <= L; k += 64) cnt[k] = 0u;
       wave_sync();
-      // each lane's next edge is loaded while the current one is counted;
-      // its rows [ystart, yend), or for a line segment those of its cells
-      const bool line = (d.kind_layer & 3u) == 1u;  // wave-uniform
+      // each lane's next segment is loaded while the current one is counted
       const uint4* sb = a.lseg + d.vbeg;
       auto rows_of = [&](int32_t e) -> int2 {
-        if (!line) return *reinterpret_cast<const int2*>(&eb[e].ystart);
         const uint4 r = sb[e];
         if (r.x >= kLsFar) return make_int2(0, 0);
         const int32_t y0 = (int32_t)((int64_t)r.y - kLsBias), y1 = (int32_t)((int64_t)(r.w & ~kLsFlag) - kLsBias);
@@ -598,11 +616,11 @@ __global__ __launch_bounds__(256) void k_band_count(BandArgs a) {
   }
 }
 
-// Scatter pass, one wave per banded item: each edge is copied into every
+// Scatter pass, one wave per banded item: each segment is copied into every
 // strip it meets, at a slot taken from the strip's LDS cursor.
 __global__ __launch_bounds__(256) void k_band_scatter(BandArgs a) {
   __shared__ uint32_t s_pos[4][kBandLds];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = wave_index(), lane = threadIdx.x & 63;
   uint32_t* pos = s_pos[wave];
   const uint32_t n_list = *a.n_list;
   for (uint32_t li = blockIdx.x * 4u + (uint32_t)wave; li < n_list; li += gridDim.x * 4u) {
@@ -610,64 +628,31 @@ __global__ __launch_bounds__(256) void k_band_scatter(BandArgs a) {
     const uint32_t ns = as_const(a.band_n)[i];
     const RZ_CONST ItemDesc& d = as_const(a.desc)[i];
     const int32_t sr0 = d.r0 / kBandRows, sr1 = (d.r1 - 1) / kBandRows;
-    const PolyEdge* eb = a.edges + d.vbeg;
     const uint64_t base = as_const(a.band_off)[d.band - 1u];
     for (uint32_t s0 = 0; s0 < ns; s0 += kBandLds) {
       const uint32_t L = min((uint32_t)kBandLds, ns - s0);
       for (uint32_t k = lane; k < L; k += 64) pos[k] = (uint32_t)(a.band_off[d.band - 1u + s0 + k] - base);
       wave_sync();
-      if ((d.kind_layer & 3u) == 1u) {  // a line item (wave-uniform): segment records
-        const uint4* sb = a.lseg + d.vbeg;
-        uint4 nr = make_uint4(kLsNone, 0u, 0u, 0u);
-        if (lane < d.nv) nr = sb[lane];
-        for (int32_t e = lane; e < d.nv; e += 64) {
-          uint4 r = nr;
-          if (e + 64 < d.nv) nr = sb[e + 64];
-          if (r.x >= kLsFar) continue;
-          const int32_t y0 = (int32_t)((int64_t)r.y - kLsBias);
-          const int32_t y1 = (int32_t)((int64_t)(r.w & ~kLsFlag) - kLsBias);
-          const int32_t ys = max(min(y0, y1), 0), ye = max(y0, y1) + 1;
-          // the band record's flag: this is the last kept edge of an open
-          // line, whose end cell is written (burners.rs:86-89)
-          const bool end = (uint64_t)(d.vbeg + e + 1) == d.last && !(r.w & kLsFlag);
-          r.w = (r.w & ~kLsFlag) | (end ? kLsFlag : 0u);
-          const int32_t b0 = max(max(ys / kBandRows, sr0) - sr0, (int32_t)s0);
-          const int32_t b1 = min(min((ye - 1) / kBandRows, sr1) - sr0, (int32_t)(s0 + L - 1));
-          for (int32_t b = b0; b <= b1; ++b) {
-            const uint64_t slot = base + atomicAdd(&pos[b - s0], 1u);
-            if (slot < a.edge_cap) a.band_segs[slot] = r;
-            else atomicOr(a.status, 8u);
-          }
-        }
-        wave_sync();
-        continue;
-      }
-      // the record as two 16-byte vectors (no struct copy through scratch);
-      // each lane's next edge is loaded while the current one is copied
-      uint4 nlo = make_uint4(0u, 0u, 0u, 0u), nhi = nlo;
-      if (lane < d.nv) {
-        nlo = reinterpret_cast<const uint4*>(eb + lane)[0];
-        nhi = reinterpret_cast<const uint4*>(eb + lane)[1];
-      }
+      const uint4* sb = a.lseg + d.vbeg;
+      uint4 nr = make_uint4(kLsNone, 0u, 0u, 0u);
+      if (lane < d.nv) nr = sb[lane];
       for (int32_t e = lane; e < d.nv; e += 64) {
-        const uint4 lo = nlo, hi = nhi;  // hi.z = ystart, hi.w = yend
-        if (e + 64 < d.nv) {
-          nlo = reinterpret_cast<const uint4*>(eb + e + 64)[0];
-          nhi = reinterpret_cast<const uint4*>(eb + e + 64)[1];
-        }
-        const int32_t ys = (int32_t)hi.z, ye = (int32_t)hi.w;
-        if (!(ys < ye)) continue;
+        uint4 r = nr;
+        if (e + 64 < d.nv) nr = sb[e + 64];
+        if (r.x >= kLsFar) continue;
+        const int32_t y0 = (int32_t)((int64_t)r.y - kLsBias);
+        const int32_t y1 = (int32_t)((int64_t)(r.w & ~kLsFlag) - kLsBias);
+        const int32_t ys = max(min(y0, y1), 0), ye = max(y0, y1) + 1;
+        // the band record's flag: this is the last kept edge of an open
+        // line, whose end cell is written (burners.rs:86-89)
+        const bool end = (uint64_t)(d.vbeg + e + 1) == d.last && !(r.w & kLsFlag);
+        r.w = (r.w & ~kLsFlag) | (end ? kLsFlag : 0u);
         const int32_t b0 = max(max(ys / kBandRows, sr0) - sr0, (int32_t)s0);
         const int32_t b1 = min(min((ye - 1) / kBandRows, sr1) - sr0, (int32_t)(s0 + L - 1));
         for (int32_t b = b0; b <= b1; ++b) {
           const uint64_t slot = base + atomicAdd(&pos[b - s0], 1u);
-          if (slot < a.edge_cap) {
-            uint4* dst = reinterpret_cast<uint4*>(a.band_edges + slot);
-            dst[0] = lo;
-            dst[1] = hi;
-          } else {
-            atomicOr(a.status, 8u);
-          }
+          if (slot < a.edge_cap) a.band_segs[slot] = r;
+          else atomicOr(a.status, 8u);
         }
       }
       wave_sync();

@@ -1,6 +1,6 @@
-// rz_launch.h -- host launchers of the tile kernels, one pair per output
+// rz_launch.h -- host launchers of the tile kernels, one per output
 // dtype.  Each is defined in its own translation unit (rz_tile_inst.hip
-// compiled once per dtype), so the k_tile / k_tile_heavy instantiations of
+// compiled once per dtype), so the k_tile / k_tile_lp instantiations of
 // the ten dtypes build in parallel.
 #pragma once
 
@@ -10,9 +10,9 @@
 
 namespace rzk {
 
-#define RZ_TILE_LAUNCHERS(NAME)                                                      \
-  void launch_tile_##NAME(int fun, const TileArgs& a, bool lines, hipStream_t s);    \
-  void launch_heavy_##NAME(int fun, const TileArgs& a, hipStream_t s);
+#define RZ_TILE_LAUNCHERS(NAME)                                                          \
+  void launch_tile_##NAME(int fun, const TileArgs& a, bool lines, hipStream_t s);         \
+  void launch_blocks_##NAME(const TileArgs& a, hipStream_t s);
 RZ_TILE_LAUNCHERS(u8)
 RZ_TILE_LAUNCHERS(u16)
 RZ_TILE_LAUNCHERS(u32)

@@ -81,13 +81,11 @@ struct rz_context {
   hipStream_t stream = nullptr;
   // workspace
   Buf edges, lseg, item_box, item_last, desc, pair_desc, counts, offsets, keys_a, vals_a, keys_b,
-      vals_b, tile_off, temp, misc, jobtab, queue, band_n, band_base, band_cnt, band_off, band_edges,
-      heavy_cnt, heavy_base, masks, scan_tmp, scan_tmp2, scan_tmp3, scan_tmp4,
-      sort_hist, sort_off, sort_tmp, cover_list, wide_units, wide_words, wide_ubase, wide_wbase,
-      wide_item, wide_masks, scan_tmp5, scan_tmp6, band_items, heavy_list, scan_tmp7, wide_j, band_segs,
-      item_win, at_words, at_base, at_bits, scan_tmp8, scan_box;
-  // pinned: [0] pairs, [1] status, [2] band entries, [3] banded edges, [4] wide units, [5] wide words,
-  // [6] all-touched PixelCache words
+      vals_b, tile_off, misc, jobtab, queue, band_n, band_base, band_cnt, band_off, masks, scan_tmp, scan_tmp2,
+      scan_tmp3, sort_hist, sort_off, sort_tmp, cover, band_items, band_segs,
+      item_win, at_words, at_base, at_bits, scan_tmp8, scan_box, sp_counts, sp_first, sp_bits, sp_bitn, sp_bit_base;
+  // pinned: [0] pairs, [1] (sparse) bit words, [2] band entries, [3] banded segments, [4..6] cover counters
+  // (CoverCounters: mask units, small | wave, block), [7] all-touched PixelCache words
   uint64_t* host_misc = nullptr;
   // job table: built in tab_build, staged in pinned host_tab (tab_ev marks
   // the end of its last upload); tab_dev / tab_dev_bytes say which device
@@ -107,16 +105,15 @@ struct rz_context {
   EventSet cur;
   double acc_ms[kStages] = {};
   uint64_t last_pairs = 0, last_tiles = 0, last_band_entries = 0, last_band_edges = 0;
-  uint64_t last_wide_units = 0, last_wide_words = 0, last_at_words = 0;
+  uint64_t last_masks = 0, last_units = 0, last_at_words = 0;
   bool burns_pending = false;
   std::vector<Buf*> all() {
-    return {&edges,  &lseg,   &item_box, &item_last, &desc, &counts,    &offsets, &keys_a,
-            &vals_a, &keys_b, &vals_b, &tile_off, &temp,      &misc, &pair_desc, &jobtab,  &queue,
-            &band_n, &band_base, &band_cnt, &band_off, &band_edges, &heavy_cnt, &heavy_base,
-            &masks, &scan_tmp, &scan_tmp2, &scan_tmp3, &scan_tmp4,
-            &sort_hist, &sort_off, &sort_tmp, &cover_list, &wide_units, &wide_words, &wide_ubase,
-            &wide_wbase, &wide_item, &wide_masks, &scan_tmp5, &scan_tmp6, &band_items, &heavy_list, &scan_tmp7,
-            &wide_j, &band_segs, &item_win, &at_words, &at_base, &at_bits, &scan_tmp8, &scan_box};
+    return {&edges,     &lseg,      &item_box,    &item_last,   &desc,       &pair_desc,  &counts,    &offsets,
+            &keys_a,    &vals_a,    &keys_b,      &vals_b,      &tile_off,   &misc,       &jobtab,    &queue,
+            &band_n,    &band_base, &band_cnt,    &band_off,    &masks,      &scan_tmp,   &scan_tmp2, &scan_tmp3,
+            &sort_hist, &sort_off,  &sort_tmp,    &cover,       &band_items,
+            &band_segs, &item_win,  &at_words,    &at_base,     &at_bits,    &scan_tmp8,  &scan_box,  &sp_counts,
+            &sp_first,  &sp_bits,   &sp_bitn,     &sp_bit_base};
   }
   // Takes an event set for the next call (events are recorded on the stream
   // and resolved later, so timing adds no synchronisation to the call).
@@ -163,6 +160,7 @@ struct rz_device_geometry {
   int64_t* item_vbeg = nullptr;
   bool has_poly = false, has_line = false, has_point = false;
   int64_t max_poly_nv = 0;  // most vertices of one polygon item
+  int64_t n_poly = 0, poly_nv = 0;  // polygon items and their vertices
   int64_t max_line_nv = 0;  // most vertices of one line item
 };
 
@@ -410,7 +408,11 @@ extern "C" rz_status rz_device_geometry_upload(rz_context* c, const rz_geometry*
     if (g->item_ring_offsets[i + 1] == g->item_ring_offsets[i]) continue;
     const int64_t nv = g->ring_vertex_offsets[g->item_ring_offsets[i + 1]] -
                        g->ring_vertex_offsets[g->item_ring_offsets[i]];
-    if (k == RZ_ITEM_POLYGONS) dg->max_poly_nv = std::max<int64_t>(dg->max_poly_nv, nv);
+    if (k == RZ_ITEM_POLYGONS) {
+      dg->max_poly_nv = std::max<int64_t>(dg->max_poly_nv, nv);
+      dg->n_poly += 1;
+      dg->poly_nv += nv;
+    }
     if (k == RZ_ITEM_LINES) dg->max_line_nv = std::max<int64_t>(dg->max_line_nv, nv);
     dg->has_poly |= k == RZ_ITEM_POLYGONS;
     dg->has_line |= k == RZ_ITEM_LINES;
@@ -507,6 +509,8 @@ extern "C" rz_status rz_device_synth_job(rz_context* c, uint64_t seed, int64_t k
   dg->V = voff[(size_t)G];
   dg->has_poly = G > 0;
   dg->max_poly_nv = max_nv;
+  dg->n_poly = dg->I;
+  dg->poly_nv = dg->V;
   hipError_t e = upload(c, &dg->geom_item_off, seq.data(), G + 1);
   if (e == hipSuccess) e = upload(c, &dg->item_kind, kinds.data(), G);
   if (e == hipSuccess) e = upload(c, &dg->item_ring_off, seq.data(), G + 1);
@@ -578,21 +582,6 @@ Tuning tuning_for(uint32_t cls) {
   return it == ts.table.end() ? Tuning{} : it->second;
 }
 
-void launch_heavy_dispatch(rz_dtype dt, int fun, const TileArgs& a, hipStream_t s) {
-  switch (dt) {
-    case RZ_U8: launch_heavy_u8(fun, a, s); break;
-    case RZ_U16: launch_heavy_u16(fun, a, s); break;
-    case RZ_U32: launch_heavy_u32(fun, a, s); break;
-    case RZ_U64: launch_heavy_u64(fun, a, s); break;
-    case RZ_I8: launch_heavy_i8(fun, a, s); break;
-    case RZ_I16: launch_heavy_i16(fun, a, s); break;
-    case RZ_I32: launch_heavy_i32(fun, a, s); break;
-    case RZ_I64: launch_heavy_i64(fun, a, s); break;
-    case RZ_F32: launch_heavy_f32(fun, a, s); break;
-    default: launch_heavy_f64(fun, a, s); break;
-  }
-}
-
 void launch_tile_dispatch(rz_dtype dt, int fun, const TileArgs& a, bool lines, hipStream_t s) {
   switch (dt) {
     case RZ_U8: launch_tile_u8(fun, a, lines, s); break;
@@ -605,6 +594,20 @@ void launch_tile_dispatch(rz_dtype dt, int fun, const TileArgs& a, bool lines, h
     case RZ_I64: launch_tile_i64(fun, a, lines, s); break;
     case RZ_F32: launch_tile_f32(fun, a, lines, s); break;
     default: launch_tile_f64(fun, a, lines, s); break;
+  }
+}
+void launch_blocks_dispatch(rz_dtype dt, const TileArgs& a, hipStream_t s) {
+  switch (dt) {
+    case RZ_U8: launch_blocks_u8(a, s); break;
+    case RZ_U16: launch_blocks_u16(a, s); break;
+    case RZ_U32: launch_blocks_u32(a, s); break;
+    case RZ_U64: launch_blocks_u64(a, s); break;
+    case RZ_I8: launch_blocks_i8(a, s); break;
+    case RZ_I16: launch_blocks_i16(a, s); break;
+    case RZ_I32: launch_blocks_i32(a, s); break;
+    case RZ_I64: launch_blocks_i64(a, s); break;
+    case RZ_F32: launch_blocks_f32(a, s); break;
+    default: launch_blocks_f64(a, s); break;
   }
 }
 
@@ -640,7 +643,7 @@ rz_status check_job_common(const rz_job& j, bool need_out) {
 // indices are global over the batch.
 // Fixed capacities of a captured batch (see rz_batch_graph_create).
 struct BatchCaps {
-  uint64_t pairs, band_entries, band_edges, wide_units, wide_words, at_words;
+  uint64_t pairs, band_entries, band_edges, masks, units, at_words;
 };
 
 // The device record of job j, whose vertex / item / tile ranges start at
@@ -692,9 +695,8 @@ static uint64_t job_record(const rz_job& j, JobDev& J, int64_t v_base, int64_t i
   return jt;
 }
 
-// masks_only: the set-up and the wide pre-pass only, for every polygon item
-// and with no cap on the masks (the sparse encoding reads them); no bins, no
-// tile launches.
+// masks_only: the set-up and the coverage masks only (the sparse encoding
+// reads them); no bins, no tile launches.
 static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
                            const BatchCaps* caps = nullptr, bool masks_only = false) {
   const bool capture = caps != nullptr;
@@ -713,21 +715,10 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     if (std::strcmp(bm, "always") == 0) binning = 1;
     else if (std::strcmp(bm, "never") == 0) binning = -1;
   }
-  // RUSTERIZE_COVERAGE=rows|edges forces one coverage layout in the wide
-  // pre-pass (tests run both on the same inputs).
-  int cov_mode = 0;
-  if (const char* cm = std::getenv("RUSTERIZE_COVERAGE")) {
-    if (std::strcmp(cm, "rows") == 0) cov_mode = 1;
-    else if (std::strcmp(cm, "edges") == 0) cov_mode = 2;
-  }
-  // RUSTERIZE_WIDE=never|always: no item / every polygon item takes the wide
-  // coverage pre-pass (tests run both on the same inputs).
-  int wide_mode = 0;
-  if (const char* wm = std::getenv("RUSTERIZE_WIDE")) {
-    if (std::strcmp(wm, "never") == 0) wide_mode = 1;
-    else if (std::strcmp(wm, "always") == 0) wide_mode = 2;
-  }
-  if (masks_only) wide_mode = 2;
+  // RUSTERIZE_WIDE=never: no polygon item gets coverage masks, the tile
+  // kernels compute them strip by strip (tests run both on the same inputs).
+  bool use_masks = true;
+  if (const char* wm = std::getenv("RUSTERIZE_WIDE")) use_masks = masks_only || std::strcmp(wm, "never") != 0;
   // (all-touched jobs walk their polygons' outlines too: the lines kernel)
   auto has_lines = [](const rz_job& j) { return j.geometry->has_line || j.geometry->has_point || j.all_touched; };
   std::vector<int64_t> order((size_t)n_in);
@@ -751,10 +742,9 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   int64_t V = 0, I = 0;
   uint64_t T = 0, out_px = 0;
   bool any_binned = false, any_poly = false, any_lp = false, any_band = false;
-  bool any_poly_band = false, any_line_band = false;
-  bool any_tw64 = false, any_tw256 = false;
   bool any_at_cache = false;  // all-touched sum / count polygons: PixelCache windows
-  bool any_wide_job = false;  // jobs whose polygons may take the wide pre-pass
+  uint64_t mask_bound = 0;    // 16-word mask units the batch can need at most
+  int64_t max_poly_nv = 0, n_poly = 0, poly_nv = 0;
   bool any_scan_compact = false;
   int max_tile_w = 64;
   for (size_t k = 0; k < n; ++k) {
@@ -780,17 +770,15 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     any_scan_compact |= J.scan_compact != 0;
     any_binned |= !scan && ni > 0;
     const bool lines = has_lines(j);
-    any_tw64 |= TW == 64;
-    any_tw256 |= TW == 256;
     max_tile_w = std::max(max_tile_w, TW);
     any_poly |= dg->has_poly;
-    // A small (scanned) job whose rings fit two 64-edge stages gains nothing
-    // from the wide pre-pass: each of its strips loads a ring's edges once
-    // either way, and the pass would add three launches to the call.
-    any_wide_job |= dg->has_poly && !(scan && dg->max_poly_nv <= kBandMinEdges);
-    any_poly_band |= dg->has_poly && dg->max_poly_nv > kBandMinEdges;
-    any_line_band |= dg->has_line && dg->max_line_nv > kLineBandMinSegs;
-    any_band = any_poly_band || any_line_band;
+    max_poly_nv = std::max(max_poly_nv, dg->max_poly_nv);
+    n_poly += dg->n_poly;
+    poly_nv += dg->poly_nv;
+    if (dg->has_poly)
+      mask_bound += std::min<uint64_t>(
+          ni * (uint64_t)((nrows + WAVE_ROWS - 1) / WAVE_ROWS) * (uint64_t)((ncols + 63) / 64), (uint64_t)1 << 40);
+    any_band |= dg->has_line && dg->max_line_nv > kLineBandMinSegs;
     any_lp |= lines;
     any_at_cache |= j.all_touched && dg->has_poly && (j.fun == RZ_SUM || j.fun == RZ_COUNT);
     if (groups.empty() || groups.back().dtype != j.dtype || groups.back().fun != (int)j.fun ||
@@ -814,12 +802,41 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   HIP_TRY(ensure(c->stream, c->jobtab, tab_bytes));
   const size_t misc_bytes = 64 + kBurnSlots * sizeof(unsigned long long);
   HIP_TRY(ensure(c->stream, c->misc, misc_bytes));
-  // per group: the tile queue, then one word: the k_tile_heavy work counter
-  const size_t queue_words = groups.size() * (kQueueWords + 1);
+  const size_t queue_words = groups.size() * kQueueWords;  // a tile queue per group
   HIP_TRY(ensure(c->stream, c->queue, queue_words * 4));
   uint32_t* d_status = (uint32_t*)c->misc.p;
   unsigned long long* d_burns = (unsigned long long*)((char*)c->misc.p + 64);
-  if (any_poly) HIP_TRY(ensure(c->stream, c->edges, (size_t)std::max<int64_t>(V, 1) * sizeof(PolyEdge)));
+  // Coverage masks.  An eager call that reads its totals back anyway (bins,
+  // line bands, the sparse encoding) sizes them exactly.  One that does not
+  // takes a capacity of 8 KiB per item and 2 bytes per pixel, with no host
+  // round trip, and a captured batch its own; should items pass those, the
+  // tile kernel computes their coverage from edge records, which are written
+  // in these cases only.
+  const bool bare = !masks_only && T <= kBlockTiles && n_poly <= kBareItems && poly_nv <= kBareVerts;
+  const bool any_mask = any_poly && use_masks && !bare && I > 0;
+  const bool read_totals = !capture && (any_binned || any_band || masks_only);
+  const uint64_t mask_fixed = capture ? caps->masks : std::min<uint64_t>(mask_bound, (uint64_t)I * 64 + out_px / 64);
+  const bool need_edges = any_poly && (!any_mask || (!read_totals && (capture || mask_bound > mask_fixed)));
+  if (need_edges) HIP_TRY(ensure(c->stream, c->edges, (size_t)std::max<int64_t>(V, 1) * sizeof(PolyEdge)));
+  CoverLists cover{};
+  // (windows hold 13 mask units or more on average, but for their items' last)
+  uint64_t unit_cap = capture ? caps->units : (uint64_t)I + (read_totals ? (uint64_t)I : mask_fixed / 8) + 1024;
+  auto place_cover = [&]() -> rz_status {  // the counters and lists, in one buffer
+    const size_t o_wave = sizeof(CoverCounters), o_block = o_wave + unit_cap * sizeof(uint2);
+    const size_t o_small = o_block + unit_cap * sizeof(uint2);
+    HIP_TRY(ensure(c->stream, c->cover, o_small + (size_t)I * 4));
+    char* p = (char*)c->cover.p;
+    cover.ctr = (CoverCounters*)p;
+    cover.wave = (uint2*)(p + o_wave);
+    cover.block = (uint2*)(p + o_block);
+    cover.small = (uint32_t*)(p + o_small);
+    cover.unit_cap = (uint32_t)std::min<uint64_t>(unit_cap, UINT32_MAX);
+    return RZ_OK;
+  };
+  if (any_mask) {
+    if (rz_status st = place_cover()) return st;
+    cover.mask_cap = read_totals ? (uint64_t)UINT32_MAX : std::min<uint64_t>(mask_fixed, UINT32_MAX);
+  }
   if (any_lp) HIP_TRY(ensure(c->stream, c->lseg, (size_t)std::max<int64_t>(V, 1) * sizeof(uint4)));
   HIP_TRY(ensure(c->stream, c->item_box, (size_t)std::max<int64_t>(I, 1) * sizeof(ItemBox)));
   HIP_TRY(ensure(c->stream, c->item_last, (size_t)std::max<int64_t>(I, 1) * 8));
@@ -837,19 +854,6 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     HIP_TRY(ensure(c->stream, c->item_win, (size_t)std::max<int64_t>(I, 1) * 64));
     HIP_TRY(ensure(c->stream, c->at_words, (size_t)(I + 1) * 4));
     HIP_TRY(ensure(c->stream, c->at_base, (size_t)(I + 1) * 8));
-  }
-  const bool any_wide = any_poly && wide_mode != 1 && I > 0 && (wide_mode == 2 || any_wide_job);
-  // A small eager call whose only pre-pass is the wide one sizes the wide
-  // buffers for the most they can hold (2 bytes per output pixel, every
-  // unit at least 16 words) instead of reading the totals back: no host
-  // round trip.
-  const bool wide_fixed =
-      !capture && !masks_only && any_wide && !any_binned && !any_band && out_px <= ((uint64_t)1 << 26);
-  if (any_wide) {
-    HIP_TRY(ensure(c->stream, c->wide_units, (size_t)(I + 1) * 4));
-    HIP_TRY(ensure(c->stream, c->wide_words, (size_t)(I + 1) * 4));
-    HIP_TRY(ensure(c->stream, c->wide_ubase, (size_t)(I + 1) * 8));
-    HIP_TRY(ensure(c->stream, c->wide_wbase, (size_t)(I + 1) * 8));
   }
   const JobDev* d_jobs = (const JobDev*)c->jobtab.p;
   const int64_t* d_vend = (const int64_t*)(d_jobs + n);
@@ -883,6 +887,9 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     c->tab_dev = c->jobtab.p;
     c->tab_dev_bytes = tab_bytes;
   }
+  // few polygons (all-touched ones count as lines) and no totals to wait for:
+  // boxes, descriptors and the small items' masks in one launch
+  const bool fused = any_mask && !read_totals && !any_lp && max_poly_nv <= kCoverBlockNv && I <= kItemsMax;
   // 1. item boxes reset and the call's counters cleared (one launch), edges /
   // pixel coordinates / item boxes, then the item descriptors
   {
@@ -897,28 +904,25 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     ia.clear(c->queue.p, queue_words);
     if (any_binned) ia.clear((uint32_t*)c->counts.p + I, 1);
     if (any_band) ia.clear((uint32_t*)c->band_n.p + I, 1);
-    if (any_wide) {
-      ia.clear((uint32_t*)c->wide_units.p + I, 1);
-      ia.clear((uint32_t*)c->wide_words.p + I, 1);
-    }
+    if (any_mask) ia.clear(c->cover.p, sizeof(CoverCounters) / 4);
     const uint64_t nz = std::max<uint64_t>((uint64_t)I, ia.words());
     hipLaunchKernelGGL(k_init, dim3(blocks_for((int64_t)nz)), dim3(256), 0, s, ia);
   }
-  if (V > 0) {
+  if (V > 0 && !fused) {
     PrepArgs pa{};
     pa.jobs = d_jobs;
     pa.job_vend = d_vend;
     pa.n_jobs = (int)n;
     pa.n_vertices = V;
-    pa.edges = (PolyEdge*)c->edges.p;
+    pa.edges = need_edges ? (PolyEdge*)c->edges.p : nullptr;
     pa.lseg = (uint4*)c->lseg.p;
     pa.item_box = (ItemBox*)c->item_box.p;
     pa.item_last = (unsigned long long*)c->item_last.p;
     pa.item_win = any_at_cache ? (unsigned long long*)c->item_win.p : nullptr;
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(V)), dim3(256), 0, s, pa);
   }
+  DescArgs da{};
   if (I > 0) {
-    DescArgs da{};
     da.jobs = d_jobs;
     da.job_iend = d_iend;
     da.n_jobs = (int)n;
@@ -928,14 +932,21 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     da.desc = (ItemDesc*)c->desc.p;
     da.counts = any_binned ? (uint32_t*)c->counts.p : nullptr;
     da.band_n = any_band ? (uint32_t*)c->band_n.p : nullptr;
-    da.wide_mode = wide_mode;
-    da.wide_units = any_wide ? (uint32_t*)c->wide_units.p : nullptr;
-    da.wide_words = any_wide ? (uint32_t*)c->wide_words.p : nullptr;
+    da.cover = cover;
     da.status = d_status;
     da.item_win = any_at_cache ? (const unsigned long long*)c->item_win.p : nullptr;
     da.at_words = any_at_cache ? (uint32_t*)c->at_words.p : nullptr;
     da.scan_box = any_scan_compact ? (uint2*)c->scan_box.p : nullptr;
-    hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I)), dim3(256), 0, s, da);
+    if (fused) {
+      HIP_TRY(ensure(c->stream, c->masks, std::max<uint64_t>(mask_fixed, 1) * 128));
+      ItemsArgs ia{};
+      ia.d = da;
+      ia.edges = need_edges ? (PolyEdge*)c->edges.p : nullptr;
+      ia.masks = (uint64_t*)c->masks.p;
+      hipLaunchKernelGGL(k_items, dim3(blocks_for(I, kItemsWaves)), dim3(64 * kItemsWaves), 0, s, ia);
+    } else {
+      hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I, kDescBlock)), dim3(kDescBlock), 0, s, da);
+    }
   }
   TileArgs ta{};
   ta.scan_box = any_scan_compact ? (const uint2*)c->scan_box.p : nullptr;
@@ -951,9 +962,9 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     if (capture) {
       words = caps->at_words;
     } else {
-      HIP_TRY(hipMemcpyAsync(&c->host_misc[6], (const uint64_t*)c->at_base.p + I, 8, hipMemcpyDeviceToHost, s));
+      HIP_TRY(hipMemcpyAsync(&c->host_misc[7], (const uint64_t*)c->at_base.p + I, 8, hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
-      words = c->host_misc[6];
+      words = c->host_misc[7];
       c->last_at_words = words;
     }
     if (words > 0 || capture) {
@@ -998,58 +1009,37 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
       HIP_TRY(hipMemcpyAsync(&c->host_misc[2], (const uint64_t*)c->band_base.p + I, 8,
                              hipMemcpyDeviceToHost, s));
   }
-  if (any_wide) {
-    HIP_TRY(ensure(c->stream, c->scan_tmp5, scan_blocks((uint64_t)I + 1) * 8));
-    HIP_TRY(ensure(c->stream, c->scan_tmp6, scan_blocks((uint64_t)I + 1) * 8));
-    exclusive_scan<uint32_t, uint64_t>((const uint32_t*)c->wide_units.p, (uint64_t*)c->wide_ubase.p,
-                                       (uint64_t)I + 1, (uint64_t*)c->scan_tmp5.p, s);
-    exclusive_scan<uint32_t, uint64_t>((const uint32_t*)c->wide_words.p, (uint64_t*)c->wide_wbase.p,
-                                       (uint64_t)I + 1, (uint64_t*)c->scan_tmp6.p, s);
-    if (!capture && !wide_fixed) {
-      HIP_TRY(hipMemcpyAsync(&c->host_misc[4], (const uint64_t*)c->wide_ubase.p + I, 8,
-                             hipMemcpyDeviceToHost, s));
-      HIP_TRY(hipMemcpyAsync(&c->host_misc[5], (const uint64_t*)c->wide_wbase.p + I, 8,
-                             hipMemcpyDeviceToHost, s));
+  if (any_mask && !capture && read_totals)
+    HIP_TRY(hipMemcpyAsync(&c->host_misc[4], c->cover.p, 24, hipMemcpyDeviceToHost, s));
+  if (read_totals) HIP_TRY(hipStreamSynchronize(s));
+  // the masks (assigned in the descriptors before they are copied per pair)
+  c->last_masks = c->last_units = 0;
+  if (any_mask) {
+    uint64_t mask_units = mask_fixed;
+    if (read_totals) {
+      CoverCounters cc{};
+      std::memcpy(&cc, &c->host_misc[4], 24);
+      mask_units = cc.mask_units;
+      c->last_masks = mask_units;
+      c->last_units = std::max(cc.n_wave, cc.n_block);
+      if (mask_units > UINT32_MAX) return rz::fail(RZ_CAPACITY_ERROR, "more than 512 GiB of coverage masks in one call");
+      if (c->last_units > unit_cap) {
+        // windows past the lists: lists of the right size, assigned again
+        unit_cap = c->last_units;
+        if (rz_status st = place_cover()) return st;
+        zero_words(c->cover.p, sizeof(CoverCounters) / 4, s);
+        da.cover = cover;
+        hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I, kDescBlock)), dim3(kDescBlock), 0, s, da);
+      }
+    } else if (!capture) {
+      c->last_masks = mask_fixed;
+      c->last_units = unit_cap;
     }
-  }
-  if (!capture && (any_binned || any_band || (any_wide && !wide_fixed))) HIP_TRY(hipStreamSynchronize(s));
-  // wide pre-pass: unit list, flags and mask bases (before the descriptors
-  // are copied per pair).  The masks take at most 2 bytes per output pixel
-  // (16 overlapping wide items per pixel at one bit); items past that stay
-  // per tile.
-  uint64_t wide_units = 0, wide_words = 0;
-  c->last_wide_units = c->last_wide_words = 0;
-  if (any_wide) {
-    // (wide_fixed: the most the masks may hold, from the output size; the
-    // actual totals stay on the device, where k_wide_assign and k_wide_cover
-    // read them)
-    const uint64_t words_cap = std::max<uint64_t>(out_px / 4, (uint64_t)1 << 20);
-    wide_units = capture ? caps->wide_units : (wide_fixed ? words_cap / 16 : c->host_misc[4]);
-    wide_words = capture ? caps->wide_words : (wide_fixed ? words_cap : c->host_misc[5]);
-    c->last_wide_units = wide_units;
-    c->last_wide_words = wide_words;
-    if (!masks_only) wide_words = std::min<uint64_t>(wide_words, words_cap);
-    wide_words = std::min<uint64_t>(wide_words, (uint64_t)1 << 36);  // ItemDesc::wide holds words / 16
-    if (wide_units > 0 && wide_words > 0) {
-      HIP_TRY(ensure(c->stream, c->wide_item, wide_units * 4));
-      HIP_TRY(ensure(c->stream, c->wide_masks, wide_words * 8));
-      WideAssignArgs wa{};
-      wa.desc = (ItemDesc*)c->desc.p;
-      wa.n_items = I;
-      wa.wide_units = (const uint32_t*)c->wide_units.p;
-      wa.unit_base = (const uint64_t*)c->wide_ubase.p;
-      wa.word_base = (const uint64_t*)c->wide_wbase.p;
-      wa.unit_cap = wide_units;
-      wa.word_cap = wide_words;
-      wa.unit_item = (uint32_t*)c->wide_item.p;
-      hipLaunchKernelGGL(k_wide_assign, dim3(blocks_for(I)), dim3(256), 0, s, wa);
-    } else {
-      wide_units = 0;
-    }
+    HIP_TRY(ensure(c->stream, c->masks, std::max<uint64_t>(mask_units, 1) * 128));
   }
   c->last_band_entries = c->last_band_edges = 0;
   if (any_band) {
-    // edge bands of long polygon rings (see kBandMinEdges)
+    // edge bands of long lines (see kLineBandMinSegs)
     const uint64_t nb = capture ? caps->band_entries : c->host_misc[2];
     c->last_band_entries = nb;
     if (nb > 0) {
@@ -1070,11 +1060,9 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
       bd.band_n = (const uint32_t*)c->band_n.p;
       bd.items = (const uint32_t*)c->band_items.p;
       bd.n_list = n_list;
-      bd.edges = (const PolyEdge*)c->edges.p;
       bd.lseg = (const uint4*)c->lseg.p;
       bd.band_cnt = (uint32_t*)c->band_cnt.p;
       bd.band_off = (const uint64_t*)c->band_off.p;
-      bd.band_edges = nullptr;
       bd.band_segs = nullptr;
       bd.edge_cap = 0;
       bd.status = d_status;
@@ -1092,54 +1080,14 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
         ne = c->host_misc[3];
       }
       c->last_band_edges = ne;
-      // polygon and line entries share one index space; each kind's
-      // records go to an array of its own record size
-      if (any_poly_band) {
-        HIP_TRY(ensure(c->stream, c->band_edges, std::max<uint64_t>(ne, 1) * sizeof(PolyEdge)));
-        bd.band_edges = (PolyEdge*)c->band_edges.p;
-      }
-      if (any_line_band) {
-        HIP_TRY(ensure(c->stream, c->band_segs, std::max<uint64_t>(ne, 1) * sizeof(uint4)));
-        bd.band_segs = (uint4*)c->band_segs.p;
-      }
+      HIP_TRY(ensure(c->stream, c->band_segs, std::max<uint64_t>(ne, 1) * sizeof(uint4)));
+      bd.band_segs = (uint4*)c->band_segs.p;
       bd.edge_cap = ne;
       if (ne > 0) hipLaunchKernelGGL(k_band_scatter, dim3(bgrid), dim3(256), 0, s, bd);
       ta.band_off = (const uint64_t*)c->band_off.p;
-      ta.band_edges = bd.band_edges;
       ta.band_segs = bd.band_segs;
     }
   }
-  // the wide pre-pass (after the bands it reads)
-  // (with heavy tiles: their counts, slot bases, pair lists and slots, so the
-  // wide items' masks also land in the heavy slots)
-  auto launch_wide = [&](const uint32_t* h_cnt, const uint64_t* h_base, const uint32_t* w_j,
-                         uint64_t* masks, uint32_t slot_words) {
-    if (wide_units > 0) {
-      WideCoverArgs wc{};
-      wc.jobs = d_jobs;
-      wc.desc = (const ItemDesc*)c->desc.p;
-      wc.n_items = I;
-      wc.unit_item = (const uint32_t*)c->wide_item.p;
-      wc.unit_base = (const uint64_t*)c->wide_ubase.p;
-      wc.n_units = (const uint64_t*)c->wide_ubase.p + I;
-      wc.unit_cap = wide_units;
-      wc.edges = (const PolyEdge*)c->edges.p;
-      wc.band_off = ta.band_off;
-      wc.band_edges = ta.band_edges;
-      wc.wide_masks = (uint64_t*)c->wide_masks.p;
-      wc.cov_mode = cov_mode;
-      wc.heavy_cnt = h_cnt;
-      wc.heavy_base = h_base;
-      wc.pair_off = (const uint64_t*)c->offsets.p;
-      wc.pair_cap = n_pairs;
-      wc.wide_j = w_j;
-      wc.masks = masks;
-      wc.slot_words = slot_words;
-      const uint32_t wgrid = (uint32_t)std::min<uint64_t>((wide_units + 3) / 4, wide_fixed ? 512 : 4096);
-      hipLaunchKernelGGL(k_wide_cover, dim3(wgrid), dim3(256), 0, s, wc);
-      ta.wide_masks = (const uint64_t*)c->wide_masks.p;
-    }
-  };
   if (any_binned) {
     const uint64_t* d_total = (const uint64_t*)c->offsets.p + I;
     n_pairs = capture ? caps->pairs : c->host_misc[0];
@@ -1198,78 +1146,27 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     ta.pair_desc = (const ItemDesc*)c->pair_desc.p;
     if (stage_ev) HIP_TRY(hipEventRecord(c->ev[3], s));
 
-    // heavy tiles (kHeavyItems items or more): coverage masks precomputed in
-    // parallel, one wave per (item, strip); the buffers are sized for every
-    // pair so no host round trip is needed
-    // the batch's class: that of its widest-tile / most-tiles group
-    const Tuning bt = tuning_for(size_class(max_tile_w, n_tiles, n_pairs));
-    const uint32_t heavy_min = bt.heavy_min ? bt.heavy_min : kHeavyItems;
-    if (n_pairs >= heavy_min) {
-      HIP_TRY(ensure(c->stream, c->heavy_cnt, ((size_t)n_tiles + 1) * 4));
-      HIP_TRY(ensure(c->stream, c->heavy_base, ((size_t)n_tiles + 1) * 8));
-      HIP_TRY(ensure(c->stream, c->scan_tmp4, scan_blocks((uint64_t)n_tiles + 1) * 8));
-      // heavy flags, their ranks and the ordered list of heavy tiles
-      HIP_TRY(ensure(c->stream, c->heavy_list, ((size_t)n_tiles + 1) * 4 * 3));
-      uint32_t* h_flag = (uint32_t*)c->heavy_list.p;
-      uint32_t* h_rank = h_flag + (n_tiles + 1);
-      uint32_t* h_list = h_rank + (n_tiles + 1);
-      HIP_TRY(ensure(c->stream, c->scan_tmp7, scan_blocks((uint64_t)n_tiles + 1) * 4));
-      hipLaunchKernelGGL(k_heavy_count, dim3(blocks_for((int64_t)n_tiles + 1)), dim3(256), 0, s,
-                         (const uint32_t*)c->tile_off.p, n_tiles, heavy_min,
-                         (uint32_t*)c->heavy_cnt.p, h_flag);
-      exclusive_scan<uint32_t, uint32_t>(h_flag, h_rank, (uint64_t)n_tiles + 1, (uint32_t*)c->scan_tmp7.p, s);
-      hipLaunchKernelGGL(k_heavy_list, dim3(blocks_for((int64_t)n_tiles)), dim3(256), 0, s,
-                         (const uint32_t*)h_flag, (const uint32_t*)h_rank, n_tiles, h_list);
-      ta.heavy_list = h_list;
-      ta.heavy_rank = h_rank;
-      exclusive_scan<uint32_t, uint64_t>((const uint32_t*)c->heavy_cnt.p, (uint64_t*)c->heavy_base.p,
-                                         (uint64_t)n_tiles + 1, (uint64_t*)c->scan_tmp4.p, s);
-      const uint32_t slot_words = 16u * (uint32_t)(max_tile_w / 64);
-      HIP_TRY(ensure(c->stream, c->cover_list, (size_t)n_pairs * 4 + 4));
-      HIP_TRY(ensure(c->stream, c->wide_j, (size_t)n_pairs * 4));
-      HIP_TRY(ensure(c->stream, c->masks, (size_t)n_pairs * 4 * slot_words * 8));
-      uint32_t* cover_count = (uint32_t*)c->cover_list.p + n_pairs;
-      zero_words(cover_count, 1, s);
-      hipLaunchKernelGGL(k_heavy_pairs, dim3(blocks_for((int64_t)n_pairs, kHeavyPairsBlock)),
-                         dim3(kHeavyPairsBlock), 0, s, d_jobs,
-                         sorted_keys, sorted_vals, (const ItemDesc*)c->pair_desc.p, d_total, n_pairs,
-                         (const uint32_t*)c->tile_off.p, (const uint64_t*)c->heavy_base.p,
-                         (const uint64_t*)c->offsets.p, (uint32_t*)c->wide_j.p, (uint32_t*)c->cover_list.p,
-                         cover_count, n_tiles);
-      CoverArgs ca{};
-      ca.jobs = d_jobs;
-      ca.job_tend = d_tend;
-      ca.n_jobs = (int)n;
-      ca.pair_tile = sorted_keys;
-      ca.pair_desc = (const ItemDesc*)c->pair_desc.p;
-      ca.heavy_base = (const uint64_t*)c->heavy_base.p;
-      ca.cover_list = (const uint32_t*)c->cover_list.p;
-      ca.cover_count = cover_count;
-      ca.n_tiles = n_tiles;
-      ca.edges = (const PolyEdge*)c->edges.p;
-      ca.band_off = ta.band_off;
-      ca.band_edges = ta.band_edges;
-      ca.tile_off = (const uint32_t*)c->tile_off.p;
-      ca.masks = (uint64_t*)c->masks.p;
-      ca.slot_words = slot_words;
-      launch_wide((const uint32_t*)c->heavy_cnt.p, (const uint64_t*)c->heavy_base.p,
-                  (const uint32_t*)c->wide_j.p, (uint64_t*)c->masks.p, slot_words);
-      const uint32_t cgrid = (uint32_t)std::min<uint64_t>(n_pairs, 2048);
-      if (any_tw64) hipLaunchKernelGGL(k_cover<1>, dim3(cgrid), dim3(256), 0, s, ca);
-      if (any_tw256) hipLaunchKernelGGL(k_cover<4>, dim3(cgrid), dim3(256), 0, s, ca);
-      ta.heavy_base = (const uint64_t*)c->heavy_base.p;
-      ta.masks = (const uint64_t*)c->masks.p;
-      ta.slot_words = slot_words;
-      ta.heavy_min = heavy_min;
-    } else {
-      launch_wide(nullptr, nullptr, nullptr, nullptr, 0);
+  } else if (stage_ev) {
+    HIP_TRY(hipEventRecord(c->ev[2], s));
+    HIP_TRY(hipEventRecord(c->ev[3], s));
+  }
+  if (any_mask) {
+    CoverArgs ca{};
+    ca.jobs = d_jobs;
+    ca.desc = (const ItemDesc*)c->desc.p;
+    ca.cover = cover;
+    ca.masks = (uint64_t*)c->masks.p;
+    // at most as many workgroups as fill the chip (6 and 4 to a CU: the
+    // lists' lengths are on the device)
+    if (max_poly_nv > kCoverBlockNv) {
+      const uint64_t g = read_totals ? std::max<uint64_t>(c->last_units, 1) : 1024;
+      hipLaunchKernelGGL(k_cover<true>, dim3((unsigned)std::min<uint64_t>(g, 1024)), dim3(256), 0, s, ca);
     }
+    const uint64_t g = ((uint64_t)I + (read_totals ? c->last_units : 0)) / 4 + 1;
+    hipLaunchKernelGGL(k_cover<false>, dim3((unsigned)std::min<uint64_t>(g, 1536)), dim3(256), 0, s, ca);
+    ta.masks = (const uint64_t*)c->masks.p;
   } else {
-    if (stage_ev) {
-      HIP_TRY(hipEventRecord(c->ev[2], s));
-      HIP_TRY(hipEventRecord(c->ev[3], s));
-    }
-    launch_wide(nullptr, nullptr, nullptr, nullptr, 0);
+    ta.masks = (const uint64_t*)c->misc.p;  // (read, never used: the tile kernels load ahead)
   }
   if (masks_only) return RZ_OK;
   if (c->profiling) HIP_TRY(hipEventRecord(c->ev[4], s));
@@ -1279,23 +1176,28 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   ta.job_tend = d_tend;
   ta.n_jobs = (int)n;
   ta.desc = (const ItemDesc*)c->desc.p;
-  ta.edges = (const PolyEdge*)c->edges.p;
+  ta.edges = need_edges ? (const PolyEdge*)c->edges.p : nullptr;
   ta.lseg = (const uint4*)c->lseg.p;
   ta.burns = c->profiling == 2 ? d_burns : nullptr;
   ta.status = d_status;
+  auto small = [&](const Group& q) { return !q.lines && q.t_hi - q.t_lo <= kBlockTiles; };
   for (size_t g = 0; g < groups.size(); ++g) {
     if (groups[g].t_hi == groups[g].t_lo) continue;
     ta.t_lo = groups[g].t_lo;
+    if (small(groups[g])) {  // ... or one launch for all neighbouring groups of few tiles
+      while (g + 1 < groups.size() && groups[g + 1].dtype == groups[g].dtype && small(groups[g + 1]) &&
+             groups[g + 1].t_lo == groups[g].t_hi)
+        ++g;
+      ta.t_hi = groups[g].t_hi;
+      launch_blocks_dispatch(groups[g].dtype, ta, s);
+      continue;
+    }
     ta.t_hi = groups[g].t_hi;
     ta.queue = (uint32_t*)c->queue.p + g * kQueueWords;
-    ta.heavy_ctr = (uint32_t*)c->queue.p + groups.size() * kQueueWords + g;
-    // polygon-only groups leave their heavy tiles to k_tile_heavy
-    ta.heavy_split = (ta.heavy_base && !groups[g].lines) ? 1 : 0;
     const uint64_t gt = groups[g].t_hi - groups[g].t_lo;
     ta.chunk = tuning_for(size_class(tile_w((int)rz_dtype_size(groups[g].dtype)), gt,
                                      n_tiles ? n_pairs * gt / n_tiles : 0)).chunk;
     launch_tile_dispatch(groups[g].dtype, groups[g].fun, ta, groups[g].lines, s);
-    if (ta.heavy_split) launch_heavy_dispatch(groups[g].dtype, groups[g].fun, ta, s);
   }
   HIP_TRY(hipGetLastError());
   if (c->profiling) HIP_TRY(hipEventRecord(c->ev[5], s));
@@ -1353,7 +1255,7 @@ extern "C" rz_status rz_batch_graph_create(int device, const rz_job* jobs, int64
   }
   auto grow = [&](uint64_t v) { return (uint64_t)((double)v * headroom) + (v ? 64 : 0); };
   const BatchCaps caps{grow(c->last_pairs),      grow(c->last_band_entries), grow(c->last_band_edges),
-                       grow(c->last_wide_units), grow(c->last_wide_words),   grow(c->last_at_words)};
+                       grow(c->last_masks),      grow(c->last_units),        grow(c->last_at_words)};
   // 2. a pass at those capacities allocates every buffer, so the captured
   // pass allocates nothing; 3. capture
   st = run_batch(c, jobs, n_jobs, &caps);
@@ -1565,7 +1467,7 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
   };
   const size_t o_tab = take(sizeof(JobDev) + 3 * sizeof(int64_t));
   const size_t o_misc = take(64 + kBurnSlots * sizeof(unsigned long long));
-  const size_t o_queue = take((kQueueWords + 1) * 4);
+  const size_t o_queue = take(kQueueWords * 4);
   const size_t o_box = take((size_t)std::max<int64_t>(I, 1) * sizeof(ItemBox));
   const size_t o_last = take((size_t)std::max<int64_t>(I, 1) * 8);
   const size_t o_desc = take((size_t)std::max<int64_t>(I, 1) * sizeof(ItemDesc));
@@ -1597,7 +1499,7 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
     ia.last = d_last;
     ia.n_items = I;
     ia.clear(d_status, 16);
-    ia.clear(d_queue, kQueueWords + 1);
+    ia.clear(d_queue, kQueueWords);
     const uint64_t nz = std::max<uint64_t>((uint64_t)I, ia.words());
     hipLaunchKernelGGL(k_init, dim3(blocks_for((int64_t)nz)), dim3(256), 0, s, ia);
   }
@@ -1623,9 +1525,8 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
     da.item_box = d_box;
     da.item_last = d_last;
     da.desc = d_desc;
-    da.wide_mode = 1;
     da.status = d_status;
-    hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I)), dim3(256), 0, s, da);
+    hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I, kDescBlock)), dim3(kDescBlock), 0, s, da);
   }
   TileArgs ta{};
   std::memset(&ta, 0, sizeof(ta));
@@ -1634,13 +1535,14 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
   ta.n_jobs = 1;
   ta.desc = d_desc;
   ta.edges = dg->has_poly ? (const PolyEdge*)(base + o_edges) : nullptr;
+  ta.masks = (const uint64_t*)d_status;  // (read, never used)
   ta.lseg = lines ? (const uint4*)(base + o_lseg) : nullptr;
   ta.status = d_status;
   ta.t_lo = 0;
   ta.t_hi = (uint32_t)jt;
   ta.queue = d_queue;
-  ta.heavy_ctr = d_queue + kQueueWords;
-  launch_tile_dispatch(dtype, (int)fun, ta, lines, s);
+  if (!lines && ta.t_hi - ta.t_lo <= kBlockTiles) launch_blocks_dispatch(dtype, ta, s);
+  else launch_tile_dispatch(dtype, (int)fun, ta, lines, s);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s));
   uint32_t flags = 0;

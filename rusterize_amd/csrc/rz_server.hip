@@ -51,8 +51,9 @@ struct Request {
 // Workspace a request may need (run_batch's buffers): per vertex its edge or
 // segment record and band copies (64 B); per item its box, statistics,
 // descriptor, scan entries and, per tile its box covers, a bin pair with its
-// sort copies, gathered descriptor and heavy-tile masks (4 x 2 KiB at most);
-// per output pixel at most 2 B of wide-pre-pass masks and the tile tables.
+// sort copies, gathered descriptor and coverage masks (2 KiB at most, and as
+// much again per item where a call takes a fixed capacity); per output pixel
+// at most 2 B of masks and the tile tables.
 size_t workspace_estimate(const rz_job& j) {
   const rz_device_geometry* g = j.geometry;
   const size_t nl = j.layer_dev ? j.n_layers : 1u;

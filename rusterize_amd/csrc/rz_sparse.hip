@@ -13,9 +13,8 @@
 // segment's cells in Bresenham order and the end cell last; points in order.
 //
 // Work units, in that order: a polygon item's 16-row strips (its coverage
-// masks come from the wide pre-pass, run for every polygon item over its
-// whole box), a line or point item's vertices (one segment or point each),
-// and a line of a job with xres != yres as a whole (LineWriter + PixelCache,
+// masks come from k_cover), a line or point item's vertices (one segment or
+// point each), and a line of a job with xres != yres as a whole (LineWriter + PixelCache,
 // burn_geometry.rs:179-185, 202-208: the first visit of each pixel only, in
 // write order, so such a line is walked sequentially).  A count pass sizes
 // every unit, an exclusive scan places it, and the emit pass writes it.
@@ -41,7 +40,7 @@ struct SparseArgs {
   int64_t n_items;
   const uint64_t* ubase;       // [n_items + 1] first unit of each position
   const uint4* lseg;           // line / point vertex records
-  const uint64_t* wide_masks;
+  const uint64_t* masks;
   uint32_t* counts;            // [units] triplets of each unit (count pass)
   const uint64_t* toff;        // [units + 1] first triplet of each unit (emit pass)
   uint64_t* rows;              // [triplets] (emit pass)
@@ -80,7 +79,7 @@ __global__ void k_sp_units(SparseArgs a, uint32_t* n_units, uint64_t* nbits) {
   uint32_t n = 0;
   uint64_t b = 0;
   if (kind == 0) {
-    n = boxed && (d.flags & kItemWide) ? (uint32_t)wide_strip_count(d.r0, d.r1) : 0u;
+    n = boxed && (d.flags & kItemMask) ? (uint32_t)mask_strip_count(d.r0, d.r1) : 0u;
     if (boxed) n += sp_outline_units(a, d);
     CacheWin cw;
     if (boxed && a.at && a.at_dedup && item_cache(a.item_win, (int64_t)d.last, cw)) {
@@ -220,9 +219,11 @@ __global__ void k_sp_dedup(SparseArgs a) {
   if (!EMIT) a.counts[u] = (uint32_t)n;
 }
 
-// Polygon units, one wave each (grid-stride): the strip's 16 mask rows, each
-// read left to right; the wave takes 64 words of a row at a time and places
-// each word's bits after the popcounts of the words before it.
+// Polygon units, one wave each (grid-stride): the strip's 16 rows, each read
+// left to right, 64 columns (one mask block, a lane per column) at a time; a
+// covered column's triplet goes after those of the columns before it.  The
+// blocks of up to kSpBlocks columns of 64 are loaded once for all rows.
+constexpr int kSpBlocks = 4;
 template <bool EMIT>
 __global__ __launch_bounds__(256) void k_sp_polys(SparseArgs a, uint64_t n_units) {
   const int lane = threadIdx.x & 63;
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(256) void k_sp_polys(SparseArgs a, uint64_t n_units
     const uint32_t n_out = sp_outline_units(a, d);
     if (u - a.ubase[p] < (uint64_t)n_out) continue;  // an outline unit
     const int32_t k = (int32_t)(u - a.ubase[p] - n_out);
-    const int32_t nw = wide_row_words(d.c0, d.c1);
+    const int32_t nw = mask_row_words(d.c0, d.c1);
     // all-touched sum / count: the fill skips pixels the outline's cache
     // contains (FillWriter, writers.rs:38-60): inside the cache window the
     // pixel's own bit, outside it the bit its wrapped index lands on
@@ -242,32 +243,29 @@ __global__ __launch_bounds__(256) void k_sp_polys(SparseArgs a, uint64_t n_units
     const bool filter = a.at && a.at_dedup && item_cache(a.item_win, (int64_t)d.last, cw) &&
                         cw.cap <= ((uint64_t)1 << 34);
     const uint64_t* cbits = filter ? a.bits + a.bit_base[p] : nullptr;
-    const uint64_t* m = a.wide_masks + (uint64_t)d.wide * 16u + (uint64_t)k * 16u * (uint64_t)nw;
+    const uint16_t* m = reinterpret_cast<const uint16_t*>(a.masks + ((uint64_t)d.mask + (uint64_t)k * (uint64_t)nw) * 16u) +
+                        mask_element(lane);
     const int32_t Rw = ((d.r0 >> 4) + k) * WAVE_ROWS, C = (d.c0 >> 6) * 64;
     uint64_t o = EMIT ? a.toff[u] : 0, n = 0;
-    for (int32_t r = 0; r < WAVE_ROWS; ++r) {
-      for (int32_t w0 = 0; w0 < nw; w0 += 64) {
-        const int32_t w = w0 + lane;
-        uint64_t word = w < nw ? m[(uint64_t)r * nw + (uint64_t)w] : 0ull;
-        if (filter) {
-          for (uint64_t b = word; b; b &= b - 1) {
-            const int bit = __builtin_ctzll(b);
-            const uint64_t ci = cache_index(cw, (int64_t)(C + w * 64 + bit), (int64_t)(Rw + r));
-            if (ci < cw.cap && ((cbits[ci >> 6] >> (ci & 63)) & 1ull)) word &= ~(1ull << bit);
-          }
-        }
-        uint32_t c = (uint32_t)__popcll(word), x = c;
+    uint32_t block[kSpBlocks];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const uint32_t y = (uint32_t)__shfl_up((int)x, off, 64);
-          if (lane >= off) x += y;
+    for (int j = 0; j < kSpBlocks; ++j) block[j] = j < nw ? (uint32_t)m[(uint64_t)j * 64u] : 0u;
+    for (int32_t r = 0; r < WAVE_ROWS; ++r) {
+      auto row_block = [&](int32_t w, uint32_t bits) {
+        bool on = (bits >> r) & 1u;
+        const int64_t col = (int64_t)C + w * 64 + lane;
+        if (filter && on) {
+          const uint64_t ci = cache_index(cw, col, (int64_t)(Rw + r));
+          if (ci < cw.cap && ((cbits[ci >> 6] >> (ci & 63)) & 1ull)) on = false;
         }
-        if (EMIT && word) {
-          uint64_t q = o + n + (x - c);
-          for (uint64_t b = word; b; b &= b - 1) sp_put(a, q++, Rw + r, C + w * 64 + __builtin_ctzll(b), d.value);
-        }
-        n += (uint32_t)__shfl((int)x, 63, 64);
-      }
+        const uint64_t b = __ballot(on);
+        if (EMIT && on) sp_put(a, o + n + (uint64_t)__popcll(b & ((1ull << lane) - 1ull)), Rw + r, col, d.value);
+        n += (uint64_t)__popcll(b);
+      };
+#pragma unroll
+      for (int j = 0; j < kSpBlocks; ++j)
+        if (j < nw) row_block(j, block[j]);
+      for (int32_t w = kSpBlocks; w < nw; ++w) row_block(w, (uint32_t)m[(uint64_t)w * 64u]);
     }
     if (!EMIT && lane == 0) a.counts[u] = (uint32_t)n;
   }
@@ -501,7 +499,7 @@ static rz_status sparse_build(rz_context* c, const rz_job& j, rz_sparse* sp) {
   a.perm = perm;
   a.n_items = I;
   a.lseg = (const uint4*)c->lseg.p;
-  a.wide_masks = (const uint64_t*)c->wide_masks.p;
+  a.masks = (const uint64_t*)c->masks.p;
   a.esz = (int)rz_dtype_size(j.dtype);
   a.dedup = j.info.xres != j.info.yres;
   a.at = j.all_touched ? 1 : 0;
@@ -511,24 +509,24 @@ static rz_status sparse_build(rz_context* c, const rz_job& j, rz_sparse* sp) {
   const bool whole = a.dedup || a.at_dedup;  // items walked whole, with first-visit bits
   HIP_TRY(ensure(s, c->counts, (size_t)(I + 1) * 4));
   HIP_TRY(ensure(s, c->offsets, (size_t)(I + 1) * 8));
-  HIP_TRY(ensure(s, c->band_base, (size_t)(I + 1) * 8));  // dedup bits per position
-  HIP_TRY(ensure(s, c->heavy_base, (size_t)(I + 1) * 8)); // their scan
+  HIP_TRY(ensure(s, c->sp_bitn, (size_t)(I + 1) * 8));  // dedup bits per position
+  HIP_TRY(ensure(s, c->sp_bit_base, (size_t)(I + 1) * 8)); // their scan
   HIP_TRY(ensure(s, c->scan_tmp, scan_blocks((uint64_t)I + 1) * 8));
   InitArgs ia{};
   std::memset(&ia, 0, sizeof(ia));
   ia.clear((uint32_t*)c->counts.p + I, 1);
-  ia.clear((uint64_t*)c->band_base.p + I, 2);
+  ia.clear((uint64_t*)c->sp_bitn.p + I, 2);
   hipLaunchKernelGGL(k_init, dim3(1), dim3(256), 0, s, ia);
   hipLaunchKernelGGL(k_sp_units, dim3(blocks_for(I)), dim3(256), 0, s, a, (uint32_t*)c->counts.p,
-                     whole ? (uint64_t*)c->band_base.p : nullptr);
+                     whole ? (uint64_t*)c->sp_bitn.p : nullptr);
   exclusive_scan<uint32_t, uint64_t>((const uint32_t*)c->counts.p, (uint64_t*)c->offsets.p, (uint64_t)I + 1,
                                      (uint64_t*)c->scan_tmp.p, s);
   a.ubase = (const uint64_t*)c->offsets.p;
   uint64_t n_bits_words = 0;
   if (whole) {
-    exclusive_scan<uint64_t, uint64_t>((const uint64_t*)c->band_base.p, (uint64_t*)c->heavy_base.p,
+    exclusive_scan<uint64_t, uint64_t>((const uint64_t*)c->sp_bitn.p, (uint64_t*)c->sp_bit_base.p,
                                        (uint64_t)I + 1, (uint64_t*)c->scan_tmp.p, s);
-    HIP_TRY(hipMemcpyAsync(&c->host_misc[1], (const uint64_t*)c->heavy_base.p + I, 8, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(&c->host_misc[1], (const uint64_t*)c->sp_bit_base.p + I, 8, hipMemcpyDeviceToHost, s));
   }
   HIP_TRY(hipMemcpyAsync(&c->host_misc[0], (const uint64_t*)c->offsets.p + I, 8, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
@@ -536,14 +534,14 @@ static rz_status sparse_build(rz_context* c, const rz_job& j, rz_sparse* sp) {
   if (whole) n_bits_words = c->host_misc[1];
   if (U >= ((uint64_t)1 << 32)) return rz::fail(RZ_CAPACITY_ERROR, "more than 2^32 sparse work units");
   // 3. triplets per unit, then their places
-  HIP_TRY(ensure(s, c->cover_list, (size_t)(U + 1) * 4));   // counts per unit
-  HIP_TRY(ensure(s, c->heavy_list, (size_t)(U + 1) * 8));   // their scan
+  HIP_TRY(ensure(s, c->sp_counts, (size_t)(U + 1) * 4));   // counts per unit
+  HIP_TRY(ensure(s, c->sp_first, (size_t)(U + 1) * 8));   // their scan
   HIP_TRY(ensure(s, c->scan_tmp2, scan_blocks(U + 1) * 8));
-  a.counts = (uint32_t*)c->cover_list.p;
+  a.counts = (uint32_t*)c->sp_counts.p;
   if (whole) {
-    HIP_TRY(ensure(s, c->wide_item, std::max<uint64_t>(2 * n_bits_words, 1) * 8));  // count + emit halves
-    a.bits = (uint64_t*)c->wide_item.p;
-    a.bit_base = (const uint64_t*)c->heavy_base.p;
+    HIP_TRY(ensure(s, c->sp_bits, std::max<uint64_t>(2 * n_bits_words, 1) * 8));  // count + emit halves
+    a.bits = (uint64_t*)c->sp_bits.p;
+    a.bit_base = (const uint64_t*)c->sp_bit_base.p;
   }
   InitArgs ib{};
   std::memset(&ib, 0, sizeof(ib));
@@ -557,8 +555,8 @@ static rz_status sparse_build(rz_context* c, const rz_job& j, rz_sparse* sp) {
     hipLaunchKernelGGL(k_sp_polys<false>, dim3((unsigned)std::min<uint64_t>((U + 3) / 4, 4096)), dim3(256), 0, s,
                        a, U);
   }
-  exclusive_scan<uint32_t, uint64_t>(a.counts, (uint64_t*)c->heavy_list.p, U + 1, (uint64_t*)c->scan_tmp2.p, s);
-  a.toff = (const uint64_t*)c->heavy_list.p;
+  exclusive_scan<uint32_t, uint64_t>(a.counts, (uint64_t*)c->sp_first.p, U + 1, (uint64_t*)c->scan_tmp2.p, s);
+  a.toff = (const uint64_t*)c->sp_first.p;
   HIP_TRY(ensure(s, c->tile_off, ((size_t)nl + 1) * 8));
   hipLaunchKernelGGL(k_sp_bands, dim3(blocks_for((int64_t)nl + 1)), dim3(256), 0, s, a.desc, perm, I, a.ubase,
                      a.toff, nl, (uint64_t*)c->tile_off.p);

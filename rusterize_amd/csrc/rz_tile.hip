@@ -1,315 +1,402 @@
-// rz_tile.hip -- coverage pre-passes of the tile kernel: heavy-tile lists
-// and masks (k_heavy_*, k_cover) and the wide pre-pass (k_wide_cover).
+// rz_tile.hip -- the coverage pre-pass of the tile kernel (k_cover).
 #pragma once
 
 #include "rz_device.h"
 
 namespace rzk {
 
-// ---------------------------------------------------------- heavy tiles --
-//
-// A tile with at least kHeavyItems items would serialise all their coverage
-// work in its four strip waves.  For such tiles the coverage masks of every
-// (polygon item, strip) are computed beforehand by k_cover, one wave per
-// (item, strip), in parallel; the tile kernel then only folds the masks in
-// geometry order (every pixel function, ordered sum included, stays exact).
-
-// Items of every heavy tile (0 for the others) and its heavy flag.
-__global__ void k_heavy_count(const uint32_t* tile_off, uint32_t n_tiles, uint32_t min_items,
-                              uint32_t* heavy_cnt, uint32_t* heavy_flag) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t > n_tiles) return;
-  uint32_t c = 0;
-  if (t < n_tiles) {
-    c = tile_off[t + 1] - tile_off[t];
-    if (c < min_items) c = 0;
+// Transposes the four 16 x 16 bit blocks of 16 lanes' words: lane i (of each
+// 16) gives row i's 64 columns and gets, in 16-bit element j, the rows' bits
+// of column 16 j + i (mask_element's order).  Four exchanges with the lane 8,
+// 4, 2 and 1 away, each a rotate and a bit select per half.
+template <int S>
+__device__ inline uint32_t exchange16(uint32_t x, int lane) {
+  constexpr uint32_t M = S == 8 ? 0x00FF00FFu : (S == 4 ? 0x0F0F0F0Fu : (S == 2 ? 0x33333333u : 0x55555555u));
+  int y;
+  if constexpr (S == 8) {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror:8
+  } else if constexpr (S == 4) {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xF, 0x5, false);  // row_shl:4 into banks 0, 2
+    y = __builtin_amdgcn_update_dpp(y, (int)x, 0x114, 0xF, 0xA, false);  // row_shr:4 into banks 1, 3
+  } else {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, S == 2 ? 0x4E : 0xB1, 0xF, 0xF, false);  // quad_perm
   }
-  heavy_cnt[t] = c;
-  heavy_flag[t] = c > 0 ? 1u : 0u;
+  const bool up = (lane & S) != 0;
+  const uint32_t K = up ? ~M : M;
+  const uint32_t r = __builtin_amdgcn_alignbit((uint32_t)y, (uint32_t)y, up ? (uint32_t)S : 32u - (uint32_t)S);
+  return (x & K) | (r & ~K);
+}
+__device__ inline uint64_t transpose16(uint64_t x, int lane) {
+  uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
+  lo = exchange16<1>(exchange16<2>(exchange16<4>(exchange16<8>(lo, lane), lane), lane), lane);
+  hi = exchange16<1>(exchange16<2>(exchange16<4>(exchange16<8>(hi, lane), lane), lane), lane);
+  return (uint64_t)lo | ((uint64_t)hi << 32);
 }
 
-// The heavy tiles in tile order: heavy_list[heavy_rank[t]] = t, so the heavy
-// tiles of tiles [t_lo, t_hi) are heavy_list[heavy_rank[t_lo] .. heavy_rank[t_hi]).
-__global__ void k_heavy_list(const uint32_t* heavy_flag, const uint32_t* heavy_rank, uint32_t n_tiles,
-                             uint32_t* heavy_list) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n_tiles && heavy_flag[t]) heavy_list[heavy_rank[t]] = t;
-}
-
-// The compact list of the pairs of heavy tiles that hold polygon items other
-// than wide ones (the only ones k_cover writes; k_wide_cover writes the wide
-// ones), appended with one atomic per block.  For a wide item's pair it also
-// records the item's place in the tile's pair list, at the pair's emission
-// index (k_bin_emit's order over the item's tile rectangle), where
-// k_wide_cover finds it with one load.
-constexpr int kHeavyPairsBlock = 1024;
-__global__ __launch_bounds__(kHeavyPairsBlock) void k_heavy_pairs(const JobDev* jobs, const uint32_t* pair_tile,
-                              const uint32_t* pair_item, const ItemDesc* pair_desc, const uint64_t* n_pairs, uint64_t cap,
-                              const uint32_t* tile_off, const uint64_t* heavy_base, const uint64_t* pair_off,
-                              uint32_t* wide_j, uint32_t* cover_list, uint32_t* cover_count, uint32_t n_tiles) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  bool poly = false;
-  if (i < min(*n_pairs, cap)) {
-    const uint32_t t = pair_tile[i];
-    // (a key past every tile: a slot of a captured batch whose pairs outgrew
-    // its capacity, whose tile lists are then all empty)
-    if (t < n_tiles && heavy_base[t + 1] > heavy_base[t]) {
-      const ItemDesc& d = pair_desc[i];
-      poly = (d.kind_layer & 3u) == 0u && !(d.flags & kItemWide);  // k_wide_cover writes those
-      int32_t tx0, tx1, ty0, ty1;
-      if ((d.flags & kItemWide) && tile_rect(d.r0, d.r1, d.c0, d.c1, jobs[d.job].tile_w, tx0, tx1, ty0, ty1)) {
-        const JobDev& J = jobs[d.job];
-        const uint32_t tl = (t - J.tile_base) % J.tiles_per_layer;
-        const int32_t ty = (int32_t)(tl / (uint32_t)J.ntx), tx = (int32_t)(tl % (uint32_t)J.ntx);
-        wide_j[pair_off[pair_item[i]] + (uint64_t)((ty - ty0) * (tx1 - tx0 + 1) + (tx - tx0))] =
-            (uint32_t)(i - tile_off[t]);
-      }
-    }
+// An item (or a window of one) whose toggle words are in LDS.
+struct __align__(16) CoverItem {
+  int32_t A, stride;  // the words of raster row r start at A + r * stride
+  int32_t W0, wid;    // first column and columns
+  int32_t R0, R1;     // raster rows [R0, R1)
+  int64_t lv;         // edge e of the unit starts at local vertex lv + e
+  uint32_t mask;      // ItemDesc::mask
+  uint32_t row0;      // rows of the unit's items before this one
+  uint32_t base, pad; // word of its first row
+  // The windows of a whole item, its rows and LDS words.
+  __device__ void set_box(int32_t r0, int32_t r1, int32_t c0, int32_t c1, uint32_t& rows, uint32_t& words) {
+    const int32_t ww = mask_row_words(c0, c1);
+    rows = (uint32_t)mask_strip_count(r0, r1) * 16u;
+    stride = ww | 1;
+    words = rows * (uint32_t)stride;
+    W0 = (c0 >> 6) * 64;
+    wid = ww * 64;
+    R0 = (r0 >> 4) * 16;
+    R1 = R0 + (int32_t)rows;
   }
-  // one atomic per block (the list's order does not matter)
-  __shared__ uint32_t s_n[kHeavyPairsBlock / 64], s_base;
-  const int wave = threadIdx.x >> 6;
-  const uint64_t m = __ballot(poly);
-  if (lane == 0) s_n[wave] = (uint32_t)__popcll(m);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t n = 0;
-    for (int w = 0; w < kHeavyPairsBlock / 64; ++w) n += s_n[w];
-    s_base = n ? atomicAdd(cover_count, n) : 0u;
-  }
-  __syncthreads();
-  uint32_t base = s_base;
-  for (int w = 0; w < wave; ++w) base += s_n[w];
-  if (poly) cover_list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)i;
-}
+};
 
-template <int NWORD>
-__global__ __launch_bounds__(256) void k_cover(CoverArgs a) {
-  constexpr int TW = 64 * NWORD;
-  __shared__ PolyEdge s_edge[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rl = lane >> 2, q = lane & 3;
-  const RZ_CONST JobDev* jobs_c = as_const(a.jobs);
-  const RZ_CONST uint64_t* band_c = as_const(a.band_off);
-  const uint64_t units = 4ull * *a.cover_count;
-  const uint64_t ustride = (uint64_t)gridDim.x * 4u;
-  uint64_t u = (uint64_t)blockIdx.x * 4u + (uint64_t)wave;
-  // the next unit's pair is loaded one unit ahead
-  uint32_t i_next = u < units ? a.cover_list[u >> 2] : 0u;
-  for (; u < units; u += ustride) {
-    const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)i_next);  // wave-uniform
-    if (u + ustride < units) i_next = a.cover_list[(u + ustride) >> 2];
-    const int32_t strip = (int32_t)(u & 3u);
-    const uint32_t t = a.pair_tile[i];
-    const ItemDesc d = load_desc(as_const(a.pair_desc) + i);
-    const RZ_CONST JobDev& J = jobs_c[d.job];
-    if (J.tile_w != TW) continue;
-    const uint32_t tj = t - J.tile_base;
-    const uint32_t layer = tj / J.tiles_per_layer;
-    const uint32_t tl = tj - layer * J.tiles_per_layer;
-    const int32_t ty = (int32_t)(tl / (uint32_t)J.ntx), tx = (int32_t)(tl % (uint32_t)J.ntx);
-    const int32_t C0 = tx * TW, Rw = ty * TILE_H + strip * WAVE_ROWS;
-    const int32_t strip_r1 = min(Rw + WAVE_ROWS, J.nrows), tile_c1 = min(C0 + TW, J.ncols);
-    if (d.r1 <= Rw || d.r0 >= strip_r1 || d.c1 <= C0 || d.c0 >= tile_c1) continue;
-    const PolyEdge* ebase = a.edges + d.vbeg;
-    uint32_t n_e = (uint32_t)d.nv;
-    if (d.band) {
-      const uint32_t bi = d.band - 1u + (uint32_t)(Rw / kBandRows - d.r0 / kBandRows);
-      const uint64_t b0 = band_c[bi];
-      ebase = a.band_edges + b0;
-      n_e = (uint32_t)(band_c[bi + 1u] - b0);
-    }
-    const uint64_t cov = strip_coverage<NWORD>(ebase, n_e, Rw, strip_r1, C0, (double)J.ncols, s_edge[wave], lane);
-    // strip-major slots: item j of heavy tile t, strip s at heavy_base[t] * 4 + s * cnt + j
-    const uint32_t p0 = a.tile_off[t], cnt = a.tile_off[t + 1] - p0;
-    const uint64_t slot = a.heavy_base[t] * 4u + (uint64_t)strip * cnt + (i - p0);
-    if (q < NWORD) a.masks[slot * a.slot_words + (uint64_t)(rl * NWORD + q)] = cov;
-  }
-}
+// A wave's share of the LDS of k_cover and k_items.
+struct CoverWave {
+  uint64_t* tog;       // toggle words
+  double (*edges)[4];  // [64] x0, y0, dxdy, (row offset, item)
+  CoverItem* items;
+  uint64_t* start;     // scratch of owner()
+  uint32_t base;       // the wave's first toggle word
+  int lane;
 
-// The wide pre-pass: one wave per unit = (kItemWide item, 16-row strip,
-// window of at most kWideWords mask words), grid-stride over the unit list.
-// The strip's edges (its band, or the whole edge list) are visited once for
-// the window, in the cheaper of the two layouts per chunk of 64 edges
-// (row-major: four lanes per row over the staged active edges; edge-major:
-// one lane per edge over the rows it crosses), and every crossing updates
-// the row's LDS state with an atomic (XOR of its toggle bit or of the left
-// parity, max of the column; order-free).  Then two rows at a time, lane
-// (half, w) turns word w of the toggles of its row into coverage (prefix
-// parity across the words from one ballot, right limit from the rightmost
-// crossing) and stores it.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_wide_cover(WideCoverArgs a) {
-  __shared__ PolyEdge s_edge[4][64];
-  // rows padded by one word, so the same word of different rows falls in
-  // different LDS banks
-  __shared__ uint64_t s_tog[4][WAVE_ROWS][kWideWords + 1];
-  __shared__ uint32_t s_lp[4][WAVE_ROWS];
-  __shared__ int32_t s_amax[4][WAVE_ROWS];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rl = lane >> 2, q = lane & 3;
-  const RZ_CONST JobDev* jobs_c = as_const(a.jobs);
-  const RZ_CONST uint64_t* band_c = as_const(a.band_off);
-  const uint64_t units = min(*a.n_units, a.unit_cap);
-  PolyEdge* stage = s_edge[wave];
-  uint64_t(*tog)[kWideWords + 1] = s_tog[wave];
-  uint32_t* lp = s_lp[wave];
-  int32_t* amax = s_amax[wave];
-  if (a.n_items <= 0) return;
-  // the toggle rows start at zero, and each unit's finalize step clears the
-  // words it read (no crossing touches a word past the unit's window)
-  for (int idx = lane; idx < WAVE_ROWS * (kWideWords + 1); idx += 64) (&tog[0][0])[idx] = 0ull;
-  const uint64_t ustride = (uint64_t)gridDim.x * 4u;
-  uint64_t u = (uint64_t)blockIdx.x * 4u + (uint64_t)wave;
-  // the next unit's item is loaded one unit ahead, and a unit's range and
-  // descriptor are loaded together (clamped to a valid item) and checked
-  // afterwards, so a unit starts after one round trip instead of three
-  uint32_t it_next = u < units ? a.unit_item[u] : 0u;
-  for (; u < units; u += ustride) {
-    // (wave-uniform: the unit's header and descriptor go to scalar registers)
-    const uint32_t it = (uint32_t)__builtin_amdgcn_readfirstlane((int)it_next);
-    if (u + ustride < units) it_next = a.unit_item[u + ustride];
-    const uint32_t itc = (int64_t)it < a.n_items ? it : (uint32_t)(a.n_items - 1);
-    const uint64_t ub = a.unit_base[itc], ue = a.unit_base[itc + 1];
-    const ItemDesc d = load_desc(as_const(a.desc) + itc);
-    // a unit of an item past the capacities, or a stale one
-    if ((int64_t)it >= a.n_items || u < ub || u >= ue || !(d.flags & kItemWide)) continue;
-    const RZ_CONST JobDev& J = jobs_c[d.job];
-    const int32_t nw = wide_row_words(d.c0, d.c1);
-    const int32_t nwin = (nw + kWideWords - 1) / kWideWords;
-    const int32_t local = (int32_t)(u - ub);
-    const int32_t k = local / nwin, w0 = (local - k * nwin) * kWideWords;
-    const int32_t ww = min(kWideWords, nw - w0);
-    const int32_t Rw = ((d.r0 >> 4) + k) * WAVE_ROWS, strip_r1 = min(Rw + WAVE_ROWS, J.nrows);
-    const int32_t W0 = ((d.c0 >> 6) + w0) * 64, WEND = W0 + ww * 64;
+  // Owners (lanes with `own`) hold consecutive runs of positions, the lane's
+  // from `first`.  Position c + lane belongs to owner number `before` plus
+  // the value returned; `before` moves past the owners that start here.
+  __device__ __attribute__((always_inline)) uint32_t owner(bool own, uint32_t first, uint32_t c, uint32_t& before) const {
+    if (lane == 0) *start = 0ull;
+    wave_sync();
+    if (own && first >= c && first - c < 64u)
+      __hip_atomic_fetch_or(start, 1ull << (first - c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    wave_sync();
+    const uint64_t v = *start;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    const uint64_t st = ((uint64_t)hi << 32) | lo, s1 = st >> 1;
+    const uint32_t at = before + (lo & 1u) - 1u +
+                        __builtin_amdgcn_mbcnt_hi((uint32_t)(s1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)s1, 0u));
+    before += (uint32_t)__popcll(st);
+    wave_sync();
+    return at;
+  }
+
+  // The toggles of edges [0, n_e) of the items in `items`, taken in
+  // chunks of 64 (first, first + step, ...).  `many`: the lane's item (own)
+  // has the edges from e0 of the one chunk; else all are item 0's.
+  __device__ __attribute__((always_inline)) void toggles(const RZ_CONST JobDev& J, bool many, bool own, uint32_t e0,
+                                                         uint32_t n_e, uint32_t first, uint32_t step, bool odd) const {
     const double ncols_f = (double)J.ncols;
-    const PolyEdge* ebase = a.edges + d.vbeg;
-    uint32_t n_e = (uint32_t)d.nv;
-    if (d.band) {
-      const uint32_t bi = d.band - 1u + (uint32_t)k;
-      const uint64_t b0 = band_c[bi];
-      ebase = a.band_edges + b0;
-      n_e = (uint32_t)(band_c[bi + 1u] - b0);
-    }
-    // the rightmost crossing of a row matters only with an odd count
-    const bool odd_rows = (d.flags & kItemOddRows) != 0;
-    if (lane < WAVE_ROWS) {
-      lp[lane] = 0u;
-      amax[lane] = -1;
-    }
-    wave_sync();
-    // one crossing of row `row` (0..15) at x
-    auto put = [&](int32_t row, double x) {
-      const int32_t col = span_col(x, ncols_f);
-      const int32_t rel = col - W0;
-      if (rel <= 0) {
-        __hip_atomic_fetch_xor(&lp[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        return;
-      }
-      if (odd_rows) __hip_atomic_fetch_max(&amax[row], col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-      if (col < WEND)
-        __hip_atomic_fetch_xor(&tog[row][rel >> 6], 1ull << (rel & 63), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
-    };
-    for (uint32_t cb = 0; cb < n_e; cb += 64) {
+    const bool sx = J.xres != 1.0, sy = J.yres != 1.0;  // (v / 1.0 is v)
+    auto px_x = [&](double X) { return isnan(X) ? X : (sx ? (X - J.xmin) / J.xres : X - J.xmin); };
+    auto px_y = [&](double Y) { return isnan(Y) ? Y : (sy ? (J.ymax - Y) / J.yres : J.ymax - Y); };
+    for (uint32_t cb = first * 64u; cb < n_e; cb += step * 64u) {
       const uint32_t e = cb + (uint32_t)lane;
-      uint4 e_lo = make_uint4(0u, 0u, 0u, 0u), e_hi = make_uint4(0u, 0u, 0u, 0u);
-      int32_t a0 = 0, span = 0;  // rows [a0, a0 + span) of the strip the edge crosses
+      uint32_t before = 0;
+      const uint32_t k = many ? owner(own, e0, 0u, before) : 0u;
+      PolyEdge ee{0.0, 0.0, 0.0, 0, 0};
+      int32_t a0 = 0;
+      uint32_t span = 0;
       if (e < n_e) {
-        const uint4* src = reinterpret_cast<const uint4*>(ebase + e);
-        e_lo = src[0];
-        e_hi = src[1];  // dxdy, ystart (z), yend (w)
-        a0 = max((int32_t)e_hi.z, Rw);
-        span = max(0, min((int32_t)e_hi.w, strip_r1) - a0);
-      }
-      const uint64_t m = __ballot(span > 0);
-      const int n = __popcll(m);
-      const int32_t steps = wave_max16(span);
-      if (a.cov_mode == 2 || (a.cov_mode == 0 && steps <= (n + 3) / 4)) {  // edge-major
-        PolyEdge ee;
-        __builtin_memcpy(&ee, &e_lo, 16);
-        __builtin_memcpy(reinterpret_cast<char*>(&ee) + 16, &e_hi, 16);
-        for (int32_t j = 0; j < steps; ++j) {
-          const int32_t rr = a0 + j;
-          const double x = crossing(ee, rr);
-          if (j < span) put(rr - Rw, x);
+        const CoverItem* it = &items[k];
+        const int64_t v = it->lv + (int64_t)e;
+        const int64_t vn = min(v + 1, J.nv - 1);
+        const uint64_t vi = J.vert_info[v];
+        const double2 p = *reinterpret_cast<const double2*>(J.xy + 2 * v);
+        const double2 q = *reinterpret_cast<const double2*>(J.xy + 2 * vn);
+        double xb, yb;
+        bool o = false;
+        if ((vi & VI_HAS_NEXT) && ring_edge(px_x(p.x), px_y(p.y), px_x(q.x), px_y(q.y), J.nrows, false, ee, xb, yb, o)) {
+          a0 = max(ee.ystart, it->R0);
+          span = (uint32_t)max(0, min(ee.yend, it->R1) - a0);
+          // (an edge of an infinite or NaN end has its slope already: its
+          // crossings are pinned or come from that slope)
+          const double inf = __builtin_inf();
+          if (span && fabs(ee.x0) < inf && fabs(xb) < inf && fabs(ee.y0) < inf && fabs(yb) < inf)
+            ee.dxdy = edge_slope(ee.x0, ee.y0, xb, yb);
         }
-        continue;
       }
-      // row-major over the staged active edges
-      if (span > 0) {
-        uint4* dst = reinterpret_cast<uint4*>(stage + __popcll(m & ((1ull << lane) - 1ull)));
-        dst[0] = e_lo;
-        dst[1] = e_hi;
+      const uint64_t act = __ballot(span != 0u);
+      if (!act) continue;
+      const uint32_t incl = wave_prefix_sum(span);
+      const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      const uint32_t excl = incl - span;
+      if (span) {  // compacted: the crossing loop finds edges by their rank
+        double* dst = edges[__popcll(act & ((1ull << lane) - 1ull))];
+        dst[0] = ee.x0;
+        dst[1] = ee.y0;
+        dst[2] = ee.dxdy;
+        const uint64_t rk = (uint64_t)(uint32_t)(a0 - (int32_t)excl) | ((uint64_t)k << 32);
+        __builtin_memcpy(dst + 3, &rk, 8);
+      }
+      before = 0;
+      for (uint32_t c = 0; c < total; c += 64u) {
+        const uint32_t at = owner(span != 0u, excl, c, before);
+        if (c + (uint32_t)lane < total) {
+          const double* src = edges[at];
+          uint64_t rk;
+          __builtin_memcpy(&rk, src + 3, 8);
+          const int32_t r = (int32_t)(c + (uint32_t)lane) + (int32_t)(uint32_t)rk;
+          const CoverItem* it = &items[many ? (int)(rk >> 32) : 0];
+          const int32_t W0 = it->W0, wid = it->wid;
+          const double x = src[0] + (((double)r + 0.5) - src[1]) * src[2];
+          const int32_t col = span_col(x, ncols_f);
+          const int32_t rel = max(col - W0, 0);
+          uint64_t* row = tog + (it->A + r * it->stride);
+          if (rel < wid)
+            __hip_atomic_fetch_xor(row + (rel >> 6), 1ull << (rel & 63), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+          // the rightmost crossing of a row matters only with an odd count
+          if (odd)
+            __hip_atomic_fetch_max(reinterpret_cast<uint32_t*>(row + (wid >> 6)), (uint32_t)col + 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
       }
       wave_sync();
-      const int32_t r = Rw + rl;
-      for (int k0 = 0; k0 < n; k0 += 4) {
-        const int kk = k0 + q;
-        const PolyEdge ee = stage[kk < n ? kk : n - 1];
-        const double x = crossing(ee, r);
-        if (kk < n && r < strip_r1 && ee.ystart <= r && r < ee.yend) put(rl, x);
+    }
+  }
+
+  // One row's toggles (ww words from `row`, cleared as they are read), the
+  // rows of a strip in 16 neighbouring lanes, into mask blocks out, out + 16,
+  // ... (out: the lane's word of a block); odd: the row's rightmost crossing
+  // + 1 lies after its words, W0 is its first column.
+  __device__ __attribute__((always_inline)) void finish_row(uint64_t* row, int32_t ww, uint64_t* out, bool odd, int32_t W0) const {
+    int64_t lim = INT_MAX;  // columns of the window left of the rightmost crossing
+    if (odd) {
+      lim = (int64_t)(uint32_t)row[ww] - 1 - (int64_t)W0;
+      row[ww] = 0ull;
+    }
+    uint64_t carry = 0ull;
+    for (int32_t w = 0; w < ww; ++w) {
+      uint64_t x = prefix_xor64(row[w]) ^ carry;
+      row[w] = 0ull;
+      carry = 0ull - (x >> 63);
+      if (odd) {
+        const int64_t l = lim - 64 * (int64_t)w;
+        x &= l <= 0 ? 0ull : (l >= 64 ? ~0ull : ((1ull << l) - 1ull));
+      }
+      out[(uint64_t)w * 16u] = transpose16(x, lane);
+    }
+  }
+
+  // The masks of small items, one per lane with `ok` (at most 64 edges and
+  // kCoverWave LDS words each; it: all but A, base and row0): as many of them
+  // as fit together form a unit.
+  __device__ __attribute__((always_inline)) void small_items(const RZ_CONST JobDev* jobs_c, uint64_t* masks,
+                                                             const CoverItem& it, bool ok, uint32_t job, uint32_t nv,
+                                                             uint32_t words, uint32_t rows) const {
+    uint64_t todo = __ballot(ok);
+    while (todo) {
+      // the unit: the next items of one job that fit together
+      const uint32_t j = (uint32_t)__builtin_amdgcn_readlane((int)job, __builtin_ctzll(todo));
+      const bool mine = (todo >> lane) & 1ull;
+      const uint32_t ei = wave_prefix_sum(mine ? nv : 0u), wi = wave_prefix_sum(mine ? words : 0u);
+      const uint64_t no = __ballot(mine && (job != j || ei > 64u || wi > (uint32_t)kCoverWave));
+      const uint64_t unit = todo & (no ? ((1ull << __builtin_ctzll(no)) - 1ull) : ~0ull);
+      todo &= ~unit;
+      const bool own = (unit >> lane) & 1ull;
+      const int last = 63 - __builtin_clzll(unit);
+      const uint32_t n_e = (uint32_t)__builtin_amdgcn_readlane((int)ei, last);
+      const uint32_t ri = wave_prefix_sum(own ? rows : 0u);
+      const uint32_t n_rows = (uint32_t)__builtin_amdgcn_readlane((int)ri, 63);
+      const RZ_CONST JobDev& J = jobs_c[j];
+      if (own) {
+        CoverItem x = it;
+        x.base = base + wi - words;
+        x.A = (int32_t)x.base - x.R0 * x.stride;
+        x.R1 = min(x.R1, J.nrows);
+        x.lv -= J.v_base + (int64_t)(ei - nv);
+        x.row0 = ri - rows;
+        items[__popcll(unit & ((1ull << lane) - 1ull))] = x;
       }
       wave_sync();
+      toggles(J, true, own, ei - nv, n_e, 0u, 1u, false);
+      uint32_t before = 0;
+      for (uint32_t c = 0; c < n_rows; c += 64u) {
+        const uint32_t at = owner(own, ri - rows, c, before);
+        if (c + (uint32_t)lane < n_rows) {
+          const CoverItem x = items[at];
+          const uint32_t r = c + (uint32_t)lane - x.row0;
+          finish_row(tog + x.base + r * (uint32_t)x.stride, x.wid >> 6,
+                     masks + ((uint64_t)x.mask + (uint64_t)(r >> 4) * (uint64_t)(x.wid >> 6)) * 16u + (uint64_t)(r & 15u),
+                     false, 0);
+        }
+      }
+      wave_sync();
+    }
+  }
+
+  // Window t of an item, by the wave or (BLOCK) the four of a workgroup.
+  template <bool BLOCK>
+  __device__ __attribute__((always_inline)) void window(const RZ_CONST JobDev& J, uint64_t* masks, int32_t r0, int32_t r1,
+                                                        int32_t c0, int32_t c1, int64_t vbeg, uint32_t nv, bool odd,
+                                                        uint32_t mask, int32_t t) const {
+    const int32_t ns = mask_strip_count(r0, r1), nw = mask_row_words(c0, c1);
+    const CoverWindows win = cover_windows(ns, nw, odd, BLOCK ? kCoverBlock : kCoverWave);
+    const int32_t row = win.n == 1 ? 0 : t / win.ncw;
+    const int32_t s0 = row * win.strips, w0 = (t - row * win.ncw) * win.ww;
+    const int32_t ww = min(win.ww, nw - w0), n_rows = min(win.strips, ns - s0) * 16;
+    const int32_t first = BLOCK ? 0 : (int32_t)base, R0 = ((r0 >> 4) + s0) * 16, W0 = ((c0 >> 6) + w0) * 64;
+    if (lane == 0) {
+      CoverItem it{};
+      it.A = first - R0 * win.stride;
+      it.stride = win.stride;
+      it.W0 = W0;
+      it.wid = ww * 64;
+      it.R0 = R0;
+      it.R1 = min(R0 + n_rows, J.nrows);
+      it.lv = vbeg - J.v_base;
+      items[0] = it;
     }
     wave_sync();
-    // two rows per step: lanes 0..31 row 2i, lanes 32..63 row 2i + 1
-    static_assert(kWideWords == 32, "two rows of window words per wave step");
-    uint64_t* out = a.wide_masks + (uint64_t)d.wide * 16u + (uint64_t)k * 16u * (uint64_t)nw + (uint64_t)w0;
-    const int half = lane >> 5, w = lane & 31;
-    // A heavy tile's fold reads its items' masks from its pre-pass slots, so
-    // each word also goes to the slot of the tile that holds it when that
-    // tile is heavy: tile column gw / (TW / 64), the item's place j in the
-    // tile's (item-ordered) pair list found by binary search.
-    uint64_t* slot = nullptr;
-    if (a.heavy_cnt && !J.scan && w < ww) {
-      const int32_t nwt = J.tile_w >> 6;  // words per tile row
-      const int32_t gw = (W0 >> 6) + w, tx = gw / nwt;
-      const uint32_t t = J.tile_base + (d.kind_layer >> 2) * J.tiles_per_layer +
-                         (uint32_t)(Rw / TILE_H) * (uint32_t)J.ntx + (uint32_t)tx;
-      const uint32_t cnt = a.heavy_cnt[t];
-      // the pair (it, t) in k_bin_emit's order over the item's tile
-      // rectangle: row Rw / TILE_H - ty0, column tx - tx0 (uniform part first)
-      int32_t tx0, tx1, ty0, ty1;
-      uint32_t j = ~0u;
-      if (cnt && a.pair_off[it + 1] <= a.pair_cap &&
-          tile_rect(d.r0, d.r1, d.c0, d.c1, J.tile_w, tx0, tx1, ty0, ty1)) {
-        const int64_t jrow = (int64_t)a.pair_off[it] + (int64_t)(Rw / TILE_H - ty0) * (tx1 - tx0 + 1) - tx0;
-        j = a.wide_j[jrow + tx];
-      }
-      if (j < cnt) {
-        const uint32_t s = (uint32_t)((Rw % TILE_H) / WAVE_ROWS);
-        slot = a.masks + (a.heavy_base[t] * 4u + (uint64_t)s * cnt + j) * a.slot_words + (uint32_t)(gw % nwt);
-      }
-    }
-    const uint64_t below = ((1ull << lane) - 1ull) & (half ? 0xFFFFFFFF00000000ull : 0xFFFFFFFFull);
-    for (int r2 = 0; r2 < WAVE_ROWS; r2 += 2) {
-      const int row = r2 + half;
-      uint64_t t = 0ull;
-      if (w < ww) {
-        t = tog[row][w];
-        tog[row][w] = 0ull;
-      }
-      const uint64_t odd = __ballot(__popcll(t) & 1);
-      const uint32_t carry = lp[row] ^ ((uint32_t)__popcll(odd & below) & 1u);
-      uint64_t x = prefix_xor64(t) ^ (carry ? ~0ull : 0ull);
-      const int32_t lim = odd_rows ? amax[row] - (W0 + 64 * w) : 64;
-      x &= lim <= 0 ? 0ull : (lim >= 64 ? ~0ull : ((1ull << lim) - 1ull));
-      if (w < ww) out[(uint64_t)row * (uint64_t)nw + (uint64_t)w] = x;
-      if (slot) {
-        // the tile's words left of the item's first word or right of its
-        // last one are empty: written as such (the fold reads every word)
-        const int32_t nwt = J.tile_w >> 6, gw = (W0 >> 6) + w, qq = gw % nwt;
-        uint64_t* srow_p = slot + row * nwt - qq;
-        srow_p[qq] = x;
-        if (gw == (d.c0 >> 6))
-          for (int z = 0; z < qq; ++z) srow_p[z] = 0ull;
-        if (gw == ((d.c1 - 1) >> 6))
-          for (int z = qq + 1; z < nwt; ++z) srow_p[z] = 0ull;
-      }
-    }
-    wave_sync();  // the rows are read and cleared before the next unit's crossings
+    toggles(J, false, false, 0u, nv, BLOCK ? threadIdx.x >> 6 : 0u, BLOCK ? 4u : 1u, odd);
+    if (BLOCK) __syncthreads();
+    else wave_sync();
+    for (int32_t r = BLOCK ? (int32_t)threadIdx.x : lane; r < n_rows; r += BLOCK ? 256 : 64)
+      finish_row(tog + first + r * win.stride, ww,
+                 masks + ((uint64_t)mask + (uint64_t)(s0 + (r >> 4)) * (uint64_t)nw + (uint64_t)w0) * 16u +
+                     (uint64_t)(r & 15),
+                 odd, W0);
+    if (BLOCK) __syncthreads();
+    else wave_sync();
   }
+};
+
+// The coverage masks of the polygon items, each edge's crossings computed
+// once (the tile kernels only read masks).
+//
+// Per unit (see CoverLists): lanes build the unit's edges from the world
+// coordinates, 64 at a time; the (edge, row) crossings of those edges are
+// then laid out one per lane (an edge of a few rows and one of hundreds cost
+// what they cross, where a lane per edge would wait for the longest one);
+// every crossing flips its toggle bit in LDS (order-free), at bit 0 when it
+// lies left of the window; and a lane per row turns the toggles into
+// coverage (inclusive prefix parity across its words, see the note above
+// row_coverage_word), the 16 lanes of a strip transpose it to the order of
+// the mask blocks and store it.  Small items are packed: as many as
+// have at most 64 edges and a wave's LDS words together form one unit.
+// Bound by the latency of its dependent loads and LDS round trips (vector
+// issue is busy about a third of the time), so LDS is sized for 6 waves per
+// SIMD.
+// BLOCK: the block list, a workgroup per unit; else the wave and small lists.
+template <bool BLOCK>
+__global__ __launch_bounds__(256) void k_cover(CoverArgs a) {
+  constexpr int RUN = BLOCK ? 1 : kCoverRun;
+  __shared__ uint64_t s_tog[BLOCK ? kCoverBlock : 4 * kCoverWave];
+  __shared__ __align__(16) double s_edge[4][64][4];  // x0, y0, dxdy, (row offset, item)
+  __shared__ CoverItem s_item[4][RUN];
+  __shared__ uint64_t s_start[4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const RZ_CONST JobDev* jobs_c = as_const(a.jobs);
+  const RZ_CONST ItemDesc* desc_c = as_const(a.desc);
+  const CoverWave cw{s_tog, s_edge[wave], s_item[wave], &s_start[wave], (uint32_t)(wave * kCoverWave), lane};
+  if (!BLOCK && !a.cover.ctr->n_wave && !a.cover.ctr->n_small) return;
+  for (int k = threadIdx.x; k < (BLOCK ? kCoverBlock : 4 * kCoverWave); k += 256) s_tog[k] = 0ull;
+  __syncthreads();
+
+  auto window = [&](const uint2 en) __attribute__((always_inline)) {
+    const ItemDesc d = load_desc(desc_c + (uint32_t)__builtin_amdgcn_readfirstlane((int)en.x));
+    const int32_t t = __builtin_amdgcn_readfirstlane((int)en.y);
+    if (d.flags & kItemMask)  // (not past a capacity)
+      cw.window<BLOCK>(jobs_c[d.job], a.masks, d.r0, d.r1, d.c0, d.c1, d.vbeg, (uint32_t)d.nv,
+                       (d.flags & kItemOddRows) != 0, d.mask, t);
+  };
+
+  if constexpr (BLOCK) {
+    const uint32_t n_block = min(a.cover.ctr->n_block, a.cover.unit_cap);
+    for (uint32_t u = blockIdx.x; u < n_block; u += gridDim.x) window(a.cover.block[u]);
+  } else {
+    const uint32_t wid = blockIdx.x * 4u + (uint32_t)wave, n_wid = gridDim.x * 4u;
+    const uint32_t n_wave = min(a.cover.ctr->n_wave, a.cover.unit_cap);
+    for (uint32_t u = wid; u < n_wave; u += n_wid) window(a.cover.wave[u]);
+    // Small items: runs of the list, one item per lane, fewer per run where
+    // there are not enough to go round.
+    const uint32_t n_small = a.cover.ctr->n_small;
+    const uint32_t run = min((uint32_t)RUN, (n_small + n_wid - 1u) / n_wid);
+    for (uint32_t b = wid * run; b < n_small; b += n_wid * run) {
+      const uint32_t n = min(run, n_small - b);
+      CoverItem it{};
+      uint32_t nv = 0, words = 0, rows = 0, job = 0;
+      bool ok = false;
+      if ((uint32_t)lane < n) {
+        const u32x4* q = reinterpret_cast<const u32x4*>(a.desc + a.cover.small[b + (uint32_t)lane]);
+        const u32x4 box = q[0], vq = q[1], fq = q[3];
+        ok = (fq[2] & kItemMask) != 0;
+        job = fq[0];
+        nv = vq[2];
+        it.set_box((int32_t)box[0], (int32_t)box[1], (int32_t)box[2], (int32_t)box[3], rows, words);
+        it.lv = (int64_t)((uint64_t)vq[0] | ((uint64_t)vq[1] << 32));
+        it.mask = fq[3];
+      }
+      cw.small_items(jobs_c, a.masks, it, ok, job, nv, words, rows);
+    }
+  }
+}
+
+// k_prep, k_item_desc and most of k_cover in one launch, for calls of few
+// items, all polygons, that do not wait for totals: a wave takes an item, a
+// lane per edge for its box (as k_prep, but in LDS), hands out its masks, and
+// covers it right away unless it has many windows.
+// These calls are bound by the latency of dependent loads and by the launches
+// between them, two of which fall away: 1,000 stars on 2048 x 2048 take 35 us
+// in all, with k_prep, k_item_desc and k_cover apart 41.  With more items
+// than waves the packed items of k_cover win (32,000 items: 54 us against 70).
+__global__ __launch_bounds__(64 * kItemsWaves) void k_items(ItemsArgs a) {
+  __shared__ uint64_t s_tog[kItemsWaves * kCoverWave];
+  __shared__ __align__(16) double s_edge[kItemsWaves][64][4];
+  __shared__ CoverItem s_item[kItemsWaves][1];
+  __shared__ uint64_t s_start[kItemsWaves];
+  __shared__ ItemBox s_box[kItemsWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint32_t base = (uint32_t)(wave * kCoverWave);
+  const CoverWave cw{s_tog, s_edge[wave], s_item[wave], &s_start[wave], base, lane};
+  const int64_t i = (int64_t)blockIdx.x * kItemsWaves + wave;
+  const bool item = i < a.d.n_items;  // (uniform)
+  const int j = a.d.n_jobs == 1 || !item ? 0 : __builtin_amdgcn_readfirstlane(find_job(a.d.job_iend, a.d.n_jobs, i));
+  const RZ_CONST JobDev& J = as_const(a.d.jobs)[j];
+  ItemDesc d;
+  __builtin_memset(&d, 0, sizeof(d));
+  if (item) {
+    if (lane == 0) s_box[wave] = ItemBox{INT_MAX, INT_MIN, INT_MAX, INT_MIN};
+    for (int k = lane; k < kCoverWave; k += 64) s_tog[base + (uint32_t)k] = 0ull;
+    wave_sync();
+    const int64_t v0 = J.item_vbeg[i - J.i_base], v1 = J.item_vbeg[i - J.i_base + 1];
+    bool odd = false;
+    for (int64_t lv = v0 + lane; lv - lane < v1; lv += 64) {
+      const bool active = lv < v1;
+      ItemBox box{INT_MAX, INT_MIN, INT_MAX, INT_MIN};
+      if (active) {
+        const int64_t ln = min(lv + 1, J.nv - 1);
+        const uint64_t vi = J.vert_info[lv];
+        const double X0 = J.xy[2 * lv], Y0 = J.xy[2 * lv + 1], X1 = J.xy[2 * ln], Y1 = J.xy[2 * ln + 1];
+        auto px_x = [&](double X) { return isnan(X) ? X : (X - J.xmin) / J.xres; };
+        auto px_y = [&](double Y) { return isnan(Y) ? Y : (J.ymax - Y) / J.yres; };
+        PolyEdge e;
+        polygon_edge(vi, px_x(X0), px_y(Y0), px_x(X1), px_y(Y1), J, a.edges != nullptr, e, box, odd);
+        if (a.edges) a.edges[J.v_base + lv] = e;
+      }
+      reduce_box(lv, 0, box, 0, &s_box[wave], nullptr, active);
+    }
+    odd = __any(odd);
+    wave_sync();
+    d = make_desc(a.d, i, s_box[wave], odd ? kItemOddBit : 0ull);
+  }
+  // (lane 0 stands for the item)
+  const bool poly = item && lane == 0 && d.nv > 0 && d.r0 < d.r1 && d.c0 < d.c1;
+  bool small, own;
+  const bool ok = assign_cover<kItemsWaves, false>(a.d.cover, poly, d, i, d.mask, small, own);
+  if (!item) return;
+  if (ok) d.flags |= kItemMask;
+  if (lane == 0) a.d.desc[i] = d;
+  if (!__any(ok && (small || own))) return;
+  const bool odd = (d.flags & kItemOddRows) != 0;
+  const int32_t n_win = (int32_t)cover_windows(mask_strip_count(d.r0, d.r1), mask_row_words(d.c0, d.c1), odd, kCoverWave).n;
+  const uint32_t mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.mask);
+  for (int32_t t = 0; t < n_win; ++t)
+    cw.window<false>(J, a.masks, d.r0, d.r1, d.c0, d.c1, d.vbeg, (uint32_t)d.nv, odd, mask, t);
 }
 
 }  // namespace rzk

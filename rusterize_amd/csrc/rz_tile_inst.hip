@@ -1,4 +1,4 @@
-// rz_tile_inst.hip -- the k_tile / k_tile_heavy instantiations of one output
+// rz_tile_inst.hip -- the k_tile / k_tile_lp instantiations of one output
 // dtype and their launchers.  Compiled once per dtype with
 // -DRZ_TILE_T=<C type> -DRZ_TILE_NAME=<u8|u16|...|f64> (rusterize_amd/build.py).
 #include <algorithm>
@@ -45,6 +45,15 @@ inline uint32_t queue_chunk(uint64_t n_tiles, uint32_t grid, uint32_t tuned) {
   return n_tiles >= (uint64_t)grid * 16 ? 4u : 1u;
 }
 
+template <int FUN, bool BARE>
+void launch_strips(TileArgs a, hipStream_t s) {
+  const uint64_t tiles = (uint64_t)(a.t_hi - a.t_lo);
+  static uint32_t cached = 0;
+  const uint32_t g = tile_grid(k_tile<T, FUN, BARE>, cached, tiles);
+  a.chunk = queue_chunk(tiles, g, a.chunk);
+  hipLaunchKernelGGL((k_tile<T, FUN, BARE>), dim3(g), dim3(256), 0, s, a);
+}
+
 template <int FUN>
 void launch_tile(TileArgs a, bool lines, hipStream_t s) {
   const uint64_t tiles = (uint64_t)(a.t_hi - a.t_lo);
@@ -53,28 +62,11 @@ void launch_tile(TileArgs a, bool lines, hipStream_t s) {
     const uint32_t g = tile_grid(k_tile_lp<T, FUN>, cached, tiles);
     a.chunk = queue_chunk(tiles, g, a.chunk);
     hipLaunchKernelGGL((k_tile_lp<T, FUN>), dim3(g), dim3(256), 0, s, a);
+  } else if (a.edges) {  // (edge records are there when an item may have no masks)
+    launch_strips<FUN, true>(a, s);
   } else {
-    static uint32_t cached = 0;
-    const uint32_t g = tile_grid(k_tile<T, FUN>, cached, tiles);
-    a.chunk = queue_chunk(tiles, g, a.chunk);
-    hipLaunchKernelGGL((k_tile<T, FUN>), dim3(g), dim3(256), 0, s, a);
+    launch_strips<FUN, false>(a, s);
   }
-}
-
-// k_tile_heavy: a persistent grid (the work counter hands out units)
-template <int FUN>
-void launch_heavy(const TileArgs& a, hipStream_t s) {
-  static uint32_t cached = 0;
-  if (!cached) {
-    int dev = 0, cus = 256, per_cu = 1;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tile_heavy<T, FUN>, 256, 0) != hipSuccess ||
-        per_cu < 1)
-      per_cu = 1;
-    cached = (uint32_t)(cus * per_cu);
-  }
-  hipLaunchKernelGGL((k_tile_heavy<T, FUN>), dim3(cached), dim3(256), 0, s, a);
 }
 
 }  // namespace
@@ -94,16 +86,9 @@ void RZ_CAT(launch_tile_, RZ_TILE_NAME)(int fun, const TileArgs& a, bool lines, 
   }
 }
 
-void RZ_CAT(launch_heavy_, RZ_TILE_NAME)(int fun, const TileArgs& a, hipStream_t s) {
-  switch (fun) {
-    case 0: launch_heavy<0>(a, s); break;
-    case 1: launch_heavy<1>(a, s); break;
-    case 2: launch_heavy<2>(a, s); break;
-    case 3: launch_heavy<3>(a, s); break;
-    case 4: launch_heavy<4>(a, s); break;
-    case 5: launch_heavy<5>(a, s); break;
-    default: launch_heavy<6>(a, s); break;
-  }
+void RZ_CAT(launch_blocks_, RZ_TILE_NAME)(const TileArgs& a, hipStream_t s) {
+  const uint32_t g = (a.t_hi - a.t_lo + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
+  hipLaunchKernelGGL(k_tile_block<T>, dim3(g), dim3(64 * kTileBlockWaves), 0, s, a);
 }
 
 }  // namespace rzk

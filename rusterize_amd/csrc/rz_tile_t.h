@@ -1,7 +1,9 @@
-// rz_tile_t.h -- the tile kernel templates (k_tile, k_tile_heavy): scanline
-// coverage, burn folds and the write-once store of every output tile.
+// rz_tile_t.h -- the tile kernel templates (k_tile, k_tile_lp): burn folds
+// and the write-once store of every output tile.
 // Instantiated per output dtype in rz_tile_inst.hip.
 #pragma once
+
+#include <type_traits>
 
 #include "rz_device.h"
 
@@ -103,9 +105,15 @@ struct StripUnit {
   int32_t nrows, ncols, C0, Rw, strip_r1, tile_c1;
 };
 
-__device__ inline StripUnit strip_unit(const TileArgs& a, uint32_t t, int32_t strip, int tw) {
+// (row0: the unit's first row in its tile; rows: its rows; job: the last
+// unit's job, tried first, as a wave's tiles mostly follow each other)
+__device__ inline StripUnit strip_unit(const TileArgs& a, uint32_t t, int32_t row0, int32_t rows, int tw, int& job) {
   StripUnit u;
-  u.J = &as_const(a.jobs)[find_job(as_const(a.job_tend), a.n_jobs, (int64_t)t)];
+  u.J = &as_const(a.jobs)[job];
+  if (t - u.J->tile_base >= u.J->n_tiles) {
+    job = find_job(as_const(a.job_tend), a.n_jobs, (int64_t)t);
+    u.J = &as_const(a.jobs)[job];
+  }
   u.nrows = u.J->nrows;
   u.ncols = u.J->ncols;
   const uint32_t tj = t - u.J->tile_base;
@@ -113,59 +121,35 @@ __device__ inline StripUnit strip_unit(const TileArgs& a, uint32_t t, int32_t st
   const uint32_t tl = tj - u.layer * u.J->tiles_per_layer;
   const int32_t ty = (int32_t)(tl / (uint32_t)u.J->ntx), tx = (int32_t)(tl % (uint32_t)u.J->ntx);
   u.C0 = tx * tw;
-  u.Rw = ty * TILE_H + strip * WAVE_ROWS;  // first row of the strip
-  u.strip_r1 = min(u.Rw + WAVE_ROWS, u.nrows);
+  u.Rw = ty * TILE_H + row0;  // first row of the strip
+  u.strip_r1 = min(u.Rw + rows, u.nrows);
   u.tile_c1 = min(u.C0 + tw, u.ncols);
   return u;
 }
 
-// A polygon item's coverage mask word for this lane's row / quarter (lane
-// rl = lane / 4, q = lane % 4): precomputed (wide item, heavy tile) or
-// computed from its edges (banded: only the strip's band).
-template <int NWORD>
-__device__ inline uint64_t polygon_mask(const TileArgs& a, const ItemDesc& d, const StripUnit& u,
-                                        bool hb_ok, uint64_t hbase, uint32_t pb, uint32_t pe, uint32_t pi,
-                                        int32_t strip, PolyEdge* stage, int lane) {
-  const int rl = lane >> 2, q = lane & 3;
-  uint64_t cov = 0;
-  if (d.flags & kItemWide) {  // the wide pre-pass wrote the item's masks
-    const int32_t nw = wide_row_words(d.c0, d.c1), wi = (u.C0 >> 6) + q - (d.c0 >> 6);
-    if (q < NWORD && wi >= 0 && wi < nw)
-      cov = as_const(a.wide_masks)[(uint64_t)d.wide * 16u +
-                                   (uint64_t)(((u.Rw >> 4) - (d.r0 >> 4)) * 16 + rl) * (uint64_t)nw + (uint64_t)wi];
-  } else if (hb_ok) {  // heavy tile: the coverage pre-pass wrote this mask
-    if (q < NWORD)
-      cov = as_const(a.masks)[(hbase * 4u + (uint64_t)strip * (pe - pb) + (pi - pb)) * a.slot_words +
-                              (uint32_t)(rl * NWORD + q)];
-  } else {
-    // the item's edges, or for a banded item only those of this strip
-    const PolyEdge* ebase = a.edges + d.vbeg;
-    uint32_t n_e = (uint32_t)d.nv;
-    if (d.band) {
-      const uint32_t bi = d.band - 1u + (uint32_t)(u.Rw / kBandRows - d.r0 / kBandRows);
-      const uint64_t b0 = as_const(a.band_off)[bi];
-      ebase = a.band_edges + b0;
-      n_e = (uint32_t)(as_const(a.band_off)[bi + 1u] - b0);
-    }
-    if constexpr (NWORD == 1) {
-      cov = strip_coverage<1>(ebase, n_e, u.Rw, u.strip_r1, u.C0, (double)u.ncols, stage, lane);
-    } else {
-      // only the tile words the item's columns [c0, c1) meet can be
-      // covered: the crossings are toggled and the parity scanned over
-      // those (1, 2 or all 4 words; crossings left of them flip the left
-      // parity, as left of a tile)
-      const int32_t wlo = max(0, (d.c0 - u.C0) >> 6), whi = min(NWORD - 1, (d.c1 - 1 - u.C0) >> 6);
-      const int32_t C0e = u.C0 + 64 * wlo;
-      const int wq = (lane & 3) - wlo;  // this lane's word in the narrowed window (negative: none)
-      if (whi == wlo)
-        cov = strip_coverage<1>(ebase, n_e, u.Rw, u.strip_r1, C0e, (double)u.ncols, stage, lane, wq == 0 ? 0 : 1);
-      else if (whi == wlo + 1)
-        cov = strip_coverage<2>(ebase, n_e, u.Rw, u.strip_r1, C0e, (double)u.ncols, stage, lane, wq < 0 ? 2 : wq);
-      else
-        cov = strip_coverage<NWORD>(ebase, n_e, u.Rw, u.strip_r1, u.C0, (double)u.ncols, stage, lane);
-    }
+// The rows an item without masks covers in column C0 + lane of the unit, as
+// bits: its coverage from its edges (strip_coverage's row words), read back
+// row by row from the lanes that hold them.
+__device__ inline uint32_t edge_bits(const TileArgs& a, const ItemDesc& d, const StripUnit& u, int32_t C0,
+                                     PolyEdge* stage, int lane) {
+  const uint64_t cov = strip_coverage<1>(a.edges + d.vbeg, (uint32_t)d.nv, u.Rw, u.strip_r1, C0, (double)u.ncols, stage, lane);
+  uint32_t bits = 0;
+  for (int r = 0; r < WAVE_ROWS; ++r) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cov, 4 * r);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cov >> 32), 4 * r);
+    bits |= ((lane < 32 ? lo : hi) >> (lane & 31) & 1u) << r;
   }
-  return cov;
+  return bits;
+}
+
+// ... of any polygon item in tile word w, for a unit of 16 rows (k_tile_lp).
+__device__ inline uint32_t column_bits(const TileArgs& a, const ItemDesc& d, const StripUnit& u, int w, PolyEdge* stage,
+                                       int lane) {
+  const int32_t wi = (u.C0 >> 6) + w - (d.c0 >> 6), nw = mask_row_words(d.c0, d.c1);
+  if (wi < 0 || wi >= nw) return 0u;
+  if (!(d.flags & kItemMask)) return edge_bits(a, d, u, u.C0 + 64 * w, stage, lane);
+  const uint64_t* p = a.masks + ((uint64_t)d.mask + (uint64_t)((u.Rw >> 4) - (d.r0 >> 4)) * (uint64_t)nw + (uint64_t)wi) * 16u;
+  return reinterpret_cast<const uint16_t*>(p)[mask_element(lane)];
 }
 
 // Writes a strip once: lane l's chunk of PPC pixels in rows
@@ -193,13 +177,402 @@ __device__ inline void store_strip(const StripUnit& u, int srow, int ccol, F&& c
   }
 }
 
-// Waves per SIMD the register allocation of k_tile targets: 7 for 4-byte
-// outputs, 6 for 1- and 2-byte outputs (measured: the latency-bound strip
-// loop gains more from the extra wave than the few spilled registers cost),
-// 5 for 8-byte outputs.
+// A unit's pixels in registers: lane l owns column 64 w + l of every row.
+// 4- and 8-byte pixels take a register (pair) each, px[w * ROWS + r]; 1- and
+// 2-byte pixels are packed, RPW rows of one column to a word, and folded
+// together.
+template <typename T, int ROWS>
+struct Pixels {
+  static constexpr bool PACKED = sizeof(T) <= 2;
+  static constexpr int RPW = PACKED ? 4 / (int)sizeof(T) : 1;
+  static constexpr int NWORD = tile_w(sizeof(T)) / 64;
+  using W = typename std::conditional<PACKED, uint32_t, T>::type;
+  W px[NWORD * ROWS / RPW];
+  __device__ void fill(const StripUnit& u) {
+    W bg;
+    if constexpr (PACKED) bg = lane_splat<T>(u.J->bg_bits);
+    else bg = from_bits<T>(u.J->bg_bits);
+#pragma unroll
+    for (int j = 0; j < NWORD * ROWS / RPW; ++j) px[j] = bg;
+  }
+  // One write of the value bits v in the rows `bits` of tile word w (rows
+  // outside [lo, hi) have none).  A packed sum or count over a background of
+  // 0 is a plain addition of 0 or the value: the empty pixel's rule gives
+  // the same.
+  template <int FUN>
+  __device__ __attribute__((always_inline)) void fold(int w, uint32_t bits, int lo, int hi, uint64_t v, uint64_t bg_bits) {
+    if constexpr (PACKED) {
+      const uint32_t bgw = lane_splat<T>(bg_bits);
+      const uint32_t vw = FUN == 5 ? Lanes<sizeof(T)>::one : lane_splat<T>(v);
+      const bool plain = bgw == 0u;
+#pragma unroll
+      for (int d = 0; d < ROWS / RPW; ++d)
+        if (lo < (d + 1) * RPW && hi > d * RPW) {
+          const uint32_t b = (bits >> (d * RPW)) & ((1u << RPW) - 1u);
+          W& x = px[w * (ROWS / RPW) + d];
+          const uint32_t m = lane_mask<(int)sizeof(T)>(b);
+          if constexpr (FUN == 0 || FUN == 5) {
+            uint32_t y = lane_add<sizeof(T)>(x, vw & m);
+            if (!plain) {
+              const uint32_t e = lane_eq<sizeof(T)>(x, bgw) & m;
+              y = (e & vw) | (~e & y);
+            }
+            x = y;
+          } else {
+            x = fold_word<T, FUN>(x, vw, bgw, m);
+          }
+        }
+    } else {
+      const T val = from_bits<T>(v), bg = from_bits<T>(bg_bits);
+#pragma unroll
+      for (int r0 = 0; r0 < ROWS; r0 += 4)
+        if (lo < r0 + 4 && hi > r0) {
+#pragma unroll
+          for (int r = r0; r < r0 + 4; ++r) {
+            T& x = px[w * ROWS + r];
+            x = bit_select(bit_mask(bits, r), fold_value<T, FUN>(x, val, bg), x);
+          }
+        }
+    }
+  }
+};
+
+// Packed pixels (1- and 2-byte outputs) as rows: f(r, v) with the dwords v of
+// lane l's columns 4 l .. 4 l + 3 in row r, the rows of a dword at a time,
+// exchanged across the lanes in LDS and transposed.  `x`: 256 words of
+// wave-private LDS.
+template <typename T, int ROWS, typename F>
+__device__ inline void each_row(const uint32_t* px, uint32_t* x, int lane, F&& f) {
+  constexpr int RPW = 4 / (int)sizeof(T);  // rows (pixels) per dword
+  constexpr int ND = ROWS / RPW;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) x[w * 64 + lane] = px[w * ND + d];
+    wave_sync();
+    const u32x4 c = *reinterpret_cast<const u32x4*>(x + 4 * lane);  // columns 4 lane .. + 3, RPW rows each
+    wave_sync();
+    uint32_t v[RPW][sizeof(T)];
+    if constexpr (sizeof(T) == 1) {
+      // 4 x 4 bytes transposed: pairs of columns, then of pairs
+      const uint32_t a01 = __builtin_amdgcn_perm(c[1], c[0], 0x05010400u), a23 = __builtin_amdgcn_perm(c[3], c[2], 0x05010400u);
+      const uint32_t b01 = __builtin_amdgcn_perm(c[1], c[0], 0x07030602u), b23 = __builtin_amdgcn_perm(c[3], c[2], 0x07030602u);
+      v[0][0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+      v[1][0] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+      v[2][0] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+      v[3][0] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
+    } else {
+      v[0][0] = __builtin_amdgcn_perm(c[1], c[0], 0x05040100u);
+      v[0][1] = __builtin_amdgcn_perm(c[3], c[2], 0x05040100u);
+      v[1][0] = __builtin_amdgcn_perm(c[1], c[0], 0x07060302u);
+      v[1][1] = __builtin_amdgcn_perm(c[3], c[2], 0x07060302u);
+    }
+#pragma unroll
+    for (int j = 0; j < RPW; ++j) f(d * RPW + j, v[j]);
+  }
+}
+
+// The 4 (1-byte) or 8 bytes of a lane's four pixels.
+template <typename T>
+struct Quad {
+  typedef uint32_t vec __attribute__((ext_vector_type(sizeof(T)), aligned(1)));
+};
+template <>
+struct Quad<uint8_t> {
+  typedef uint32_t vec __attribute__((aligned(1)));
+};
+template <>
+struct Quad<int8_t> : Quad<uint8_t> {};
+
+// Writes four neighbouring pixels of a row from column c on; `part`: those in
+// [lo, hi) only.
+template <typename T>
+__device__ inline void put_quad(T* orow, int32_t c, bool part, int32_t lo, int32_t hi, const uint32_t (&v)[sizeof(T)]) {
+  if (!part || (c >= lo && c + 4 <= hi)) {
+    typename Quad<T>::vec y;
+    __builtin_memcpy(&y, v, 4 * sizeof(T));
+    __builtin_nontemporal_store(y, (typename Quad<T>::vec*)(orow + c));
+  } else {
+    T px[4];
+    __builtin_memcpy(px, v, sizeof(px));
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (c + k >= lo && c + k < hi) orow[c + k] = px[k];
+  }
+}
+
+// Writes a unit's rows (background + burns), each pixel once.
+template <typename T, int ROWS>
+__device__ inline void store_rows(const StripUnit& u, const Pixels<T, ROWS>& p, uint32_t* x, int lane) {
+  T* out = (T*)u.J->out + ((uint64_t)u.layer * (uint64_t)u.nrows + (uint64_t)u.Rw) * (uint64_t)u.ncols;
+  if constexpr (sizeof(T) >= 4) {
+    if (u.C0 + lane < u.ncols) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r)
+        if (u.Rw + r < u.nrows) __builtin_nontemporal_store(p.px[r], out + (uint64_t)r * (uint64_t)u.ncols + u.C0 + lane);
+    }
+  } else {
+    const bool part = u.C0 + tile_w(sizeof(T)) > u.ncols;
+    each_row<T, ROWS>(p.px, x, lane, [&](int r, const uint32_t (&v)[sizeof(T)]) {
+      if (u.Rw + r < u.nrows) put_quad<T>(out + (uint64_t)r * (uint64_t)u.ncols, u.C0 + 4 * lane, part, 0, u.ncols, v);
+    });
+  }
+}
+
+// The strips of a wave's consecutive tiles, written in whole 128-byte lines
+// wherever a row starts: a unit writes a row from the last line start at or
+// before its first column on, with the columns before that from the unit to
+// its left, which it left out.  (A 256-byte piece of a row that starts
+// inside a line takes three lines, two of them in part: 2.3 times as long for
+// float32 of 40,008 columns as of 40,000.)  A unit whose left neighbour was
+// another wave's starts at its own first column, and one whose right
+// neighbour is writes its last columns too.
+template <typename T>
+struct LineWriter {
+  static constexpr int ROWS = WAVE_ROWS, TW = tile_w(sizeof(T));
+  static constexpr int LINE = 128 / (int)sizeof(T);      // pixels of a line
+  static constexpr bool NARROW = sizeof(T) <= 2;
+  // the pixels left out: 4- and 8-byte ones in registers (lanes as in
+  // Pixels), 1- and 2-byte ones in LDS, the last LINE pixels of every row
+  T keep[NARROW ? 1 : ROWS];
+  uint32_t* tail;          // [ROWS][(LINE + TW) * sizeof(T) / 4 + 1] words (narrow)
+  static constexpr int PITCH = (LINE + TW) * (int)sizeof(T) / 4 + 1;
+
+  __device__ static uint32_t skew(const T* p) { return ((uint32_t)(uintptr_t)p & 127u) / (uint32_t)sizeof(T); }
+
+  // cont: the unit to the left left its last pixels out; more: the unit to
+  // the right will write this one's.
+  __device__ void store(const StripUnit& u, const Pixels<T, ROWS>& p, uint32_t* x, int lane, bool cont, bool more) {
+    T* out = (T*)u.J->out + ((uint64_t)u.layer * (uint64_t)u.nrows + (uint64_t)u.Rw) * (uint64_t)u.ncols;
+    if ((skew(out) | ((uint32_t)u.ncols % (uint32_t)LINE)) == 0u) {  // every row starts a line
+      store_rows<T, ROWS>(u, p, x, lane);
+      return;
+    }
+    if constexpr (!NARROW) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        if (u.Rw + r < u.nrows) {
+          T* orow = out + (uint64_t)r * (uint64_t)u.ncols;
+          const int32_t s = (int32_t)skew(orow + u.C0);
+          // lane l: column C0 - s + l, from lane l - s of this unit or, wrapped,
+          // of the one to the left
+          const T v = lane >= 64 - s ? keep[r] : p.px[r];
+          const int from = ((lane - s) & 63) * 4;
+          T y;
+          if constexpr (sizeof(T) == 8) {
+            uint2 w;
+            __builtin_memcpy(&w, &v, 8);
+            w.x = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)w.x);
+            w.y = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)w.y);
+            __builtin_memcpy(&y, &w, 8);
+          } else {
+            int w;
+            __builtin_memcpy(&w, &v, 4);
+            w = __builtin_amdgcn_ds_bpermute(from, w);
+            __builtin_memcpy(&y, &w, 4);
+          }
+          const int32_t c = u.C0 - s + lane;
+          if ((cont || lane >= s) && c < u.ncols) __builtin_nontemporal_store(y, orow + c);
+          if (!more && lane >= 64 - s && u.C0 + lane < u.ncols) orow[u.C0 + lane] = p.px[r];
+          keep[r] = p.px[r];
+        }
+      }
+    } else {
+      constexpr int LW = LINE * (int)sizeof(T) / 4, NW = (int)sizeof(T);  // words of a line, of a lane's pixels
+      each_row<T, ROWS>(p.px, x, lane, [&](int r, const uint32_t (&v)[sizeof(T)]) {
+#pragma unroll
+        for (int k = 0; k < NW; ++k) tail[r * PITCH + LW + lane * NW + k] = v[k];
+      });
+      wave_sync();
+      const bool part = !cont || u.C0 + TW > u.ncols;
+      const int n = min(ROWS, u.nrows - u.Rw);
+      for (int r = 0; r < n; ++r) {
+        T* orow = out + (uint64_t)r * (uint64_t)u.ncols;
+        const int32_t s = (int32_t)skew(orow + u.C0);
+        const int32_t b = LW * 4 + (4 * lane - s) * NW;  // byte of the row's buffer
+        const uint32_t* t = tail + r * PITCH;
+        uint32_t w[NW + 1], y[NW];
+#pragma unroll
+        for (int k = 0; k <= NW; ++k) w[k] = t[(b >> 2) + k];
+#pragma unroll
+        for (int k = 0; k < NW; ++k) y[k] = __builtin_amdgcn_alignbyte(w[k + 1], w[k], (uint32_t)b & 3u);
+        put_quad<T>(orow, u.C0 - s + 4 * lane, part, cont ? 0 : u.C0, u.ncols, y);
+      }
+      for (int r = 0; r < n && !more; ++r) {
+        T* orow = out + (uint64_t)r * (uint64_t)u.ncols;
+        const int32_t s = (int32_t)skew(orow + u.C0);
+        uint32_t y[NW];
+#pragma unroll
+        for (int k = 0; k < NW; ++k) y[k] = tail[r * PITCH + LW + lane * NW + k];
+        if (4 * lane + 4 > TW - s) put_quad<T>(orow, u.C0 + 4 * lane, true, u.C0 + TW - s, u.ncols, y);
+      }
+      // the last line of every row is the next unit's first
+      for (int k = lane; k < ROWS * LW; k += 64) {
+        const int r = k / LW, j = k % LW;
+        tail[r * PITCH + j] = tail[r * PITCH + TW * NW / 4 + j];
+      }
+      wave_sync();
+    }
+  }
+};
+
+// A lane's polygon item of a batch of up to 64: as loaded, then what the
+// folds need of it in one unit.
+struct RawItem {
+  u32x4 box, fq;      // r0, r1, c0, c1; job, band, flags, mask
+  uint32_t kl, v0, v1;  // kind | band, value
+};
+__device__ inline RawItem load_raw(const ItemDesc* d) {
+  const u32x4* q = reinterpret_cast<const u32x4*>(d);
+  const u32x4 a = q[1], b = q[2];
+  return RawItem{q[0], q[3], a[3], b[0], b[1]};
+}
+// Up to 64 visits of a unit in order, visit k in lane k: an item (its value
+// bits v0, v1) and a column of 64 it meets.
+struct Visits {
+  uint32_t blk;   // the mask block
+  uint32_t v0, v1;
+  uint32_t info;  // tile word, first row << 8, row end << 16, no masks << 31
+  uint32_t item;  // lane of the item's descriptor in its batch
+  uint32_t n;     // visits (uniform)
+};
+
+__device__ inline uint32_t push_lane(uint32_t v, uint32_t to) {
+  return (uint32_t)__builtin_amdgcn_ds_permute((int)(to * 4u), (int)v);
+}
+
+// The visits of the batch's items q (lanes `cand`) that meet the unit.  At
+// most 64: `left` returns the lanes whose items did not fit (0 with one word
+// per row), to be passed as `cand` again.  `x`: 256 words of wave-private LDS
+// (more than one word per row).  Every lane calls it.
+template <int NWORD, int ROWS, bool WIDE_VALUE>
+__device__ inline Visits visits_of(const RawItem& q, const StripUnit& u, bool cand, uint64_t& left, uint32_t* x) {
+  const int lane = threadIdx.x & 63;
+  const int32_t r0 = (int32_t)q.box[0], r1 = (int32_t)q.box[1], c0 = (int32_t)q.box[2], c1 = (int32_t)q.box[3];
+  bool hit = cand && r0 < u.strip_r1 && r1 > u.Rw && c0 < u.tile_c1 && c1 > u.C0 && r0 < r1 && c0 < c1 &&
+             (q.kl >> 2) == u.layer;
+  const int32_t nw = mask_row_words(c0, c1);
+  const int32_t wlo = max(0, (c0 >> 6) - (u.C0 >> 6)), whi = min(NWORD - 1, ((c1 - 1) >> 6) - (u.C0 >> 6));
+  const int32_t wi = (u.C0 >> 6) + wlo - (c0 >> 6);  // the item's word in tile word wlo
+  const bool bare = !(q.fq[2] & kItemMask);
+  const uint32_t blk = bare ? 0u : q.fq[3] + (uint32_t)((u.Rw >> 4) - (r0 >> 4)) * (uint32_t)nw + (uint32_t)wi;
+  const uint32_t info = (uint32_t)wlo | (uint32_t)min(max(r0 - u.Rw, 0), ROWS - 1) << 8 |
+                        (uint32_t)min(max(r1 - u.Rw, 0), ROWS) << 16 | (bare ? 1u << 31 : 0u);
+  Visits v{0u, 0u, 0u, 0u, 0u, 0u};
+  left = 0ull;
+  if constexpr (NWORD == 1) {
+    const uint64_t m = __ballot(hit);
+    v.n = (uint32_t)__popcll(m);
+    // (a permutation of all lanes: the others go after the visits)
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t to = hit ? (uint32_t)__popcll(m & below) : v.n + (uint32_t)__popcll(~m & below);
+    v.blk = push_lane(blk, to);
+    v.v0 = push_lane(q.v0, to);
+    if (WIDE_VALUE) v.v1 = push_lane(q.v1, to);
+    v.info = push_lane(info, to);
+    v.item = push_lane((uint32_t)lane, to);
+  } else {
+    const uint32_t words = hit ? (uint32_t)(whi - wlo + 1) : 0u;
+    const uint32_t end = wave_prefix_sum(words);
+    const bool fits = end <= 64u;
+    left = __ballot(hit && !fits);
+    hit = hit && fits;
+    const uint64_t m = __ballot(hit);
+    if (m) v.n = (uint32_t)__builtin_amdgcn_readlane((int)end, 63 - __builtin_clzll(m));
+    wave_sync();
+    if (hit)
+      for (uint32_t j = 0; j < words; ++j)
+        *reinterpret_cast<uint4*>(x + 4u * (end - words + j)) = make_uint4(bare ? 0u : blk + j, q.v0, info + j, (uint32_t)lane);
+    wave_sync();
+    if ((uint32_t)lane < v.n) {
+      const uint4 y = *reinterpret_cast<const uint4*>(x + 4 * lane);
+      v.blk = y.x;
+      v.v0 = y.y;
+      v.info = y.z;
+      v.item = y.w;
+    }
+    wave_sync();
+  }
+  return v;
+}
+
+// Visits whose mask blocks are loaded ahead of their folds.
+template <typename T>
+constexpr int kAhead = sizeof(T) == 8 ? 3 : (sizeof(T) <= 2 ? 2 : 6);
+
+// The column bits (16 rows) of visits k .. k + N - 1 (past the last one: the
+// last one's again).
+template <int N>
+__device__ inline void load_bits(const TileArgs& a, const Visits& v, uint32_t k, uint32_t (&bits)[N], int lane) {
+  const uint16_t* base = reinterpret_cast<const uint16_t*>(a.masks) + mask_element(lane);
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    const uint32_t blk = (uint32_t)__builtin_amdgcn_readlane((int)v.blk, (int)min(k + (uint32_t)g, v.n - 1u));
+    bits[g] = base[(uint64_t)blk * 64u];
+  }
+}
+
+// Folds the visits in order; `bits` holds the first N ones' column bits
+// (load_bits).  Lane l owns column 64 w + l of every row, so its 16 row bits
+// come with one load and each row takes a bit extract, the fold (1 to 5
+// instructions) and a bit select.  (Spreading a row over the lanes that
+// store it took about 80 instructions per item and strip before the folds,
+// and computing the coverage in the strip about 200.  Reading the masks as
+// execution masks through scalar loads needs half the vector instructions,
+// but the scalar cache's misses bound it.)  BARE: items without masks may be
+// among them.
+template <typename T, int FUN, int ROWS, bool BARE, int N, typename F>
+__device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels<T, ROWS>& p, const Visits& v,
+                                   uint32_t (&bits)[N], PolyEdge* stage, int lane, uint32_t& burns, F&& desc_of) {
+  constexpr int NWORD = Pixels<T, ROWS>::NWORD;
+  const int shift = ROWS < 16 ? (u.Rw & 15) : 0;
+  auto fold = [&](uint32_t k, uint32_t y) __attribute__((always_inline)) {
+    const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
+    const uint32_t v0 = (uint32_t)__builtin_amdgcn_readlane((int)v.v0, (int)k);
+    const uint32_t v1 = sizeof(T) == 8 ? (uint32_t)__builtin_amdgcn_readlane((int)v.v1, (int)k) : 0u;
+    if (a.burns) burns += (uint32_t)__popc(y);
+    const int lo = (int)((info >> 8) & 31u), hi = (int)((info >> 16) & 31u);
+#pragma unroll
+    for (int w = 0; w < NWORD; ++w)
+      if (NWORD == 1 || (info & 3u) == (uint32_t)w) {  // (uniform)
+        p.template fold<FUN>(w, y, lo, hi, (uint64_t)v0 | ((uint64_t)v1 << 32), u.J->bg_bits);
+      }
+  };
+  auto rows = [&](uint32_t y) { return ROWS < 16 ? (y >> shift) & ((1u << ROWS) - 1u) : y; };
+  if (BARE && __any((uint32_t)lane < v.n && (v.info >> 31))) {
+    for (uint32_t k = 0; k < v.n; ++k) {
+      const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
+      uint32_t y;
+      if (info >> 31) {
+        y = edge_bits(a, desc_of(__builtin_amdgcn_readlane((int)v.item, (int)k)), u, u.C0 + 64 * (int32_t)(info & 3u), stage,
+                      lane);
+      } else {
+        uint32_t one[1];
+        load_bits(a, v, k, one, lane);
+        y = rows(one[0]);
+      }
+      fold(k, y);
+    }
+    return;
+  }
+  for (uint32_t k = 0; k < v.n; k += (uint32_t)N) {
+    uint32_t nxt[N] = {};
+    const bool more = k + (uint32_t)N < v.n;
+    if (more) load_bits(a, v, k + (uint32_t)N, nxt, lane);
+#pragma unroll
+    for (int g = 0; g < N; ++g)
+      if (k + (uint32_t)g < v.n) fold(k + (uint32_t)g, rows(bits[g]));
+    if (more) {
+#pragma unroll
+      for (int g = 0; g < N; ++g) bits[g] = nxt[g];
+    }
+  }
+}
+
+// Waves per SIMD the register allocation of k_tile targets.
 template <typename T>
 struct TileOccupancy {
-  static constexpr int value = sizeof(T) == 4 ? 7 : (sizeof(T) == 8 ? 5 : 6);
+  static constexpr int value = sizeof(T) == 4 ? 5 : 4;
 };
 
 // Tile kernel of polygon-only groups, one launch per pixel-function group of
@@ -207,173 +580,248 @@ struct TileOccupancy {
 //
 // Per unit (16 rows x TW columns of the job's output): the background fill
 // of RasterInfo::build_raster (rust/src/geo/raster.rs:23-28) and every write
-// of every item meeting the strip, folded in geometry order in registers,
-// then written to HBM once.
+// of every item meeting the strip, folded in geometry order in registers
+// (fold_visits), then written to HBM once.
 //
-// Two lane layouts per wave:
-//  * coverage: lane (rl = lane/4, q = lane%4) takes every 4th active edge of
-//    row rl; the four lanes of a row XOR-combine their crossing toggles and
-//    publish the row's coverage mask in LDS;
-//  * fold / store: lane l owns the 16-byte chunk l % LPR of rows
-//    l / LPR + k * RSTEP, so every store instruction writes whole tile rows
-//    (full 128-byte lines, contiguous across lanes).
-// The polygon path is branch-free per lane (predicated crossings and folds).
-template <typename T, int FUN>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(TileOccupancy<T>::value))) void k_tile(TileArgs a) {
+// The masks and descriptors come from HBM, about 2 us away while the strips
+// are written, and the loads of one strip depend on each other (range,
+// descriptors, masks), so a wave works on four units at once: it folds one
+// (A) while the masks of the next (B), the descriptors of the one after (C)
+// and the range of the last (D) are loading.  A wait for a load waits for
+// everything issued before it, stores included, so all loads of a step are
+// issued at its start, arrive during the fold and are waited for once, after
+// it; the strip is stored last, and its stores complete during the next fold.
+// BARE: compiled with the path for items without masks (its registers would
+// cost the other calls spills).
+template <typename T, int FUN, bool BARE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupancy<T>::value))) void k_tile(TileArgs a) {
   constexpr int TW = tile_w(sizeof(T));
-  constexpr int NWORD = TW / 64;                    // u64 words of a row mask
-  constexpr int PPC = 16 / (int)sizeof(T);          // pixels per 16-byte chunk
-  constexpr int LPR = TW / PPC;                     // lanes per row (store layout)
-  constexpr int RSTEP = 64 / LPR;                   // rows per store instruction
-  constexpr int RPL = WAVE_ROWS / RSTEP;            // rows per lane
-  constexpr int NPIX = RPL * PPC;                   // pixels per lane
-  // 1- and 2-byte outputs keep their pixels packed, four (two) per 32-bit
-  // word, and fold them lane-wise (fold_word)
-  constexpr bool PACKED = sizeof(T) <= 2;
-  constexpr int NW = PACKED ? NPIX * (int)sizeof(T) / 4 : 1;  // words per lane
-  constexpr int PPW = 4 / (int)sizeof(T);                     // pixels per word (packed)
-  __shared__ PolyEdge s_edge[4][64];
-  __shared__ uint64_t s_mask[4][2][WAVE_ROWS][NWORD];
+  constexpr int NWORD = TW / 64;  // mask words per row
+  __shared__ PolyEdge s_edge[BARE ? 4 : 1][64];
+  __shared__ __align__(16) uint32_t s_x[4][NWORD > 1 ? 256 : 1];
+  __shared__ uint32_t s_tail[4][NWORD > 1 ? WAVE_ROWS * LineWriter<T>::PITCH : 1];
 
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rl = lane >> 2, q = lane & 3;            // coverage layout
-  const int srow = lane / LPR, ch = lane % LPR;      // store layout
-  const int ccol = ch * PPC;                         // first local column of the chunk
-  PolyEdge* stage = s_edge[wave];
-  unsigned long long burns = 0;
-  int mbuf = 0;  // alternating row-mask buffer: one wave_sync per polygon item
-
+  const int wave = wave_index(), lane = threadIdx.x & 63;
+  uint32_t burns = 0;
   TileQueue tq(a, wave, lane);
   const RZ_CONST uint32_t* toff_c = as_const(a.tile_off);
-  const RZ_CONST ItemDesc* pdesc_c = as_const(a.pair_desc);
-  const RZ_CONST ItemDesc* desc_c = as_const(a.desc);
-  uint32_t pb = 0, pe = 0;
-  auto fetch_range = [&](uint32_t tl) {
-    if (a.tile_off) {
-      pb = toff_c[a.t_lo + tl];
-      pe = toff_c[a.t_lo + tl + 1u];
-    }
+  int job = 0;
+
+  // a unit's candidates: the tile's list (binned jobs) or the items of the job
+  struct Range {
+    const ItemDesc* list;
+    int64_t ib, ie;
   };
-  bool have = tq.begin();
-  if (have) fetch_range(tq.t_cur);
-  const int32_t strip = wave;
+  constexpr bool WIDE = sizeof(T) == 8;
+  struct Unit {
+    StripUnit u;
+    Range g;
+    bool have;
+  };
+  auto pop_unit = [&](bool have) {  // the next unit, its range loading
+    Unit x{};
+    x.have = have;
+    if (have) {
+      const uint32_t t = a.t_lo + tq.pop();
+      uint32_t pb = 0, pe = 0;
+      if (a.tile_off) {
+        pb = toff_c[t];
+        pe = toff_c[t + 1u];
+      }
+      x.u = strip_unit(a, t, wave * WAVE_ROWS, WAVE_ROWS, TW, job);
+      x.g = x.u.J->scan ? Range{a.desc, x.u.J->i_base, x.u.J->i_base + x.u.J->ni}
+                        : Range{a.pair_desc, (int64_t)pb, (int64_t)pe};
+    }
+    return x;
+  };
+  auto load_first = [&](const Unit& x) {
+    RawItem q{};
+    if (x.have && x.g.ib + lane < x.g.ie) q = load_raw(x.g.list + x.g.ib + lane);
+    return q;
+  };
+  auto first_visits = [&](const Unit& x, const RawItem& q, uint64_t& left) {
+    return visits_of<NWORD, WAVE_ROWS, WIDE>(q, x.u, x.have && x.g.ib + lane < x.g.ie, left, s_x[wave]);
+  };
 
-  while (have) {
-    const uint32_t t = a.t_lo + tq.pop();
-    const StripUnit u = strip_unit(a, t, strip, TW);
-    const RZ_CONST JobDev& J = *u.J;
-    const T bg = from_bits<T>(J.bg_bits);
-    // heavy tile (many items): every polygon mask comes from the pre-pass
-    // (a tile is heavy iff its pair range holds at least heavy_min items, so
-    // the slot base is only loaded for heavy tiles)
-    uint64_t hbase = 0;
-    const bool hb_ok = a.heavy_base && !J.scan && pe - pb >= a.heavy_min;
-    if (hb_ok) hbase = as_const(a.heavy_base)[t];
+  Unit A = pop_unit(tq.begin()), B{}, C{};
+  if (A.have) B = pop_unit(tq.advance());
+  if (B.have) C = pop_unit(tq.advance());
+  uint64_t left_a = 0, left_b = 0;  // lanes of the first batch whose visits are still to come
+  uint32_t bits_a[kAhead<T>] = {};
+  Visits va{}, vb{};
+  if (A.have) {
+    const RawItem qa = load_first(A), qb = load_first(B);
+    va = first_visits(A, qa, left_a);
+    vb = first_visits(B, qb, left_b);
+    if (va.n) load_bits(a, va, 0u, bits_a, lane);
+  }
+  LineWriter<T> lines;
+  lines.tail = s_tail[wave];
+  bool cont = false;
+  while (A.have) {
+    uint32_t bits_b[kAhead<T>] = {};
+    if (vb.n) load_bits(a, vb, 0u, bits_b, lane);
+    const RawItem qc = load_first(C);
+    const Unit D = pop_unit(C.have && tq.advance());
 
-    T acc[PACKED ? 1 : NPIX];  // acc[k * PPC + j]: row srow + k*RSTEP, column ccol + j
-    uint32_t accw[NW];         // packed: pixel k * PPC + j in word (k * PPC + j) / PPW
-    const uint32_t bgw = PACKED ? lane_splat<T>(J.bg_bits) : 0u;
-    if constexpr (PACKED) {
-#pragma unroll
-      for (int i = 0; i < NW; ++i) accw[i] = bgw;
-    } else {
-#pragma unroll
-      for (int j = 0; j < NPIX; ++j) acc[j] = bg;
+    Pixels<T, WAVE_ROWS> p;
+    p.fill(A.u);
+    if (va.n)
+      fold_visits<T, FUN, WAVE_ROWS, BARE>(a, A.u, p, va, bits_a, s_edge[BARE ? wave : 0], lane, burns,
+                                           [&](int b) { return load_desc(as_const(A.g.list) + A.g.ib + b); });
+    // the candidates past the first batch (64 items or visits), in order; scan
+    // jobs of one band test the 8-byte boxes in strip and tile units first
+    for (int64_t base = A.g.ib; left_a || base + 64 < A.g.ie;) {
+      bool cand;
+      if (NWORD > 1 && left_a) {
+        cand = (left_a >> lane) & 1ull;
+      } else {
+        base += 64;
+        cand = base + lane < A.g.ie;
+        if (cand && A.u.J->scan && A.u.J->scan_compact && a.scan_box)
+          cand = scan_box_meets(a.scan_box[base + lane], (uint32_t)A.u.Rw / WAVE_ROWS, (uint32_t)A.u.C0 / (uint32_t)TW);
+      }
+      RawItem q{};
+      if (cand) q = load_raw(A.g.list + base + lane);
+      const Visits v = visits_of<NWORD, WAVE_ROWS, WIDE>(q, A.u, cand, left_a, s_x[wave]);
+      if (!v.n) continue;
+      uint32_t bits[kAhead<T>];
+      load_bits(a, v, 0u, bits, lane);
+      fold_visits<T, FUN, WAVE_ROWS, BARE>(a, A.u, p, v, bits, s_edge[BARE ? wave : 0], lane, burns,
+                                           [&](int b) { return load_desc(as_const(A.g.list) + base + b); });
     }
 
-    auto process_item = [&](const ItemDesc d, uint32_t pi) {
-      // wave-uniform skip: the item box misses this strip
-      if (d.r1 <= u.Rw || d.r0 >= u.strip_r1 || d.c1 <= u.C0 || d.c0 >= u.tile_c1) return;
-      const T v = from_bits<T>(d.value);
-      const uint64_t vbits = d.value;
-      const uint64_t cov = polygon_mask<NWORD>(a, d, u, hb_ok, hbase, pb, pe, pi, strip, stage, lane);
-      if (q < NWORD) s_mask[wave][mbuf][rl][q] = cov;
-      wave_sync();
+    // everything loaded has arrived
 #pragma unroll
-      for (int k = 0; k < RPL; ++k) {
-        const uint64_t row_word = s_mask[wave][mbuf][srow + k * RSTEP][ccol >> 6];
-        const uint32_t bits = (uint32_t)(row_word >> (ccol & 63)) & ((1u << PPC) - 1u);
-        if (__any(bits != 0u)) {  // wave-uniform skip of uncovered row groups
-          burns += (unsigned long long)__popc(bits);
-          if constexpr (PACKED) {
-            const uint32_t vw = lane_splat<T>(vbits);
+    for (int g = 0; g < kAhead<T>; ++g) asm volatile("" : "+v"(bits_b[g]));
+    asm volatile("" : "+v"(tq.pending));
+    uint64_t left_c = 0;
+    const Visits vc = first_visits(C, qc, left_c);
+    // (neighbours: the next tile of the same rows)
+    const bool more = B.have && B.u.J == A.u.J && B.u.layer == A.u.layer && B.u.Rw == A.u.Rw && B.u.C0 == A.u.C0 + TW;
+    lines.store(A.u, p, s_x[wave], lane, cont, more);
+    cont = more;
+    A = B;
+    B = C;
+    C = D;
+    va = vb;
+    vb = vc;
+    left_a = left_b;
+    left_b = left_c;
 #pragma unroll
-            for (int i = 0; i < PPC / PPW; ++i)
-              accw[k * (PPC / PPW) + i] = fold_word<T, FUN>(
-                  accw[k * (PPC / PPW) + i], vw, bgw,
-                  lane_mask<(int)sizeof(T)>((bits >> (i * PPW)) & ((1u << PPW) - 1u)));
-          } else {
-#pragma unroll
-            for (int j = 0; j < PPC; ++j)
-              acc[k * PPC + j] = fold_select<T, FUN>(acc[k * PPC + j], v, bg, (bits >> j) & 1u);
-          }
-        }
-      }
-      mbuf ^= 1;  // the next polygon writes the other buffer
-    };
-
-    if (!J.scan) {
-      // (a heavy tile of a polygon-only group is folded by k_tile_heavy,
-      // which runs after this kernel and stores over this strip)
-      const uint32_t pend = (hb_ok && a.heavy_split) ? pb : pe;
-      for (uint32_t i = pb; i < pend; ++i) process_item(load_desc(pdesc_c + i), i);
-    } else if (J.scan_compact && a.scan_box) {
-      // scan job of one band: the 8-byte item boxes in strip and tile units,
-      // 64 at a time, the next 64 loaded while this batch's hits are
-      // processed
-      const int64_t ib = J.i_base, ie = J.i_base + J.ni;
-      const uint32_t sidx = (uint32_t)u.Rw / WAVE_ROWS, tx = (uint32_t)u.C0 / (uint32_t)TW;
-      const uint2* sb = a.scan_box;
-      uint2 nbx = ib + lane < ie ? sb[ib + lane] : make_uint2(0xFFFFu, 0u);
-      for (int64_t base = ib; base < ie; base += 64) {
-        const uint2 bx = nbx;
-        const bool valid = base + lane < ie;
-        if (base + 64 + lane < ie) nbx = sb[base + 64 + lane];
-        uint64_t m = __ballot(valid && scan_box_meets(bx, sidx, tx));
-        while (m) {
-          const int bit = __builtin_ctzll(m);
-          m &= m - 1;
-          process_item(load_desc(desc_c + base + bit), 0u);
-        }
-      }
-    } else {
-      // scan job: test every item's box in order (small item counts), 64
-      // boxes at a time, the next 64 loaded while this batch's hits are
-      // processed
-      const int64_t ib = J.i_base, ie = J.i_base + J.ni;
-      BoxLayer nbx = ib + lane < ie ? load_box(desc_c + ib + lane) : BoxLayer{0, 0, 0, 0, 0u};
-      for (int64_t base = ib; base < ie; base += 64) {
-        const BoxLayer bx = nbx;
-        const bool valid = base + lane < ie;
-        if (base + 64 + lane < ie) nbx = load_box(desc_c + base + 64 + lane);
-        const bool hit = valid && (bx.kind_layer >> 2) == u.layer && bx.r0 < u.strip_r1 && bx.r1 > u.Rw &&
-                         bx.c0 < u.tile_c1 && bx.c1 > u.C0 && bx.r0 < bx.r1 && bx.c0 < bx.c1;
-        uint64_t m = __ballot(hit);
-        while (m) {
-          const int bit = __builtin_ctzll(m);
-          m &= m - 1;
-          process_item(load_desc(desc_c + base + bit), 0u);
-        }
-      }
-    }
-
-    // take the next tile (and its item range) before this strip's stores
-    have = tq.advance();
-    if (have) fetch_range(tq.t_cur);
-
-    // ---- write the strip once (background + burns)
-    store_strip<T, PPC, RPL, RSTEP>(u, srow, ccol, [&](int k) {
-      u32x4 vec;
-      if constexpr (PACKED) vec = u32x4{accw[k * 4], accw[k * 4 + 1], accw[k * 4 + 2], accw[k * 4 + 3]};
-      else __builtin_memcpy(&vec, &acc[k * PPC], 16);
-      return vec;
-    });
+    for (int g = 0; g < kAhead<T>; ++g) bits_a[g] = bits_b[g];
   }
   if (a.burns) {
+    unsigned long long n = burns;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) burns += __shfl_xor(burns, off, 64);
-    if (lane == 0 && burns) atomicAdd(&a.burns[blockIdx.x % kBurnSlots], burns);
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (lane == 0 && n) atomicAdd(&a.burns[blockIdx.x % kBurnSlots], n);
+  }
+}
+
+// The same for launches of few tiles, where latency counts: a workgroup per
+// tile, 8 rows to a wave, so a dense tile's items are folded by twice the
+// waves; the waves of a scan job's tile test 64 boxes each and share the list
+// of those that meet the tile (every strip testing every box took half of the
+// kernel's instructions on 1,000 items); and the pixel function is the job's,
+// so one launch takes the groups of all functions (32 jobs of 256 to 1,024
+// pixels square: 47 us, a launch per function one after the other 165).
+// Bound by the chain from the job record over the boxes, the descriptors and
+// the masks to the stores, so as many tiles as possible are resident: with 8
+// waves 1,000 stars on 2048 x 2048 take 17.4 us, with 16 waves (4 rows each,
+// half the tiles at a time) 23.5, with 4 waves 16.5 but 52 on the 32 jobs.
+constexpr int kTileBlockWaves = 8;
+template <typename T>
+__global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a) {
+  constexpr int TW = tile_w(sizeof(T));
+  constexpr int NWORD = TW / 64;
+  constexpr int ROWS = TILE_H / kTileBlockWaves;
+  __shared__ PolyEdge s_edge[kTileBlockWaves][64];
+  __shared__ __align__(16) uint32_t s_x[kTileBlockWaves][NWORD > 1 ? 256 : 1];
+  __shared__ uint32_t s_list[64 * kTileBlockWaves], s_n[kTileBlockWaves];
+  const int wave = wave_index(), lane = threadIdx.x & 63;
+  uint32_t burns = 0;
+  // neighbouring tiles on one XCD (workgroup b runs on XCD b % 8)
+  const uint32_t n_tiles = a.t_hi - a.t_lo, xcd = blockIdx.x % NUM_XCD;
+  const uint32_t tl = xcd_unit_lo(xcd, n_tiles) + blockIdx.x / NUM_XCD;
+  if (tl >= xcd_unit_lo(xcd + 1u, n_tiles)) return;  // (the whole workgroup)
+  int job = 0;
+  const StripUnit u = strip_unit(a, a.t_lo + tl, wave * ROWS, ROWS, TW, job);
+  const RZ_CONST JobDev& J = *u.J;
+  Pixels<T, ROWS> p;
+  p.fill(u);
+  auto fold = [&](const ItemDesc* d, bool cand) __attribute__((always_inline)) {
+    RawItem q{};
+    if (cand) q = load_raw(d);
+    uint64_t left = __ballot(cand);
+    while (left) {
+      const Visits v = visits_of<NWORD, ROWS, sizeof(T) == 8>(q, u, (left >> lane) & 1ull, left, s_x[wave]);
+      if (!v.n) break;
+      uint32_t bits[kAhead<T>];
+      load_bits(a, v, 0u, bits, lane);
+      auto desc_of = [&](int b) {
+        const uint64_t at = (uint64_t)d;
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, b);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), b);
+        return load_desc((const RZ_CONST ItemDesc*)((uint64_t)lo | ((uint64_t)hi << 32)));
+      };
+      auto fold_fun = [&](auto fun) __attribute__((always_inline)) {
+        fold_visits<T, decltype(fun)::value, ROWS, true>(a, u, p, v, bits, s_edge[wave], lane, burns, desc_of);
+      };
+      switch (J.fun) {
+        case 0: fold_fun(std::integral_constant<int, 0>{}); break;
+        case 1: fold_fun(std::integral_constant<int, 1>{}); break;
+        case 2: fold_fun(std::integral_constant<int, 2>{}); break;
+        case 3: fold_fun(std::integral_constant<int, 3>{}); break;
+        case 4: fold_fun(std::integral_constant<int, 4>{}); break;
+        case 5: fold_fun(std::integral_constant<int, 5>{}); break;
+        default: fold_fun(std::integral_constant<int, 6>{}); break;
+      }
+    }
+  };
+  if (!J.scan) {
+    const uint32_t pb = as_const(a.tile_off)[a.t_lo + tl], pe = as_const(a.tile_off)[a.t_lo + tl + 1u];
+    for (uint32_t i = pb; i < pe; i += 64u) fold(a.pair_desc + i + lane, (uint32_t)lane < pe - i);
+  } else {
+    const bool compact = J.scan_compact && a.scan_box;
+    const int32_t T0 = u.Rw - wave * ROWS, T1 = min(T0 + TILE_H, u.nrows);  // the tile's rows
+    for (int64_t base = 0; base < J.ni; base += 64 * kTileBlockWaves) {
+      const int64_t i = base + wave * 64 + lane;
+      bool meets = i < J.ni;
+      if (meets) {
+        if (compact) {
+          const uint2 bx = a.scan_box[J.i_base + i];
+          const uint32_t tx = (uint32_t)u.C0 / (uint32_t)TW, s0 = (uint32_t)T0 / WAVE_ROWS;
+          meets = (bx.x & 0xFFFFu) <= s0 + TILE_H / WAVE_ROWS - 1 && s0 <= (bx.x >> 16) && (bx.y & 0xFFFFu) <= tx &&
+                  tx <= (bx.y >> 16);
+        } else {
+          const u32x4 q = *reinterpret_cast<const u32x4*>(a.desc + J.i_base + i);
+          meets = (int32_t)q[0] < T1 && (int32_t)q[1] > T0 && (int32_t)q[2] < u.tile_c1 && (int32_t)q[3] > u.C0;
+        }
+      }
+      const uint64_t m = __ballot(meets);
+      if (lane == 0) s_n[wave] = (uint32_t)__popcll(m);
+      __syncthreads();
+      uint32_t n = 0, at = 0;
+      for (int w = 0; w < kTileBlockWaves; ++w) {
+        if (w == wave) at = n;
+        n += s_n[w];
+      }
+      if (meets) s_list[at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)(i - base);
+      __syncthreads();
+      for (uint32_t k = 0; k < n; k += 64u) {
+        const bool cand = k + (uint32_t)lane < n;
+        fold(a.desc + J.i_base + base + (cand ? (int64_t)s_list[k + lane] : 0), cand);
+      }
+      __syncthreads();  // the next boxes overwrite the list
+    }
+  }
+  store_rows<T, ROWS>(u, p, s_x[wave], lane);
+  if (a.burns) {
+    unsigned long long n = burns;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (lane == 0 && n) atomicAdd(&a.burns[(blockIdx.x * kTileBlockWaves + wave) % kBurnSlots], n);
   }
 }
 
@@ -447,7 +895,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   constexpr int CW = NPIXS * CB / 32;                  // words of one item's counters
   constexpr int KCNT = COUNTED ? (CNT_WORDS / CW < KGRP ? CNT_WORDS / CW : KGRP) : 1;
   __shared__ PolyEdge s_edge[4][64];
-  __shared__ uint64_t s_mask[4][2][WAVE_ROWS][NWORD];
   __shared__ __align__(16) T s_acc[4][NPIXS];
   __shared__ __align__(16) uint32_t s_cnt[4][CNT_WORDS];
   __shared__ uint32_t s_mark[4][KGRP * MW];
@@ -456,8 +903,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   constexpr bool FSUM = FUN == 0 && (sizeof(T) == 4 || sizeof(T) == 8) && (T)0.5 != (T)0;
   __shared__ uint32_t s_wr[4][FSUM ? NPIXS / 32 : 1];
 
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rl = lane >> 2, q = lane & 3;
+  const int wave = wave_index(), lane = threadIdx.x & 63;
   const int srow = lane / LPR, ch = lane % LPR;
   const int ccol = ch * PPC;
   PolyEdge* stage = s_edge[wave];
@@ -470,7 +916,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     for (int w = lane; w < CNT_WORDS; w += 64) cnt[w] = 0u;
   for (int w = lane; w < KGRP * MW; w += 64) mark[w] = 0u;
   unsigned long long burns = 0;
-  int mbuf = 0;
 
   TileQueue tq(a, wave, lane);
   const RZ_CONST uint32_t* toff_c = as_const(a.tile_off);
@@ -486,15 +931,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   bool have = tq.begin();
   if (have) fetch_range(tq.t_cur);
   const int32_t strip = wave;
+  int job = 0;
 
   while (have) {
     const uint32_t t = a.t_lo + tq.pop();
-    const StripUnit u = strip_unit(a, t, strip, TW);
+    const StripUnit u = strip_unit(a, t, strip * WAVE_ROWS, WAVE_ROWS, TW, job);
     const RZ_CONST JobDev& J = *u.J;
     const T bg = from_bits<T>(J.bg_bits);
-    uint64_t hbase = 0;
-    const bool hb_ok = a.heavy_base && !J.scan && pe - pb >= a.heavy_min;
-    if (hb_ok) hbase = as_const(a.heavy_base)[t];
     const bool dedup_job = J.dedup_lines != 0;
     const bool at_job = J.all_touched != 0;
 
@@ -567,63 +1010,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // does not contain: inside the cache window that is every fill pixel off
     // the outline, again the union; a fill pixel outside the window is
     // skipped when the cache bit its wrapped index lands on is set.
-    auto polygon_at = [&](const ItemDesc& d, uint32_t pi) {
+    auto polygon_at = [&](const ItemDesc& d) {
       const T v = from_bits<T>(d.value);
       for (int64_t e = lane; e < d.nv; e += 64) walk_at(d.vbeg + e - J.v_base, mark);
-      const uint64_t cov = polygon_mask<NWORD>(a, d, u, hb_ok, hbase, pb, pe, pi, strip, stage, lane);
       wave_sync();
-      if (q < NWORD) {
-        uint64_t m = cov;
-        if (COUNTED && (d.flags & kItemAtCache) && m && a.at_bits && a.at_base[d.last + 1] <= a.at_cap) {
-          CacheWin cw;
-          item_cache(a.item_win, (int64_t)d.last, cw);
-          const uint64_t length = cw.cap / cw.width;
-          const unsigned long long* bits = a.at_bits + a.at_base[d.last];
-          const int64_t y = (int64_t)u.Rw + rl, xb = (int64_t)u.C0 + q * 64;
-          for (uint64_t mm = m; mm; mm &= mm - 1) {
-            const int b = __builtin_ctzll(mm);
-            const int64_t x = xb + b;
-            if ((uint64_t)x - (uint64_t)cw.x0 < cw.width && (uint64_t)y - (uint64_t)cw.y0 < length) continue;
-            const uint64_t ci = cache_index(cw, x, y);
-            if (ci < cw.cap && ((bits[ci >> 6] >> (ci & 63)) & 1ull)) m &= ~(1ull << b);
-          }
+      // the fill's row words: word w of row `lane` in lanes 0 .. 15
+      for (int w = 0; w < NWORD; ++w) {
+        const uint32_t bits = column_bits(a, d, u, w, stage, lane);
+        uint64_t m = 0ull;
+        for (int r = 0; r < WAVE_ROWS; ++r) {
+          const uint64_t row = __ballot((bits >> r) & 1u);
+          if (lane == r) m = row;
         }
-        const int idx = rl * TW + q * 64;
-        mark[idx >> 5] |= (uint32_t)m;
-        mark[(idx >> 5) + 1] |= (uint32_t)(m >> 32);
+        if (lane < WAVE_ROWS) {
+          if (COUNTED && (d.flags & kItemAtCache) && m && a.at_bits && a.at_base[d.last + 1] <= a.at_cap) {
+            CacheWin cw;
+            item_cache(a.item_win, (int64_t)d.last, cw);
+            const uint64_t length = cw.cap / cw.width;
+            const unsigned long long* cb = a.at_bits + a.at_base[d.last];
+            const int64_t y = (int64_t)u.Rw + lane, xb = (int64_t)u.C0 + w * 64;
+            for (uint64_t mm = m; mm; mm &= mm - 1) {
+              const int b = __builtin_ctzll(mm);
+              const int64_t x = xb + b;
+              if ((uint64_t)x - (uint64_t)cw.x0 < cw.width && (uint64_t)y - (uint64_t)cw.y0 < length) continue;
+              const uint64_t ci = cache_index(cw, x, y);
+              if (ci < cw.cap && ((cb[ci >> 6] >> (ci & 63)) & 1ull)) m &= ~(1ull << b);
+            }
+          }
+          const int idx = lane * TW + w * 64;
+          mark[idx >> 5] |= (uint32_t)m;
+          mark[(idx >> 5) + 1] |= (uint32_t)(m >> 32);
+        }
       }
       apply_marks(v);
     };
 
-    auto polygon = [&](const ItemDesc& d, uint32_t pi) {
+    auto polygon = [&](const ItemDesc& d) {
       const T v = from_bits<T>(d.value);
-      const uint64_t cov = polygon_mask<NWORD>(a, d, u, hb_ok, hbase, pb, pe, pi, strip, stage, lane);
-      if (q < NWORD) s_mask[wave][mbuf][rl][q] = cov;
-      wave_sync();
-#pragma unroll
-      for (int k = 0; k < RPL; ++k) {
-        const int r = srow + k * RSTEP;
-        const uint64_t row_word = s_mask[wave][mbuf][r][ccol >> 6];
-        const uint32_t bits = (uint32_t)(row_word >> (ccol & 63)) & ((1u << PPC) - 1u);
-        if (__any(bits != 0u)) {
-          burns += (unsigned long long)__popc(bits);
-          T* p = acc + r * TW + ccol;
-          T px[PPC];
-          __builtin_memcpy(px, p, 16);
-          if (FSUM && unord) {
-#pragma unroll
-            for (int j = 0; j < PPC; ++j) px[j] = ((bits >> j) & 1u) ? px[j] + v : px[j];
-            const int idx = r * TW + ccol;
-            if (bits) atomicOr(&wr[idx >> 5], bits << (idx & 31));
-          } else {
-#pragma unroll
-            for (int j = 0; j < PPC; ++j) px[j] = fold_select<T, FUN>(px[j], v, bg, (bits >> j) & 1u);
+      for (int w = 0; w < NWORD; ++w) {
+        const uint32_t bits = column_bits(a, d, u, w, stage, lane);
+        burns += (unsigned long long)__popc(bits);
+        // (lane: a column; each row's pixels are one LDS access)
+        for (int r = 0; r < WAVE_ROWS; ++r) {
+          if (!__any((bits >> r) & 1u)) continue;
+          if ((bits >> r) & 1u) {
+            const int idx = r * TW + w * 64 + lane;
+            if (FSUM && unord) {
+              acc[idx] = acc[idx] + v;
+              atomicOr(&wr[idx >> 5], 1u << (idx & 31));
+            } else {
+              acc[idx] = fold_select<T, FUN>(acc[idx], v, bg, true);
+            }
           }
-          __builtin_memcpy(p, px, 16);
         }
       }
       wave_sync();
-      mbuf ^= 1;
     };
 
     // a line or a multi-point item: its segment / cell records, lanes over
@@ -1012,11 +1453,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       fold_points(P & ~C);
     };
 
-    auto process_item = [&](const ItemDesc& d, uint32_t pi) {
+    auto process_item = [&](const ItemDesc& d) {
       if (d.r1 <= u.Rw || d.r0 >= u.strip_r1 || d.c1 <= u.C0 || d.c0 >= u.tile_c1) return;
       if ((d.kind_layer & 3u) == 0u) {
-        if (at_job) polygon_at(d, pi);
-        else polygon(d, pi);
+        if (at_job) polygon_at(d);
+        else polygon(d);
       } else {
         const uint4* recs;
         uint32_t n_r;
@@ -1138,9 +1579,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             const bool banded = __builtin_amdgcn_readlane((int)bnd, p) != 0;
             lines(d, recs, n_r, banded, cur);
           } else if (at_job) {
-            polygon_at(d, i0 + (uint32_t)p);
+            polygon_at(d);
           } else {
-            polygon(d, i0 + (uint32_t)p);
+            polygon(d);
           }
         }
       }
@@ -1160,7 +1601,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         while (m) {
           const int bit = __builtin_ctzll(m);
           m &= m - 1;
-          process_item(load_desc(desc_c + base + bit), 0u);
+          process_item(load_desc(desc_c + base + bit));
         }
       }
     } else {
@@ -1179,7 +1620,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         while (m) {
           const int bit = __builtin_ctzll(m);
           m &= m - 1;
-          process_item(load_desc(desc_c + base + bit), 0u);
+          process_item(load_desc(desc_c + base + bit));
         }
       }
     }
@@ -1203,173 +1644,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       return vec;
     });
     wave_sync();  // the next strip's background overwrites these pixels
-  }
-  if (a.burns) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) burns += __shfl_xor(burns, off, 64);
-    if (lane == 0 && burns) atomicAdd(&a.burns[blockIdx.x % kBurnSlots], burns);
-  }
-}
-
-// Heavy tiles of a polygon-only group (k_tile skips them): one wave per
-// (heavy tile, strip) unit, taken from a work counter.  Every item's strip
-// mask was written by the pre-pass (k_cover), strip-major per tile.  Masks
-// and descriptors go through LDS kBlk items at a time: the next block is
-// loaded into registers while the current block is folded from LDS, then
-// stored to LDS, so the per-item loads of a tile with thousands of items
-// overlap instead of serialising.  Same folds, geometry order and stores as
-// k_tile.
-template <typename T, int FUN>
-__global__ __launch_bounds__(256) void k_tile_heavy(TileArgs a) {
-  constexpr int TW = tile_w(sizeof(T));
-  constexpr int NWORD = TW / 64;
-  constexpr int PPC = 16 / (int)sizeof(T);
-  constexpr int LPR = TW / PPC;
-  constexpr int RSTEP = 64 / LPR;
-  constexpr int RPL = WAVE_ROWS / RSTEP;
-  constexpr int NPIX = RPL * PPC;
-  constexpr bool PACKED = sizeof(T) <= 2;  // pixels packed in 32-bit words (fold_word)
-  constexpr int NW = PACKED ? NPIX * (int)sizeof(T) / 4 : 1;
-  constexpr int PPW = 4 / (int)sizeof(T);
-  constexpr int SW = 16 * NWORD;          // words of one item's strip mask
-  constexpr uint32_t kBlk = 256 / SW;     // items per block (16 or 4)
-  __shared__ uint64_t s_mk[4][256];
-  __shared__ ItemDesc s_ds[4][16];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int srow = lane / LPR, ch = lane % LPR, ccol = ch * PPC;
-  const RZ_CONST JobDev* jobs_c = as_const(a.jobs);
-  const RZ_CONST int64_t* tend_c = as_const(a.job_tend);
-  // this launch's heavy tiles: heavy_list[h0 .. h1), four units (strips) each
-  const uint32_t h0 = a.heavy_rank[a.t_lo], units = 4u * (a.heavy_rank[a.t_hi] - h0);
-  // units per counter grab: a few per wave of the grid, at most 16
-  const uint32_t grab = max(1u, min(16u, units / (gridDim.x * 4u * 4u)));
-  uint64_t* mk = s_mk[wave];
-  ItemDesc* ds = s_ds[wave];
-  unsigned long long burns = 0;
-  // A wave's first units are its own share (no atomic), and the counter hands
-  // out those past every wave's share.  One atomic per wave to learn that no
-  // unit is left took 95 us a launch on its own (8,192 waves on one word,
-  // about 11.6 ns each); most launches have fewer units than waves.
-  const uint32_t first = gridDim.x * 4u * grab;
-  uint32_t u = min(units, (blockIdx.x * 4u + (uint32_t)wave) * grab), u_end = min(units, u + grab);
-  for (;;) {
-    if (u == u_end) {
-      if (first >= units) break;
-      uint32_t g = 0;
-      if (lane == 0) g = atomicAdd(a.heavy_ctr, grab);
-      u = first + (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
-      if (u >= units) break;
-      u_end = min(u + grab, units);
-    }
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.heavy_list[h0 + (u >> 2)]);
-    const int32_t strip = (int32_t)(u & 3u);
-    ++u;
-    const RZ_CONST JobDev& J = jobs_c[find_job(tend_c, a.n_jobs, (int64_t)t)];
-    const int32_t nrows = J.nrows, ncols = J.ncols;
-    const T bg = from_bits<T>(J.bg_bits);
-    const uint32_t tj = t - J.tile_base;
-    const uint32_t layer = tj / J.tiles_per_layer;
-    const uint32_t tl = tj - layer * J.tiles_per_layer;
-    const int32_t ty = (int32_t)(tl / (uint32_t)J.ntx), tx = (int32_t)(tl % (uint32_t)J.ntx);
-    const int32_t C0 = tx * TW, Rw = ty * TILE_H + strip * WAVE_ROWS;
-    const int32_t strip_r1 = min(Rw + WAVE_ROWS, nrows), tile_c1 = min(C0 + TW, ncols);
-    const uint32_t pb = a.tile_off[t], cnt = a.tile_off[t + 1] - pb;
-    const uint64_t* sbase = a.masks + (a.heavy_base[t] * 4u + (uint64_t)strip * cnt) * a.slot_words;
-    const ItemDesc* dbase = a.pair_desc + pb;
-
-    T acc[PACKED ? 1 : NPIX];
-    uint32_t accw[NW];
-    const uint32_t bgw = PACKED ? lane_splat<T>(J.bg_bits) : 0u;
-    if constexpr (PACKED) {
-#pragma unroll
-      for (int i = 0; i < NW; ++i) accw[i] = bgw;
-    } else {
-#pragma unroll
-      for (int j = 0; j < NPIX; ++j) acc[j] = bg;
-    }
-
-    // block j0 into registers: masks (lane L: words 4L .. 4L + 3 of the
-    // block) and descriptors (lane L: bytes 16 (L % 4) .. of descriptor L / 4)
-    const uint32_t jm = (uint32_t)(lane * 4) / SW, om = (uint32_t)(lane * 4) % SW, jd = (uint32_t)lane >> 2;
-    uint4 m_lo = make_uint4(0u, 0u, 0u, 0u), m_hi = m_lo, d_q = m_lo;
-    auto load_block = [&](uint32_t j0) {
-      if (j0 + jm < cnt) {
-        const uint4* src = reinterpret_cast<const uint4*>(sbase + (uint64_t)(j0 + jm) * a.slot_words + om);
-        m_lo = src[0];
-        m_hi = src[1];
-      }
-      if (jd < kBlk && j0 + jd < cnt)
-        d_q = reinterpret_cast<const uint4*>(dbase + j0 + jd)[lane & 3];
-    };
-    auto stage_block = [&]() {
-      wave_sync();  // the previous block's reads are done
-      uint4* dm = reinterpret_cast<uint4*>(mk + lane * 4);
-      dm[0] = m_lo;
-      dm[1] = m_hi;
-      if (jd < kBlk) reinterpret_cast<uint4*>(ds + jd)[lane & 3] = d_q;
-      wave_sync();
-    };
-    load_block(0u);
-    for (uint32_t j0 = 0; j0 < cnt; j0 += kBlk) {
-      stage_block();
-      if (j0 + kBlk < cnt) load_block(j0 + kBlk);  // in flight during the folds below
-      const uint32_t gn = min(kBlk, cnt - j0);
-      for (uint32_t g = 0; g < gn; ++g) {
-        const ItemDesc& d = ds[g];
-        if (d.r1 <= Rw || d.r0 >= strip_r1 || d.c1 <= C0 || d.c0 >= tile_c1) continue;
-        const T v = from_bits<T>(d.value);
-        const uint64_t vbits = d.value;
-        const uint64_t* m = mk + g * SW;
-#pragma unroll
-        for (int k = 0; k < RPL; ++k) {
-          const uint64_t row_word = m[(srow + k * RSTEP) * NWORD + (ccol >> 6)];
-          const uint32_t bits = (uint32_t)(row_word >> (ccol & 63)) & ((1u << PPC) - 1u);
-          if (__any(bits != 0u)) {
-            burns += (unsigned long long)__popc(bits);
-            if constexpr (PACKED) {
-              const uint32_t vw = lane_splat<T>(vbits);
-#pragma unroll
-              for (int i = 0; i < PPC / PPW; ++i)
-                accw[k * (PPC / PPW) + i] = fold_word<T, FUN>(
-                    accw[k * (PPC / PPW) + i], vw, bgw,
-                    lane_mask<(int)sizeof(T)>((bits >> (i * PPW)) & ((1u << PPW) - 1u)));
-            } else {
-#pragma unroll
-              for (int j = 0; j < PPC; ++j)
-                acc[k * PPC + j] = fold_select<T, FUN>(acc[k * PPC + j], v, bg, (bits >> j) & 1u);
-            }
-          }
-        }
-      }
-    }
-
-    // write the strip once, as k_tile does
-    const int32_t c = C0 + ccol;
-#pragma unroll
-    for (int k = 0; k < RPL; ++k) {
-      const int32_t row = Rw + srow + k * RSTEP;
-      if (row < nrows) {
-        T* orow = (T*)J.out + ((uint64_t)layer * (uint64_t)nrows + (uint64_t)row) * (uint64_t)ncols;
-        if (c + PPC <= ncols && ((uintptr_t)(orow + c) & 15u) == 0) {
-          u32x4 vec;
-          if constexpr (PACKED) vec = u32x4{accw[k * 4], accw[k * 4 + 1], accw[k * 4 + 2], accw[k * 4 + 3]};
-          else __builtin_memcpy(&vec, &acc[k * PPC], 16);
-          __builtin_nontemporal_store(vec, (u32x4*)(orow + c));
-        } else {
-#pragma unroll
-          for (int j = 0; j < PPC; ++j)
-            if (c + j < ncols) {
-              if constexpr (PACKED) {
-                T x;
-                __builtin_memcpy(&x, reinterpret_cast<const char*>(accw) + (k * PPC + j) * sizeof(T), sizeof(T));
-                orow[c + j] = x;
-              } else {
-                orow[c + j] = acc[k * PPC + j];
-              }
-            }
-        }
-      }
-    }
   }
   if (a.burns) {
 #pragma unroll
