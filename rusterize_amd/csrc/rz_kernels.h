@@ -330,7 +330,7 @@ struct InitArgs {
 // A window is a run of whole strips by at most (words / 16 - 2) mask words.
 // Masks and list entries are handed out by counters, one atomic of each per
 // workgroup; their order does not matter.
-constexpr int kCoverWave = 448, kCoverBlock = 3840;
+constexpr int kCoverWave = 448, kCoverBlockWaves = 4, kCoverBlock = 3840;
 constexpr int kCoverRun = 16;  // small items a wave takes at once
 constexpr int kCoverBlockNv = 320;
 struct CoverWindows {
@@ -355,7 +355,9 @@ __host__ __device__ inline CoverWindows cover_windows(int32_t ns, int32_t nw, bo
 constexpr int kDescBlock = 512;  // threads of a k_item_desc workgroup
 struct CoverCounters {
   unsigned long long mask_units;  // 16-word units of masks handed out
-  uint32_t n_small, n_wave, n_block, pad[11];
+  uint32_t n_small, n_wave, n_block;
+  uint32_t next;                  // block entries taken beyond one per workgroup
+  uint32_t pad[10];
 };
 struct CoverLists {
   CoverCounters* ctr;   // zero at launch

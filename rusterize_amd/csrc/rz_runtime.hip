@@ -1160,7 +1160,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     // lists' lengths are on the device)
     if (max_poly_nv > kCoverBlockNv) {
       const uint64_t g = read_totals ? std::max<uint64_t>(c->last_units, 1) : 1024;
-      hipLaunchKernelGGL(k_cover<true>, dim3((unsigned)std::min<uint64_t>(g, 1024)), dim3(256), 0, s, ca);
+      hipLaunchKernelGGL(k_cover<true>, dim3((unsigned)std::min<uint64_t>(g, 1024)), dim3(64 * kCoverBlockWaves), 0, s, ca);
     }
     const uint64_t g = ((uint64_t)I + (read_totals ? c->last_units : 0)) / 4 + 1;
     hipLaunchKernelGGL(k_cover<false>, dim3((unsigned)std::min<uint64_t>(g, 1536)), dim3(256), 0, s, ca);
