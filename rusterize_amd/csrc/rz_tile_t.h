@@ -332,11 +332,11 @@ struct LineWriter {
   static constexpr int ROWS = WAVE_ROWS, TW = tile_w(sizeof(T));
   static constexpr int LINE = 128 / (int)sizeof(T);      // pixels of a line
   static constexpr bool NARROW = sizeof(T) <= 2;
-  // the pixels left out: 4- and 8-byte ones in registers (lanes as in
-  // Pixels), 1- and 2-byte ones in LDS, the last LINE pixels of every row
-  T keep[NARROW ? 1 : ROWS];
-  uint32_t* tail;          // [ROWS][(LINE + TW) * sizeof(T) / 4 + 1] words (narrow)
-  static constexpr int PITCH = (LINE + TW) * (int)sizeof(T) / 4 + 1;
+  // the pixels left out, in LDS (registers would cost a wave per SIMD): the
+  // last LINE pixels of every row, PITCH words apart; narrow ones are
+  // followed by room for the row itself
+  uint32_t* tail;
+  static constexpr int PITCH = NARROW ? (LINE + TW) * (int)sizeof(T) / 4 + 1 : 32;
 
   __device__ static uint32_t skew(const T* p) { return ((uint32_t)(uintptr_t)p & 127u) / (uint32_t)sizeof(T); }
 
@@ -354,9 +354,11 @@ struct LineWriter {
         if (u.Rw + r < u.nrows) {
           T* orow = out + (uint64_t)r * (uint64_t)u.ncols;
           const int32_t s = (int32_t)skew(orow + u.C0);
-          // lane l: column C0 - s + l, from lane l - s of this unit or, wrapped,
-          // of the one to the left
-          const T v = lane >= 64 - s ? keep[r] : p.px[r];
+          // lane l: column C0 - s + l, from lane l - s of this unit or from the
+          // last pixels of the one to the left
+          T* last = reinterpret_cast<T*>(tail + r * PITCH);
+          const T left = last[(LINE - s + lane) & (LINE - 1)];
+          const T v = p.px[r];
           const int from = ((lane - s) & 63) * 4;
           T y;
           if constexpr (sizeof(T) == 8) {
@@ -371,10 +373,12 @@ struct LineWriter {
             w = __builtin_amdgcn_ds_bpermute(from, w);
             __builtin_memcpy(&y, &w, 4);
           }
+          if (lane < s) y = left;
           const int32_t c = u.C0 - s + lane;
           if ((cont || lane >= s) && c < u.ncols) __builtin_nontemporal_store(y, orow + c);
           if (!more && lane >= 64 - s && u.C0 + lane < u.ncols) orow[u.C0 + lane] = p.px[r];
-          keep[r] = p.px[r];
+          wave_sync();
+          if (lane >= 64 - LINE) last[lane - (64 - LINE)] = p.px[r];
         }
       }
     } else {
@@ -569,10 +573,14 @@ __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels
   }
 }
 
-// Waves per SIMD the register allocation of k_tile targets.
-template <typename T>
+// Waves per SIMD the register allocation of k_tile targets: 5 where the
+// pixels are 4 or 8 bytes (a million polygons on 40000^2 float32: 5.24 ms a
+// call, with 6 waves 5.31, with the last pixels of LineWriter in registers
+// and 5 waves 5.53; float64 with 5 waves 3.85 ms on 24 uneven jobs, with 4
+// waves 4.04); 4 where that would spill.
+template <typename T, bool BARE>
 struct TileOccupancy {
-  static constexpr int value = sizeof(T) == 4 ? 5 : 4;
+  static constexpr int value = sizeof(T) <= 2 || BARE ? 4 : 5;
 };
 
 // Tile kernel of polygon-only groups, one launch per pixel-function group of
@@ -594,12 +602,12 @@ struct TileOccupancy {
 // BARE: compiled with the path for items without masks (its registers would
 // cost the other calls spills).
 template <typename T, int FUN, bool BARE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupancy<T>::value))) void k_tile(TileArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupancy<T, BARE>::value))) void k_tile(TileArgs a) {
   constexpr int TW = tile_w(sizeof(T));
   constexpr int NWORD = TW / 64;  // mask words per row
   __shared__ PolyEdge s_edge[BARE ? 4 : 1][64];
   __shared__ __align__(16) uint32_t s_x[4][NWORD > 1 ? 256 : 1];
-  __shared__ uint32_t s_tail[4][NWORD > 1 ? WAVE_ROWS * LineWriter<T>::PITCH : 1];
+  __shared__ __align__(16) uint32_t s_tail[4][WAVE_ROWS * LineWriter<T>::PITCH];
 
   const int wave = wave_index(), lane = threadIdx.x & 63;
   uint32_t burns = 0;
