@@ -351,8 +351,8 @@ rz_status rz_batch_graph_destroy(rz_batch_graph* graph);
 /* ------------------------------------------------------------- autotuner -- */
 
 /* No reference counterpart: per size class (tile width, tiles of a launch,
- * items per tile) the tiles a work-queue grab takes and the item count from
- * which a tile's polygon coverage is precomputed in parallel.  rz_autotune
+ * items per tile) the tiles a work-queue grab takes (heavy_min is kept as it
+ * is set and has no effect: all polygon coverage is precomputed).  rz_autotune
  * times every candidate on each job (reps timed runs each) and stores the
  * fastest for that job's class in a process-wide table that every later call
  * and batch uses; run it while no other rasterisation runs in the process.

@@ -539,12 +539,13 @@ namespace {
 // ---- autotuned launch knobs
 //
 // Per size class (tile width, launch tiles, items per tile) the autotuner
-// (rz_autotune) stores the tiles per queue grab and the item count from which
-// a tile's coverage is precomputed by the k_cover pre-pass.  Classes without
-// an entry use the defaults below.
+// (rz_autotune) stores the tiles per queue grab.  heavy_min, an item count
+// from which a tile's coverage was computed beforehand, changes nothing any
+// more (all coverage is) and is kept as the table has it.  Classes without an
+// entry use the defaults below.
 struct Tuning {
   uint32_t chunk = 0;      // 0: default
-  uint32_t heavy_min = 0;  // 0: default (kHeavyItems)
+  uint32_t heavy_min = 0;
 };
 
 struct TuneState {
@@ -1298,7 +1299,7 @@ extern "C" rz_status rz_autotune(rz_context* c, const rz_job* jobs, int64_t n_jo
   if (!c || (!jobs && n_jobs > 0) || reps < 1) return rz::fail(RZ_VALUE_ERROR, "bad argument to rz_autotune");
   HIP_TRY(hipSetDevice(c->device));
   static const uint32_t kChunks[] = {1, 2, 4, 8};
-  static const uint32_t kHeavy[] = {16, 32, 64, 1u << 30};
+  const uint32_t kHeavy = 32;  // (stored for the table's readers)
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
@@ -1309,28 +1310,27 @@ extern "C" rz_status rz_autotune(rz_context* c, const rz_job* jobs, int64_t n_jo
     Tuning best;
     float best_ms = 1e30f;
     uint32_t cls = 0;
-    for (uint32_t ch : kChunks)
-      for (uint32_t hv : kHeavy) {
-        {
-          std::lock_guard<std::mutex> lk(ts.mu);
-          ts.force = true;
-          ts.forced = Tuning{ch, hv};
-        }
-        st = run_batch(c, jobs + k, 1);  // warm-up (workspace)
-        if (st == RZ_OK) st = rz_context_synchronize(c);
-        float ms = 0.f;
-        if (st == RZ_OK && hipEventRecord(e0, c->stream) != hipSuccess) st = RZ_DEVICE_ERROR;
-        for (int r = 0; r < reps && st == RZ_OK; ++r) st = run_batch(c, jobs + k, 1);
-        if (st == RZ_OK && (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                            hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
-          st = rz::fail(RZ_DEVICE_ERROR, "autotune timing failed");
-        if (st) break;
-        if (ms < best_ms) {
-          best_ms = ms;
-          best = Tuning{ch, hv};
-        }
-        cls = size_class(tile_w((int)rz_dtype_size(jobs[k].dtype)), c->last_tiles, c->last_pairs);
+    for (uint32_t ch : kChunks) {
+      {
+        std::lock_guard<std::mutex> lk(ts.mu);
+        ts.force = true;
+        ts.forced = Tuning{ch, kHeavy};
       }
+      st = run_batch(c, jobs + k, 1);  // warm-up (workspace)
+      if (st == RZ_OK) st = rz_context_synchronize(c);
+      float ms = 0.f;
+      if (st == RZ_OK && hipEventRecord(e0, c->stream) != hipSuccess) st = RZ_DEVICE_ERROR;
+      for (int r = 0; r < reps && st == RZ_OK; ++r) st = run_batch(c, jobs + k, 1);
+      if (st == RZ_OK && (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+                          hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+        st = rz::fail(RZ_DEVICE_ERROR, "autotune timing failed");
+      if (st) break;
+      if (ms < best_ms) {
+        best_ms = ms;
+        best = Tuning{ch, kHeavy};
+      }
+      cls = size_class(tile_w((int)rz_dtype_size(jobs[k].dtype)), c->last_tiles, c->last_pairs);
+    }
     if (st == RZ_OK) {
       std::lock_guard<std::mutex> lk(ts.mu);
       if (!ts.table.count(cls)) ++tuned;

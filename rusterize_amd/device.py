@@ -288,7 +288,7 @@ def autotune(ctx: Context, jobs: list[Job], reps: int = 2) -> int:
 
 
 def autotune_table() -> dict:
-    """The process-wide table: size class -> (tiles per grab, heavy-tile items)."""
+    """The process-wide table: size class -> (tiles per grab, heavy-tile items: kept, without effect)."""
     L = _lib.lib()
     n = L.rz_autotune_table(None, None, None, 0)
     cls, ch, hv = (c_uint32 * max(n, 1))(), (c_uint32 * max(n, 1))(), (c_uint32 * max(n, 1))()
