@@ -500,9 +500,10 @@ __device__ inline Visits visits_of(const RawItem& q, const StripUnit& u, bool ca
   return v;
 }
 
-// Visits whose mask blocks are loaded ahead of their folds.
+// Visits whose mask blocks are loaded ahead of their folds (more cost waves;
+// 4-byte pixels with 1 and 7 waves: 5.34 ms where 2 take 5.17).
 template <typename T>
-constexpr int kAhead = sizeof(T) == 8 ? 3 : (sizeof(T) <= 2 ? 2 : 6);
+constexpr int kAhead = sizeof(T) == 8 ? 3 : 2;
 
 // The column bits (16 rows) of visits k .. k + N - 1 (past the last one: the
 // last one's again).
@@ -573,14 +574,14 @@ __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels
   }
 }
 
-// Waves per SIMD the register allocation of k_tile targets: 5 where the
-// pixels are 4 or 8 bytes (a million polygons on 40000^2 float32: 5.24 ms a
-// call, with 6 waves 5.31, with the last pixels of LineWriter in registers
-// and 5 waves 5.53; float64 with 5 waves 3.85 ms on 24 uneven jobs, with 4
-// waves 4.04); 4 where that would spill.
+// Waves per SIMD the register allocation of k_tile targets: 7 for 4-byte
+// pixels (a million polygons on 40000^2 float32 in 2 bands: 5.17 ms a call,
+// in 8 bands, about one item to a tile, 12.1; with 5 waves and 6 visits ahead
+// 5.24 and 14.3), 5 for 8-byte ones (24 uneven jobs 3.85 ms, with 4 waves
+// 4.04); 4 where more would spill.
 template <typename T, bool BARE>
 struct TileOccupancy {
-  static constexpr int value = sizeof(T) <= 2 || BARE ? 4 : 5;
+  static constexpr int value = sizeof(T) <= 2 || BARE ? 4 : (sizeof(T) == 4 ? 7 : 5);
 };
 
 // Tile kernel of polygon-only groups, one launch per pixel-function group of
