@@ -716,10 +716,14 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     if (std::strcmp(bm, "always") == 0) binning = 1;
     else if (std::strcmp(bm, "never") == 0) binning = -1;
   }
-  // RUSTERIZE_WIDE=never: no polygon item gets coverage masks, the tile
-  // kernels compute them strip by strip (tests run both on the same inputs).
-  bool use_masks = true;
-  if (const char* wm = std::getenv("RUSTERIZE_WIDE")) use_masks = masks_only || std::strcmp(wm, "never") != 0;
+  // RUSTERIZE_WIDE=never|always: no polygon item gets coverage masks, the tile
+  // kernels compute them strip by strip; or every one does, also in calls too
+  // small for them (tests run both on the same inputs).
+  bool use_masks = true, force_masks = masks_only;
+  if (const char* wm = std::getenv("RUSTERIZE_WIDE")) {
+    use_masks = masks_only || std::strcmp(wm, "never") != 0;
+    force_masks |= std::strcmp(wm, "always") == 0;
+  }
   // (all-touched jobs walk their polygons' outlines too: the lines kernel)
   auto has_lines = [](const rz_job& j) { return j.geometry->has_line || j.geometry->has_point || j.all_touched; };
   std::vector<int64_t> order((size_t)n_in);
@@ -813,7 +817,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   // round trip, and a captured batch its own; should items pass those, the
   // tile kernel computes their coverage from edge records, which are written
   // in these cases only.
-  const bool bare = !masks_only && T <= kBlockTiles && n_poly <= kBareItems && poly_nv <= kBareVerts;
+  const bool bare = !force_masks && T <= kBlockTiles && n_poly <= kBareItems && poly_nv <= kBareVerts;
   const bool any_mask = any_poly && use_masks && !bare && I > 0;
   const bool read_totals = !capture && (any_binned || any_band || masks_only);
   const uint64_t mask_fixed = capture ? caps->masks : std::min<uint64_t>(mask_bound, (uint64_t)I * 64 + out_px / 64);

@@ -12,7 +12,8 @@ import pytest
 from oracle import oracle
 from rusterize_amd import _lib
 from rusterize_amd._lib import Geometry
-from tests.test_gpu_parity import assert_same, field_for
+from rusterize_amd.device import BatchGraph, Context, DeviceBuffer, DeviceGeometry, Job, grid, rasterize_device
+from tests.test_gpu_parity import assert_same, degenerate_geometry, field_for, polygon_rings
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +53,150 @@ def test_coverage_sizes(rows, cols, n_layers, dtype, binning, monkeypatch):
         ref = oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, layer_of_geom=layers,
                                n_layers=n_layers, background=bg)
         assert_same(got, ref, f"{rows}x{cols}x{n_layers} {dtype} {fun} {binning}")
+
+
+def test_forced_masks_in_a_small_call(monkeypatch):
+    # 10 polygons get no masks by themselves; RUSTERIZE_WIDE=always gives them
+    # theirs (a context that never made a mask has no buffers for them), with
+    # the same raster
+    g = degenerate_geometry()
+    field = field_for("float64", g.n_geoms, seed=3)
+    info = grid(300, 200)
+    ref = oracle.rasterize(g, oracle.copy_info(info), "float64", "sum", field=field, background=float("nan"))
+    held = {}
+    for wide in ("never", "always"):
+        monkeypatch.setenv("RUSTERIZE_WIDE", wide)
+        with Context(0) as ctx:
+            dg, out = DeviceGeometry(ctx, g), DeviceBuffer(ctx, 200 * 300 * 8)
+            d_field = DeviceBuffer.from_array(ctx, field)
+            job = Job(dg, info, "float64", "sum", out, field=d_field, background=float("nan"))
+            rasterize_device(ctx, job)
+            ctx.synchronize()
+            assert_same(job.result(), ref, f"wide {wide}")
+            held[wide] = ctx.workspace_bytes()
+            out.free()
+            d_field.free()
+            dg.free()
+    assert held["always"] > held["never"]
+
+
+def degenerate_rings(long):
+    """The degenerate rings among 520 ordinary ones (so that the call takes
+    masks); long: also rings of 400 vertices with one NaN, infinite or huge
+    vertex each, and one left open."""
+    rng = np.random.default_rng(5)
+    d = degenerate_geometry()
+    rings = [[d.xy[d.ring_vertex_offsets[r]:d.ring_vertex_offsets[r + 1]]
+              for r in range(d.item_ring_offsets[i], d.item_ring_offsets[i + 1])] for i in range(d.n_geoms)]
+    for k in range(520):
+        p = rng.uniform(0, 300, (4, 2))
+        rings.insert(int(rng.integers(0, len(rings))), [np.concatenate([p, p[:1]])])
+    bad = [(np.nan, 90.0), (-np.nan, 60.0), (np.inf, 100.0), (-np.inf, 50.0), (1e300, 120.0), (120.0, np.nan),
+           (150.0, -1e300), None]
+    for k, v in enumerate(bad if long else []):
+        a = np.linspace(0, 2 * np.pi, 401)
+        p = np.stack([150 + (40 + 9 * k) * np.cos(a), 100 + (30 + 8 * k) * np.sin(a)], 1)
+        p[400] = p[0]
+        if v is None:
+            p = p[:-3]
+        else:
+            p[97 + 30 * k] = v
+        rings.insert(60 * k, [p])
+    return polygon_rings(rings)
+
+
+@pytest.mark.parametrize("binning,long", [("never", False), ("never", True), ("always", False), ("always", True)])
+def test_degenerate_rings_in_masks(binning, long, monkeypatch):
+    monkeypatch.setenv("RUSTERIZE_BINNING", binning)
+    g = degenerate_rings(long)
+    info = grid(300, 200)
+    for dtype, fun, bg in (("float64", "sum", float("nan")), ("uint8", "count", 0), ("int32", "last", 0)):
+        field = field_for(dtype, g.n_geoms, seed=7)
+        got = _lib.rasterize(g, info, dtype, fun, field, None, None, 1, bg)
+        ref = oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, background=bg)
+        assert_same(got, ref, f"degenerate {dtype} {fun}")
+
+
+def quads(n, size, long=False):
+    """n quadrilaterals over most of size x size pixels; long: the first has
+    400 vertices."""
+    rng = np.random.default_rng(n + size)
+    lo, hi = rng.uniform(-20, 0.08 * size, (n, 2)), rng.uniform(0.92 * size, size + 20, (n, 2))
+    rings = []
+    for k, ((x0, y0), (x1, y1)) in enumerate(zip(lo, hi)):
+        p = np.array([(x0, y0), (x1, y0 + 7), (x1, y1), (x0 + 5, y1), (x0, y0)])
+        if long and k == 0:
+            p = np.concatenate([np.linspace(p[0], p[1], 397)[:-1], p[1:]])
+        rings.append([p])
+    return polygon_rings(rings)
+
+
+@pytest.mark.parametrize("long", [False, True])
+@pytest.mark.parametrize("dtype,fun,bg", [("float64", "sum", float("nan")), ("uint8", "count", 0),
+                                          ("int16", "last", 0), ("int32", "max", 0)])
+def test_masks_past_their_capacity(dtype, fun, bg, long, monkeypatch):
+    # 600 items of about 240 mask blocks (128 bytes, 16 x 64 pixels each) on
+    # 512 x 512 pixels: 148,000 blocks, where a scanned call holds at most
+    # 2 bytes per pixel and 8 KiB per item: 42,496.  The items past that
+    # compute their coverage from their edges, next to those with masks.
+    monkeypatch.setenv("RUSTERIZE_BINNING", "never")
+    g = quads(600, 512, long)
+    field = field_for(dtype, g.n_geoms, seed=21)
+    info = grid(512, 512)
+    got = _lib.rasterize(g, info, dtype, fun, field, None, None, 1, bg)
+    ref = oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, background=bg)
+    assert_same(got, ref, f"past the mask capacity {dtype} {fun} {long}")
+
+
+@pytest.mark.parametrize("binning,long,lines", [("never", False, 0), ("always", False, 0), ("always", True, 0),
+                                                ("always", True, 60)])
+def test_graph_replay_past_the_mask_capacity(binning, long, lines, monkeypatch):
+    # 600 polygons captured while they are 16 x 16 pixels (2 mask blocks each)
+    # and replayed grown to 62 x 62 in the same tiles (4 each): binned, the
+    # capacity is the captured need + 64 = 1,264 of 2,400; scanned it is 64 per
+    # item and more, so those grow to the whole raster.  60 lines of 79
+    # segments beside them outgrow their bands in the same replay (4 entries
+    # each where 2 were captured, with room for 64 more).
+    monkeypatch.setenv("RUSTERIZE_BINNING", binning)
+    rng = np.random.default_rng(8)
+    centre = np.repeat(rng.uniform([32, 32], [96, 480], (600, 2)), 5, 0) // 64 * 64 + 32
+    unit = np.tile([(-1, -1), (1, -0.9), (1, 1), (-0.9, 1), (-1, -1)], (600, 1))
+    if long:  # the first ring has 400 vertices
+        first = np.concatenate([np.linspace(unit[0], unit[1], 397)[:-1], unit[1:5]])
+        unit, centre = np.concatenate([first, unit[5:]]), np.concatenate([centre[:1].repeat(400, 0), centre[5:]])
+    nv = np.array([400 if long and k == 0 else 5 for k in range(600)] + [80] * lines)
+    n = len(nv)
+    kind = np.array([0] * 600 + [1] * lines, np.int32)
+
+    def shape(half, tall):
+        xy = [centre + half * unit]
+        for k in range(lines):
+            t = np.linspace(0, 1, 80)
+            xy.append(np.stack([8 + 8 * k + 3 * np.sin(40 * t), 256.5 + tall * (t - 0.5)], 1))
+        return Geometry(np.arange(n + 1), kind, np.arange(n + 1), np.concatenate([[0], np.cumsum(nv)]),
+                        np.concatenate(xy))
+
+    small, grown = shape(8.0, 12.0), shape(31.0 if binning == "always" else 1000.0, 62.0)
+    info = grid(512, 512)
+    field = field_for("float64", n, seed=5)
+    with Context(0) as ctx:
+        dg, out = DeviceGeometry(ctx, small), DeviceBuffer(ctx, 512 * 512 * 8)
+        d_field = DeviceBuffer.from_array(ctx, field)
+        job = Job(dg, info, "float64", "sum", out, field=d_field, background=float("nan"))
+        graph = BatchGraph([job])
+        try:
+            for geom in (small, grown, grown, small):
+                dg.set_xy(geom.xy)
+                graph.launch()
+                graph.synchronize()
+                ref = oracle.rasterize(geom, oracle.copy_info(info), "float64", "sum", field=field,
+                                       background=float("nan"))
+                assert_same(job.result(), ref, "replay")
+                rasterize_device(ctx, job)
+                ctx.synchronize()
+                assert_same(job.result(), ref, "eager between replays")
+        finally:
+            graph.close()
+            out.free()
+            d_field.free()
+            dg.free()
