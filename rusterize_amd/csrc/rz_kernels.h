@@ -352,6 +352,17 @@ __host__ __device__ inline CoverWindows cover_windows(int32_t ns, int32_t nw, bo
   c.n = c.ncw * ((ns + c.strips - 1) / c.strips);
   return c;
 }
+// The LDS words of a unit whose raster row R0 is at word `first`: those of row
+// r start at cover_word(cover_origin(first, R0, stride), r, stride).  Unsigned,
+// since the products pass 2^31 on rasters of some million rows (a signed
+// overflow would not be a constant below).
+__host__ __device__ constexpr uint32_t cover_origin(uint32_t first, int32_t R0, int32_t stride) {
+  return first - (uint32_t)R0 * (uint32_t)stride;
+}
+__host__ __device__ constexpr uint32_t cover_word(uint32_t A, int32_t r, int32_t stride) {
+  return A + (uint32_t)r * (uint32_t)stride;
+}
+static_assert(cover_word(cover_origin(7u, 9000000, 239), 9000015, 239) == 7u + 15u * 239u, "rows past 2^31 words");
 constexpr int kDescBlock = 512;  // threads of a k_item_desc workgroup
 struct CoverCounters {
   unsigned long long mask_units;  // 16-word units of masks handed out

@@ -35,7 +35,8 @@ __device__ inline uint64_t transpose16(uint64_t x, int lane) {
 
 // An item (or a window of one) whose toggle words are in LDS.
 struct __align__(16) CoverItem {
-  int32_t A, stride;  // the words of raster row r start at A + r * stride
+  uint32_t A;         // the words of raster row r start at cover_word(A, r, stride)
+  int32_t stride;
   int32_t W0, wid;    // first column and columns
   int32_t R0, R1;     // raster rows [R0, R1)
   int64_t lv;         // edge e of the unit starts at local vertex lv + e
@@ -106,7 +107,7 @@ struct CoverWave {
       const double x = x0 + (((double)r + 0.5) - y0) * dxdy;
       const int32_t col = span_col(x, ncols_f);
       const int32_t rel = max(col - W0, 0);
-      uint64_t* row = tog + (it->A + r * it->stride);
+      uint64_t* row = tog + cover_word(it->A, r, it->stride);
       if (rel < wid)
         __hip_atomic_fetch_xor(row + (rel >> 6), 1ull << (rel & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       // the rightmost crossing of a row matters only with an odd count
@@ -242,7 +243,7 @@ struct CoverWave {
       if (own) {
         CoverItem x = it;
         x.base = base + wi - words;
-        x.A = (int32_t)x.base - x.R0 * x.stride;
+        x.A = cover_origin(x.base, x.R0, x.stride);
         x.R1 = min(x.R1, J.nrows);
         x.lv -= J.v_base + (int64_t)(ei - nv);
         x.row0 = ri - rows;
@@ -278,7 +279,7 @@ struct CoverWave {
     const int32_t first = BLOCK ? 0 : (int32_t)base, R0 = ((r0 >> 4) + s0) * 16, W0 = ((c0 >> 6) + w0) * 64;
     if (lane == 0) {
       CoverItem it{};
-      it.A = first - R0 * win.stride;
+      it.A = cover_origin((uint32_t)first, R0, win.stride);
       it.stride = win.stride;
       it.W0 = W0;
       it.wid = ww * 64;
