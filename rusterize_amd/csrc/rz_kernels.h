@@ -49,6 +49,10 @@ constexpr uint32_t kBlockTiles = 12288;
 // only where all of them meet the same few tiles are masks ahead, 25 against
 // 33 for 32 stars on 100 x 200).
 constexpr int64_t kBareItems = 512, kBareVerts = 4096;
+// Pixels up to which a call reserves masks without knowing what it needs
+// (reading the need back takes about 10 us, and a call of more pixels at
+// least 100 for its stores alone).
+constexpr uint64_t kMaskBlindPx = (uint64_t)1 << 26;
 constexpr int TILE_H = 64;       // rows per tile (4 waves x 16 rows)
 constexpr int WAVE_ROWS = 16;    // rows per wave strip
 constexpr int NUM_XCD = 8;       // MI355X: 8 XCDs, workgroups dispatched round-robin

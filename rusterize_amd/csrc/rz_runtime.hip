@@ -811,17 +811,20 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   HIP_TRY(ensure(c->stream, c->queue, queue_words * 4));
   uint32_t* d_status = (uint32_t*)c->misc.p;
   unsigned long long* d_burns = (unsigned long long*)((char*)c->misc.p + 64);
-  // Coverage masks.  An eager call that reads its totals back anyway (bins,
-  // line bands, the sparse encoding) sizes them exactly.  One that does not
-  // takes a capacity of 8 KiB per item and 2 bytes per pixel, with no host
-  // round trip, and a captured batch its own; should items pass those, the
-  // tile kernel computes their coverage from edge records, which are written
-  // in these cases only.
+  // Coverage masks.  They hold at most 8 KiB per item and 2 bytes per pixel
+  // (and, of binned items, the tiles of their pairs): as many small items or
+  // 16 deep layers of large ones.  An eager call that reads its totals back
+  // anyway (bins, line bands, the sparse encoding) sizes them exactly; one
+  // that does not takes that capacity unseen, with no host round trip, up to
+  // kMaskBlindPx pixels (128 MiB), and reads its totals past them; a captured
+  // batch has its own capacity.  Of the items that pass it the tile kernel
+  // computes the coverage from edge records, written in these cases only.
   const bool bare = !force_masks && T <= kBlockTiles && n_poly <= kBareItems && poly_nv <= kBareVerts;
   const bool any_mask = any_poly && use_masks && !bare && I > 0;
-  const bool read_totals = !capture && (any_binned || any_band || masks_only);
-  const uint64_t mask_fixed = capture ? caps->masks : std::min<uint64_t>(mask_bound, (uint64_t)I * 64 + out_px / 64);
-  const bool need_edges = any_poly && (!any_mask || (!read_totals && (capture || mask_bound > mask_fixed)));
+  const bool read_totals = !capture && (any_binned || any_band || masks_only || (any_mask && out_px > kMaskBlindPx));
+  const uint64_t mask_limit = (uint64_t)I * 64 + out_px / 64;
+  const uint64_t mask_fixed = capture ? caps->masks : std::min<uint64_t>(mask_bound, mask_limit);
+  bool need_edges = any_poly && (!any_mask || (!read_totals && (capture || mask_bound > mask_fixed)));
   if (need_edges) HIP_TRY(ensure(c->stream, c->edges, (size_t)std::max<int64_t>(V, 1) * sizeof(PolyEdge)));
   CoverLists cover{};
   // (windows hold 13 mask units or more on average, but for their items' last)
@@ -913,8 +916,8 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     const uint64_t nz = std::max<uint64_t>((uint64_t)I, ia.words());
     hipLaunchKernelGGL(k_init, dim3(blocks_for((int64_t)nz)), dim3(256), 0, s, ia);
   }
+  PrepArgs pa{};
   if (V > 0 && !fused) {
-    PrepArgs pa{};
     pa.jobs = d_jobs;
     pa.job_vend = d_vend;
     pa.n_jobs = (int)n;
@@ -1024,14 +1027,25 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     if (read_totals) {
       CoverCounters cc{};
       std::memcpy(&cc, &c->host_misc[4], 24);
-      mask_units = cc.mask_units;
-      c->last_masks = mask_units;
       c->last_units = std::max(cc.n_wave, cc.n_block);
-      if (mask_units > UINT32_MAX) return rz::fail(RZ_CAPACITY_ERROR, "more than 512 GiB of coverage masks in one call");
-      if (c->last_units > unit_cap) {
-        // windows past the lists: lists of the right size, assigned again
-        unit_cap = c->last_units;
+      if (masks_only && cc.mask_units > UINT32_MAX)
+        return rz::fail(RZ_CAPACITY_ERROR, "more than 512 GiB of coverage masks in one call");
+      const uint64_t of_pairs = any_binned ? c->host_misc[0] * 4u * (uint64_t)(max_tile_w / 64) : 0u;
+      const uint64_t limit = masks_only ? UINT32_MAX : std::min<uint64_t>(mask_limit + of_pairs, UINT32_MAX);
+      mask_units = std::min<uint64_t>(cc.mask_units, limit);
+      c->last_masks = mask_units;
+      if (c->last_units > unit_cap || cc.mask_units > limit) {
+        // windows past the lists, or items past the limit: lists of the right
+        // size and edge records, and the masks assigned again
+        unit_cap = std::max(unit_cap, c->last_units);
         if (rz_status st = place_cover()) return st;
+        if (cc.mask_units > limit) {
+          cover.mask_cap = limit;
+          need_edges = true;
+          HIP_TRY(ensure(c->stream, c->edges, (size_t)std::max<int64_t>(V, 1) * sizeof(PolyEdge)));
+          pa.edges = (PolyEdge*)c->edges.p;  // (the same boxes once more)
+          hipLaunchKernelGGL(k_prep, dim3(blocks_for(V)), dim3(256), 0, s, pa);
+        }
         zero_words(c->cover.p, sizeof(CoverCounters) / 4, s);
         da.cover = cover;
         hipLaunchKernelGGL(k_item_desc, dim3(blocks_for(I, kDescBlock)), dim3(kDescBlock), 0, s, da);

@@ -12,7 +12,8 @@ import pytest
 from oracle import oracle
 from rusterize_amd import _lib
 from rusterize_amd._lib import Geometry
-from rusterize_amd.device import BatchGraph, Context, DeviceBuffer, DeviceGeometry, Job, grid, rasterize_device
+from rusterize_amd.device import BatchGraph, Context, DeviceBuffer, DeviceGeometry, Job, batch_rasterize, grid, \
+    rasterize_device
 from tests.test_gpu_parity import assert_same, degenerate_geometry, field_for, polygon_rings
 
 pytestmark = pytest.mark.gpu
@@ -200,3 +201,56 @@ def test_graph_replay_past_the_mask_capacity(binning, long, lines, monkeypatch):
             out.free()
             d_field.free()
             dg.free()
+
+
+def test_masks_of_a_large_raster_take_what_they_need(monkeypatch):
+    # 600 quadrilaterals of 20 pixels on 8200 x 8200 (more pixels than masks are
+    # reserved for unseen): at most 4 blocks of 128 bytes each, beside 2 bytes
+    # per pixel (134 MB) if they were reserved by the raster's size
+    monkeypatch.setenv("RUSTERIZE_BINNING", "never")
+    n = 8200
+    rng = np.random.default_rng(4)
+    c = np.repeat(rng.uniform(40, n - 40, (600, 1, 2)), 5, 1)
+    g = polygon_rings([[p] for p in c + 10 * np.array([(-1, -1), (1, -0.8), (1, 1), (-0.9, 1), (-1, -1)])])
+    field = field_for("uint8", 600, seed=2)
+    info = grid(n, n)
+    with Context(0) as ctx:
+        dg, out, d_field = DeviceGeometry(ctx, g), DeviceBuffer(ctx, n * n), DeviceBuffer.from_array(ctx, field)
+        job = Job(dg, info, "uint8", "max", out, field=d_field)
+        rasterize_device(ctx, job)
+        ctx.synchronize()
+        ref = oracle.rasterize(g, oracle.copy_info(info), "uint8", "max", field=field, background=0)
+        assert_same(job.result(), ref, "600 small polygons on a large raster")
+        assert ctx.workspace_bytes() < 16 << 20
+        for b in (out, d_field, dg):
+            b.free()
+
+
+def test_masks_past_their_limit_when_the_need_is_known(monkeypatch):
+    # the 600 quadrilaterals of test_masks_past_their_capacity in a batch whose
+    # line bands make it read its totals: 148,000 blocks (19 MB) needed, of
+    # which 42,000 and some (5.5 MB) are given
+    monkeypatch.setenv("RUSTERIZE_BINNING", "never")
+    t = np.linspace(0, 1, 80)
+    lines = [np.stack([10 + 100 * t, 20 + 90 * t + 5 * np.sin(9 * t + k)], 1) for k in range(3)]
+    sets = [quads(600, 512), Geometry(np.arange(4), np.ones(3, np.int32), np.arange(4), np.arange(4) * 80,
+                                      np.concatenate(lines))]
+    with Context(0) as ctx:
+        jobs, refs, held = [], [], []
+        for g, side, fun in zip(sets, (512, 128), ("sum", "count")):
+            field = field_for("float64", g.n_geoms, seed=side)
+            info = grid(side, side)
+            dg, d_field = DeviceGeometry(ctx, g), DeviceBuffer.from_array(ctx, field)
+            out = DeviceBuffer(ctx, side * side * 8)
+            held += [dg, d_field, out]
+            jobs.append(Job(dg, info, "float64", fun, out, field=d_field, background=float("nan")))
+            refs.append(oracle.rasterize(g, oracle.copy_info(info), "float64", fun, field=field,
+                                         background=float("nan")))
+        for _ in range(2):
+            batch_rasterize(ctx, jobs)
+            ctx.synchronize()
+            for job, ref in zip(jobs, refs):
+                assert_same(job.result(), ref, job.fun)
+        assert ctx.workspace_bytes() < 12 << 20
+        for b in held:
+            b.free()
