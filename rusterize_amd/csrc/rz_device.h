@@ -344,6 +344,57 @@ __device__ inline uint32_t wave_prefix_sum(uint32_t x) {
   return x;
 }
 
+// Minimum over the wave, in its last lane (as wave_prefix_sum).
+__device__ inline int32_t wave_min_last(int32_t x) {
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x111, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x112, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x114, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x118, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x142, 0xA, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x143, 0xC, 0xF, false));
+  return x;
+}
+
+// The chunks of 64 vertices of an item's rings whose edges may meet rows
+// [R0, R1), in order, those of numbers with a bit in `mine` (of number % 64):
+// `rows` holds the row range of each (null: all chunks are taken), 64 of which
+// are tested at a time while the next 64 are loading.  A long ring is mostly
+// local, so a window or strip reads about the edges it needs where it would
+// read all of them (see k_cover and strip_coverage).  Every lane of the wave
+// calls next().
+struct Chunks {
+  const int2* rows;
+  uint32_t n, sb;         // chunks; those of [sb, sb + 64) with a bit in m are still to come
+  int32_t R0, R1;
+  uint64_t mine, m;
+  int2 ahead;
+  int lane;
+
+  __device__ Chunks(const int2* rows_, uint32_t n_, int32_t R0_, int32_t R1_, uint64_t mine_, int lane_)
+      : rows(rows_), n(n_), sb(0), R0(R0_), R1(R1_), mine(mine_), ahead(make_int2(0, 0)), lane(lane_) {
+    if (rows && (uint32_t)lane < n) ahead = rows[lane];
+    test();
+  }
+  __device__ void test() {
+    const uint32_t left = n - sb;
+    m = left < 64u ? mine & ((1ull << left) - 1ull) : mine;
+    if (rows) {
+      m &= __ballot(ahead.x < R1 && ahead.y > R0);
+      if (left > 64u && (uint32_t)lane < left - 64u) ahead = rows[sb + 64u + (uint32_t)lane];
+    }
+  }
+  __device__ bool next(uint32_t& c) {
+    while (!m) {
+      if (n - sb <= 64u) return false;
+      sb += 64u;
+      test();
+    }
+    c = sb + (uint32_t)__builtin_ctzll(m);
+    m &= m - 1ull;
+    return true;
+  }
+};
+
 // One 64-byte descriptor from a read-only table (four 16-byte loads).
 __device__ inline ItemDesc load_desc(const RZ_CONST ItemDesc* p) {
   const RZ_CONST u32x4* q = (const RZ_CONST u32x4*)p;
@@ -378,9 +429,10 @@ __device__ inline uint32_t xcd_unit_lo(uint32_t x, uint32_t n) {
 // 4th active edge; their crossing toggles are XOR-combined with DPP and the
 // row mask follows from the note above row_coverage_word in rz_kernels.h.
 // `stage` is 64 edges of wave-private LDS.
+// (the item's edges are edges[vbeg .. vbeg + n_e); chunk_rows: see Chunks)
 template <int NWORD>
-__device__ inline uint64_t strip_coverage(const PolyEdge* ebase, uint32_t n_e, int32_t Rw,
-                                          int32_t strip_r1, int32_t C0, double ncols_f,
+__device__ inline uint64_t strip_coverage(const PolyEdge* edges, int64_t vbeg, uint32_t n_e, const int2* chunk_rows,
+                                          int32_t Rw, int32_t strip_r1, int32_t C0, double ncols_f,
                                           PolyEdge* stage, int lane) {
   const int rl = lane >> 2, q = lane & 3;
   const int32_t r = Rw + rl;
@@ -390,10 +442,16 @@ __device__ inline uint64_t strip_coverage(const PolyEdge* ebase, uint32_t n_e, i
   for (int w = 0; w < NWORD; ++w) tog[w] = 0ull;
   uint32_t lp = 0;
   int32_t amax = -1;
-  for (uint32_t cb = 0; cb < n_e; cb += 64) {
+  // (chunks start at multiples of 64 vertices of the batch)
+  const bool local = chunk_rows && n_e > (uint32_t)kChunkNv;
+  const uint32_t skew = local ? (uint32_t)vbeg & 63u : 0u;
+  const PolyEdge* ebase = edges + vbeg;
+  Chunks chunks(local ? chunk_rows + (vbeg >> 6) : nullptr, (n_e + skew + 63u) >> 6, Rw, strip_r1, ~0ull, lane);
+  uint32_t c;
+  while (chunks.next(c)) {
     // stage the edges of this chunk that reach the strip, compacted
     // (two 16-byte vector loads and stores: no struct copy through scratch)
-    const uint32_t e = cb + (uint32_t)lane;
+    const uint32_t e = c * 64u + (uint32_t)lane - skew;  // (those before the item wrap)
     uint4 e_lo = make_uint4(0u, 0u, 0u, 0u), e_hi = make_uint4(0u, 0u, 0u, 0u);
     bool act = false;
     if (e < n_e) {

@@ -171,6 +171,8 @@ struct PrepArgs {
   int n_jobs;
   int64_t n_vertices;       // batch total
   PolyEdge* edges;          // [n_vertices], or null: every polygon has masks (k_cover reads xy)
+  int2* chunk_rows;         // [ceil(n_vertices / 64)] rows [x, y) that the items of each 64 vertices
+                            // meet (see Chunks), or null
   uint4* lseg;              // [n_vertices] segment / cell records of line and point vertices
   ItemBox* item_box;        // [n_items]
   unsigned long long* item_last;  // [n_items] lines: last kept segment + 1 (global; 0: none)
@@ -337,6 +339,9 @@ struct InitArgs {
 constexpr int kCoverWave = 448, kCoverBlockWaves = 4, kCoverBlock = 3840;
 constexpr int kCoverRun = 16;  // small items a wave takes at once
 constexpr int kCoverBlockNv = 320;
+// Rings of more vertices than this are read by way of the row ranges of their
+// chunks of 64 vertices (see Chunks).  A ring of two chunks is read whole.
+constexpr int kChunkNv = 128;
 struct CoverWindows {
   int32_t ww, stride, strips;  // mask words, padded words and strips of a window
   int32_t ncw, n;              // windows across, windows in all
@@ -432,6 +437,7 @@ struct CoverArgs {
   const ItemDesc* desc;  // [n_items], masks and lists assigned
   CoverLists cover;
   uint64_t* masks;
+  const int2* chunk_rows;  // (see PrepArgs)
 };
 
 // Per-item edge-band build: one wave per item (grid-stride), counters of
@@ -499,6 +505,7 @@ struct TileArgs {
   // scan jobs: every item of the job is tested against the tile
   const ItemDesc* desc;
   const PolyEdge* edges;    // read for polygon items without masks only
+  const int2* chunk_rows;   // (see PrepArgs; null: none)
   const uint4* lseg;        // line / point vertex records (kLs*)
   // all-touched polygons with sum / count: outline boxes (PixelCache
   // windows) and, for those whose fill reaches beyond them, the PixelCache

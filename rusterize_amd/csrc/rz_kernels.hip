@@ -301,6 +301,10 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   } else if (active) {
     vertex(as_const(a.jobs)[find_job(a.job_vend, a.n_jobs, v)]);
   }
+  if (a.chunk_rows) {
+    const int32_t lo = wave_min_last(box.r0), hi = ~wave_min_last(~box.r1);
+    if ((threadIdx.x & 63u) == 63u && v0 < a.n_vertices) a.chunk_rows[v0 >> 6] = make_int2(lo, hi);
+  }
   reduce_box(v, item, box, stat, a.item_box, a.item_last, active);
   if (odd) atomicOr(&a.item_last[item], kItemOddBit);
   if (far) atomicOr(&a.item_last[item], kItemFarBit);

@@ -83,7 +83,7 @@ struct rz_context {
   Buf edges, lseg, item_box, item_last, desc, pair_desc, counts, offsets, keys_a, vals_a, keys_b,
       vals_b, tile_off, misc, jobtab, queue, band_n, band_base, band_cnt, band_off, masks, scan_tmp, scan_tmp2,
       scan_tmp3, sort_hist, sort_off, sort_tmp, cover, band_items, band_segs,
-      item_win, at_words, at_base, at_bits, scan_tmp8, scan_box, sp_counts, sp_first, sp_bits, sp_bitn, sp_bit_base;
+      item_win, at_words, at_base, at_bits, scan_tmp8, scan_box, sp_counts, sp_first, sp_bits, sp_bitn, sp_bit_base, chunk_rows;
   // pinned: [0] pairs, [1] (sparse) bit words, [2] band entries, [3] banded segments, [4..6] cover counters
   // (CoverCounters: mask units, small | wave, block), [7] all-touched PixelCache words
   uint64_t* host_misc = nullptr;
@@ -113,7 +113,7 @@ struct rz_context {
             &band_n,    &band_base, &band_cnt,    &band_off,    &masks,      &scan_tmp,   &scan_tmp2, &scan_tmp3,
             &sort_hist, &sort_off,  &sort_tmp,    &cover,       &band_items,
             &band_segs, &item_win,  &at_words,    &at_base,     &at_bits,    &scan_tmp8,  &scan_box,  &sp_counts,
-            &sp_first,  &sp_bits,   &sp_bitn,     &sp_bit_base};
+            &sp_first,  &sp_bits,   &sp_bitn,     &sp_bit_base, &chunk_rows};
   }
   // Takes an event set for the next call (events are recorded on the stream
   // and resolved later, so timing adds no synchronisation to the call).
@@ -845,6 +845,10 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     if (rz_status st = place_cover()) return st;
     cover.mask_cap = read_totals ? (uint64_t)UINT32_MAX : std::min<uint64_t>(mask_fixed, UINT32_MAX);
   }
+  // the row ranges of the chunks of long rings (k_items writes none: its calls
+  // have no rings of more than kCoverBlockNv vertices)
+  const bool any_long = any_poly && max_poly_nv > kChunkNv;
+  if (any_long) HIP_TRY(ensure(c->stream, c->chunk_rows, (size_t)((V + 63) / 64) * sizeof(int2)));
   if (any_lp) HIP_TRY(ensure(c->stream, c->lseg, (size_t)std::max<int64_t>(V, 1) * sizeof(uint4)));
   HIP_TRY(ensure(c->stream, c->item_box, (size_t)std::max<int64_t>(I, 1) * sizeof(ItemBox)));
   HIP_TRY(ensure(c->stream, c->item_last, (size_t)std::max<int64_t>(I, 1) * 8));
@@ -927,6 +931,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     pa.item_box = (ItemBox*)c->item_box.p;
     pa.item_last = (unsigned long long*)c->item_last.p;
     pa.item_win = any_at_cache ? (unsigned long long*)c->item_win.p : nullptr;
+    pa.chunk_rows = any_long ? (int2*)c->chunk_rows.p : nullptr;
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(V)), dim3(256), 0, s, pa);
   }
   DescArgs da{};
@@ -1175,6 +1180,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     ca.desc = (const ItemDesc*)c->desc.p;
     ca.cover = cover;
     ca.masks = (uint64_t*)c->masks.p;
+    ca.chunk_rows = pa.chunk_rows;
     // at most as many workgroups as fill the chip (6 and 4 to a CU: the
     // lists' lengths are on the device)
     if (max_poly_nv > kCoverBlockNv) {
@@ -1196,6 +1202,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
   ta.n_jobs = (int)n;
   ta.desc = (const ItemDesc*)c->desc.p;
   ta.edges = need_edges ? (const PolyEdge*)c->edges.p : nullptr;
+  ta.chunk_rows = pa.chunk_rows;
   ta.lseg = (const uint4*)c->lseg.p;
   ta.burns = c->profiling == 2 ? d_burns : nullptr;
   ta.status = d_status;
@@ -1496,6 +1503,9 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
                     "the geometry needs " + std::to_string(off) +
                         " bytes of workspace; the allocation-free entry point holds at most " +
                         std::to_string(kScratchBytes) + " (use rz_rasterize_device)");
+  // (where there is room left: without them a long ring is read whole)
+  const size_t o_rows = take(dg->max_poly_nv > kChunkNv ? (size_t)((V + 63) / 64) * sizeof(int2) : 0);
+  const bool any_long = dg->max_poly_nv > kChunkNv && off <= kScratchBytes;
   std::lock_guard<std::mutex> lk(g_noalloc_mu[c->device]);
   HIP_TRY(hipSetDevice(c->device));
   char* base = (char*)g_scratch[c->device];
@@ -1531,6 +1541,7 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
     pa.lseg = lines ? (uint4*)(base + o_lseg) : nullptr;
     pa.item_box = d_box;
     pa.item_last = d_last;
+    pa.chunk_rows = any_long ? (int2*)(base + o_rows) : nullptr;
     hipLaunchKernelGGL(k_prep, dim3(blocks_for(V)), dim3(256), 0, s, pa);
   }
   if (I > 0) {
@@ -1553,6 +1564,7 @@ extern "C" rz_status rz_rasterize_device_noalloc(rz_context* c, const rz_device_
   ta.n_jobs = 1;
   ta.desc = d_desc;
   ta.edges = dg->has_poly ? (const PolyEdge*)(base + o_edges) : nullptr;
+  ta.chunk_rows = any_long ? (const int2*)(base + o_rows) : nullptr;
   ta.masks = (const uint64_t*)d_status;  // (read, never used)
   ta.lseg = lines ? (const uint4*)(base + o_lseg) : nullptr;
   ta.status = d_status;

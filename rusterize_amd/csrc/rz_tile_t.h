@@ -132,7 +132,8 @@ __device__ inline StripUnit strip_unit(const TileArgs& a, uint32_t t, int32_t ro
 // row by row from the lanes that hold them.
 __device__ inline uint32_t edge_bits(const TileArgs& a, const ItemDesc& d, const StripUnit& u, int32_t C0,
                                      PolyEdge* stage, int lane) {
-  const uint64_t cov = strip_coverage<1>(a.edges + d.vbeg, (uint32_t)d.nv, u.Rw, u.strip_r1, C0, (double)u.ncols, stage, lane);
+  const uint64_t cov = strip_coverage<1>(a.edges, d.vbeg, (uint32_t)d.nv, a.chunk_rows, u.Rw, u.strip_r1, C0,
+                                         (double)u.ncols, stage, lane);
   uint32_t bits = 0;
   for (int r = 0; r < WAVE_ROWS; ++r) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cov, 4 * r);

@@ -254,3 +254,45 @@ def test_masks_past_their_limit_when_the_need_is_known(monkeypatch):
         assert ctx.workspace_bytes() < 12 << 20
         for b in held:
             b.free()
+
+
+@pytest.mark.parametrize("wide", [None, "never"])
+@pytest.mark.parametrize("rows,cols", [(300, 400), (1500, 130)])
+def test_long_rings_by_chunks(rows, cols, wide, monkeypatch):
+    # rings on both sides of one, two and many chunks of 64 vertices, starting
+    # anywhere in a chunk; smooth ones, whose chunks meet few rows, and ragged
+    # ones, whose chunks meet most; with masks and computed strip by strip, in
+    # a lone call and in a batch with a job before it
+    if wide:
+        monkeypatch.setenv("RUSTERIZE_WIDE", wide)
+    rng = np.random.default_rng(rows)
+    rings = []
+    for k, nv in enumerate([5, 63, 64, 65, 128, 129, 130, 191, 320, 321, 4096, 4097, 4161, 9000]):
+        for inner in (0.98, 0.2):
+            a = np.sort(rng.uniform(0, 2 * np.pi, nv - 1))
+            r = rng.uniform(inner, 1.0, nv - 1)
+            p = np.stack([rng.uniform(0, cols) + cols * 0.6 * r * np.cos(a),
+                          rng.uniform(0, rows) + rows * 0.6 * r * np.sin(a)], 1)
+            rings.append([np.concatenate([p, p[:1]])])
+            rings.append([np.array([(k, k), (k + 9, k), (k + 4, k + 7 + inner), (k, k)])[:3 + k % 2]])
+    g = polygon_rings(rings)
+    with Context(0) as ctx:
+        dg = DeviceGeometry(ctx, g)
+        held, jobs, refs = [dg], [], []
+        for dtype, fun, bg in (("float64", "sum", float("nan")), ("uint8", "count", 0)):
+            field = field_for(dtype, g.n_geoms, seed=cols)
+            info = grid(cols, rows)
+            out = DeviceBuffer(ctx, rows * cols * np.dtype(dtype).itemsize)
+            d_field = DeviceBuffer.from_array(ctx, field)
+            held += [out, d_field]
+            jobs.append(Job(dg, info, dtype, fun, out, field=d_field, background=bg))
+            refs.append(oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, background=bg))
+            rasterize_device(ctx, jobs[-1])
+            ctx.synchronize()
+            assert_same(jobs[-1].result(), refs[-1], f"{dtype} {fun}")
+        batch_rasterize(ctx, jobs[::-1])
+        ctx.synchronize()
+        for job, ref in zip(jobs, refs):
+            assert_same(job.result(), ref, f"batch {job.dtype} {job.fun}")
+        for b in held:
+            b.free()
