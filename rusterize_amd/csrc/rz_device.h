@@ -308,20 +308,51 @@ __device__ inline T bit_select(int32_t mask, T n, T p) {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// XOR-combine a value across the four lanes of a quad with DPP quad
-// permutations ([1,0,3,2] then [2,3,0,1]): VALU data movement, no LDS.
-__device__ inline uint32_t quad_xor_all(uint32_t x) {
+// Combine a value across groups of LANES (4 or 8) lanes with DPP quad
+// permutations ([1,0,3,2] then [2,3,0,1]) and, for 8, a mirror of each half
+// row (the quads hold one value each by then): VALU data movement, no LDS.
+template <int LANES>
+__device__ inline uint32_t group_xor(uint32_t x) {
   x ^= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, false);
   x ^= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xF, 0xF, false);
+  if constexpr (LANES == 8) x ^= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xF, 0xF, false);
   return x;
 }
-__device__ inline uint64_t quad_xor_all64(uint64_t x) {
-  return (uint64_t)quad_xor_all((uint32_t)x) | ((uint64_t)quad_xor_all((uint32_t)(x >> 32)) << 32);
+template <int LANES>
+__device__ inline uint64_t group_xor64(uint64_t x) {
+  return (uint64_t)group_xor<LANES>((uint32_t)x) | ((uint64_t)group_xor<LANES>((uint32_t)(x >> 32)) << 32);
 }
-__device__ inline int32_t quad_max_all(int32_t x) {
+template <int LANES>
+__device__ inline int32_t group_max(int32_t x) {
   x = max(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));
   x = max(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));
+  if constexpr (LANES == 8) x = max(x, __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false));
   return x;
+}
+
+// Transposes 16 x 16 bit blocks over 16 lanes' words: lane i (of each 16)
+// gives row i of the low and of the high block and gets column i of each.
+// Four exchanges with the lane 8, 4, 2 and 1 away, each a rotate and a bit
+// select.
+template <int S>
+__device__ inline uint32_t exchange16(uint32_t x, int lane) {
+  constexpr uint32_t M = S == 8 ? 0x00FF00FFu : (S == 4 ? 0x0F0F0F0Fu : (S == 2 ? 0x33333333u : 0x55555555u));
+  int y;
+  if constexpr (S == 8) {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror:8
+  } else if constexpr (S == 4) {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xF, 0x5, false);  // row_shl:4 into banks 0, 2
+    y = __builtin_amdgcn_update_dpp(y, (int)x, 0x114, 0xF, 0xA, false);  // row_shr:4 into banks 1, 3
+  } else {
+    y = __builtin_amdgcn_update_dpp(0, (int)x, S == 2 ? 0x4E : 0xB1, 0xF, 0xF, false);  // quad_perm
+  }
+  const bool up = (lane & S) != 0;
+  const uint32_t K = up ? ~M : M;
+  const uint32_t r = __builtin_amdgcn_alignbit((uint32_t)y, (uint32_t)y, up ? (uint32_t)S : 32u - (uint32_t)S);
+  return (x & K) | (r & ~K);
+}
+__device__ inline uint32_t transpose16x2(uint32_t x, int lane) {
+  return exchange16<1>(exchange16<2>(exchange16<4>(exchange16<8>(x, lane), lane), lane), lane);
 }
 
 // A workgroup barrier that orders LDS accesses only: global loads and stores
@@ -358,10 +389,11 @@ __device__ inline int32_t wave_min_last(int32_t x) {
 // The chunks of 64 vertices of an item's rings whose edges may meet rows
 // [R0, R1), in order, those of numbers with a bit in `mine` (of number % 64):
 // `rows` holds the row range of each (null: all chunks are taken), 64 of which
-// are tested at a time while the next 64 are loading.  A long ring is mostly
-// local, so a window or strip reads about the edges it needs where it would
-// read all of them (see k_cover and strip_coverage).  Every lane of the wave
-// calls next().
+// are tested at a time (AHEAD: while the next 64 are loading; without it
+// nothing is kept in vector registers).  A long ring is mostly local, so a
+// window or strip reads about the edges it needs where it would read all of
+// them (see k_cover and strip_coverage).  Every lane of the wave calls next().
+template <bool AHEAD>
 struct Chunks {
   const int2* rows;
   uint32_t n, sb;         // chunks; those of [sb, sb + 64) with a bit in m are still to come
@@ -372,15 +404,19 @@ struct Chunks {
 
   __device__ Chunks(const int2* rows_, uint32_t n_, int32_t R0_, int32_t R1_, uint64_t mine_, int lane_)
       : rows(rows_), n(n_), sb(0), R0(R0_), R1(R1_), mine(mine_), ahead(make_int2(0, 0)), lane(lane_) {
-    if (rows && (uint32_t)lane < n) ahead = rows[lane];
+    if (AHEAD && rows && (uint32_t)lane < n) ahead = rows[lane];
     test();
   }
   __device__ void test() {
     const uint32_t left = n - sb;
     m = left < 64u ? mine & ((1ull << left) - 1ull) : mine;
     if (rows) {
+      if (!AHEAD) {
+        ahead = make_int2(0, 0);
+        if ((uint32_t)lane < left) ahead = rows[sb + (uint32_t)lane];
+      }
       m &= __ballot(ahead.x < R1 && ahead.y > R0);
-      if (left > 64u && (uint32_t)lane < left - 64u) ahead = rows[sb + 64u + (uint32_t)lane];
+      if (AHEAD && left > 64u && (uint32_t)lane < left - 64u) ahead = rows[sb + 64u + (uint32_t)lane];
     }
   }
   __device__ bool next(uint32_t& c) {
@@ -422,19 +458,22 @@ __device__ inline uint32_t xcd_unit_lo(uint32_t x, uint32_t n) {
   return x * per + min(x, rem);
 }
 
-// Coverage of one polygon item over the 16 rows [Rw, Rw + 16) (rows from
+// Coverage of one polygon item over ROWS (16 or 8) rows from Rw on (rows from
 // strip_r1 on excluded) and the columns [C0, C0 + 64 * NWORD): lane
-// (rl = lane / 4, q = lane % 4) returns word q of row Rw + rl's mask (lanes
-// with q >= NWORD return 0).  Lane layout: the four lanes of a row take every
-// 4th active edge; their crossing toggles are XOR-combined with DPP and the
-// row mask follows from the note above row_coverage_word in rz_kernels.h.
+// (rl = lane / LPR, q = lane % LPR, LPR = 64 / ROWS) returns word q of row
+// Rw + rl's mask (lanes with q >= NWORD return 0).  Lane layout: the LPR lanes
+// of a row take every LPR-th active edge; their crossing toggles are
+// XOR-combined with DPP and the row mask follows from the note above
+// row_coverage_word in rz_kernels.h.  The item's edges are edges[vbeg .. vbeg
+// + n_e), in the chunks of 64 that meet the rows (chunk_rows: see Chunks).
 // `stage` is 64 edges of wave-private LDS.
-// (the item's edges are edges[vbeg .. vbeg + n_e); chunk_rows: see Chunks)
-template <int NWORD>
+template <int NWORD, int ROWS>
 __device__ inline uint64_t strip_coverage(const PolyEdge* edges, int64_t vbeg, uint32_t n_e, const int2* chunk_rows,
                                           int32_t Rw, int32_t strip_r1, int32_t C0, double ncols_f,
                                           PolyEdge* stage, int lane) {
-  const int rl = lane >> 2, q = lane & 3;
+  constexpr int LPR = 64 / ROWS;  // lanes per row
+  static_assert(LPR == 4 || LPR == 8, "16 or 8 rows");
+  const int rl = lane / LPR, q = lane % LPR;
   const int32_t r = Rw + rl;
   const bool row_ok = r < strip_r1;
   uint64_t tog[NWORD];
@@ -446,7 +485,7 @@ __device__ inline uint64_t strip_coverage(const PolyEdge* edges, int64_t vbeg, u
   const bool local = chunk_rows && n_e > (uint32_t)kChunkNv;
   const uint32_t skew = local ? (uint32_t)vbeg & 63u : 0u;
   const PolyEdge* ebase = edges + vbeg;
-  Chunks chunks(local ? chunk_rows + (vbeg >> 6) : nullptr, (n_e + skew + 63u) >> 6, Rw, strip_r1, ~0ull, lane);
+  Chunks<false> chunks(local ? chunk_rows + (vbeg >> 6) : nullptr, (n_e + skew + 63u) >> 6, Rw, strip_r1, ~0ull, lane);
   uint32_t c;
   while (chunks.next(c)) {
     // stage the edges of this chunk that reach the strip, compacted
@@ -469,7 +508,7 @@ __device__ inline uint64_t strip_coverage(const PolyEdge* edges, int64_t vbeg, u
     }
     wave_sync();
     const int n = __popcll(m);
-    for (int k0 = 0; k0 < n; k0 += 4) {  // uniform trip count, predicated lanes
+    for (int k0 = 0; k0 < n; k0 += LPR) {  // uniform trip count, predicated lanes
       const int k = k0 + q;
       const PolyEdge ee = stage[k < n ? k : n - 1];
       const bool on = k < n && row_ok && ee.ystart <= r && r < ee.yend;
@@ -478,10 +517,10 @@ __device__ inline uint64_t strip_coverage(const PolyEdge* edges, int64_t vbeg, u
     }
     wave_sync();
   }
-  lp = quad_xor_all(lp);
-  amax = quad_max_all(amax);
+  lp = group_xor<LPR>(lp);
+  amax = group_max<LPR>(amax);
 #pragma unroll
-  for (int w = 0; w < NWORD; ++w) tog[w] = quad_xor_all64(tog[w]);
+  for (int w = 0; w < NWORD; ++w) tog[w] = group_xor64<LPR>(tog[w]);
   return q < NWORD ? row_coverage_word<NWORD>(tog, lp, amax, C0, q) : 0ull;
 }
 

@@ -5,32 +5,11 @@
 
 namespace rzk {
 
-// Transposes the four 16 x 16 bit blocks of 16 lanes' words: lane i (of each
-// 16) gives row i's 64 columns and gets, in 16-bit element j, the rows' bits
-// of column 16 j + i (mask_element's order).  Four exchanges with the lane 8,
-// 4, 2 and 1 away, each a rotate and a bit select per half.
-template <int S>
-__device__ inline uint32_t exchange16(uint32_t x, int lane) {
-  constexpr uint32_t M = S == 8 ? 0x00FF00FFu : (S == 4 ? 0x0F0F0F0Fu : (S == 2 ? 0x33333333u : 0x55555555u));
-  int y;
-  if constexpr (S == 8) {
-    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);  // row_ror:8
-  } else if constexpr (S == 4) {
-    y = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xF, 0x5, false);  // row_shl:4 into banks 0, 2
-    y = __builtin_amdgcn_update_dpp(y, (int)x, 0x114, 0xF, 0xA, false);  // row_shr:4 into banks 1, 3
-  } else {
-    y = __builtin_amdgcn_update_dpp(0, (int)x, S == 2 ? 0x4E : 0xB1, 0xF, 0xF, false);  // quad_perm
-  }
-  const bool up = (lane & S) != 0;
-  const uint32_t K = up ? ~M : M;
-  const uint32_t r = __builtin_amdgcn_alignbit((uint32_t)y, (uint32_t)y, up ? (uint32_t)S : 32u - (uint32_t)S);
-  return (x & K) | (r & ~K);
-}
+// A strip's row words, row i's 64 columns in lane i of each 16, to
+// mask_element's order: 16-bit element j of lane i gets the rows' bits of
+// column 16 j + i.
 __device__ inline uint64_t transpose16(uint64_t x, int lane) {
-  uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
-  lo = exchange16<1>(exchange16<2>(exchange16<4>(exchange16<8>(lo, lane), lane), lane), lane);
-  hi = exchange16<1>(exchange16<2>(exchange16<4>(exchange16<8>(hi, lane), lane), lane), lane);
-  return (uint64_t)lo | ((uint64_t)hi << 32);
+  return (uint64_t)transpose16x2((uint32_t)x, lane) | ((uint64_t)transpose16x2((uint32_t)(x >> 32), lane) << 32);
 }
 
 // An item (or a window of one) whose toggle words are in LDS.
@@ -98,7 +77,7 @@ struct CoverWave {
   // that `chunks` hands out, its first `skew` edges before the item's.
   template <bool AHEAD>
   __device__ __attribute__((always_inline)) void toggles(const RZ_CONST JobDev& J, bool many, bool own, uint32_t e0,
-                                                         uint32_t n_e, Chunks* chunks, uint32_t skew, bool odd) const {
+                                                         uint32_t n_e, Chunks<true>* chunks, uint32_t skew, bool odd) const {
     const double ncols_f = (double)J.ncols;
     const bool sx = J.xres != 1.0, sy = J.yres != 1.0;  // (v / 1.0 is v)
     auto px_x = [&](double X) { return isnan(X) ? X : (sx ? (X - J.xmin) / J.xres : X - J.xmin); };
@@ -304,7 +283,7 @@ struct CoverWave {
       const bool all = win.n == 1;
       const uint32_t skew = all ? 0u : (uint32_t)vbeg & 63u;
       static_assert(kCoverBlockWaves == 4, "every fourth chunk is a wave's");
-      Chunks chunks(all ? nullptr : chunk_rows + (vbeg >> 6), (nv + skew + 63u) >> 6, R0, R0 + n_rows,
+      Chunks<true> chunks(all ? nullptr : chunk_rows + (vbeg >> 6), (nv + skew + 63u) >> 6, R0, R0 + n_rows,
                     0x1111111111111111ull << wave_index(), lane);
       toggles<true>(J, false, false, 0u, nv, &chunks, skew, odd);
     } else {

@@ -127,28 +127,59 @@ __device__ inline StripUnit strip_unit(const TileArgs& a, uint32_t t, int32_t ro
   return u;
 }
 
-// The rows an item without masks covers in column C0 + lane of the unit, as
-// bits: its coverage from its edges (strip_coverage's row words), read back
-// row by row from the lanes that hold them.
-__device__ inline uint32_t edge_bits(const TileArgs& a, const ItemDesc& d, const StripUnit& u, int32_t C0,
-                                     PolyEdge* stage, int lane) {
-  const uint64_t cov = strip_coverage<1>(a.edges, d.vbeg, (uint32_t)d.nv, a.chunk_rows, u.Rw, u.strip_r1, C0,
-                                         (double)u.ncols, stage, lane);
-  uint32_t bits = 0;
-  for (int r = 0; r < WAVE_ROWS; ++r) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cov, 4 * r);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cov >> 32), 4 * r);
-    bits |= ((lane < 32 ? lo : hi) >> (lane & 31) & 1u) << r;
+// The row words of an item without masks in a unit of ROWS rows, from its
+// edges: word w of row r in lane r * 64 / ROWS + w - wlo.  One reading of the
+// edges for all the tile words it meets, and of the words only the one where
+// it meets no other (a word less per crossing to toggle and combine).
+template <int NWORD, int ROWS>
+__device__ __attribute__((always_inline)) inline uint64_t edge_words(const TileArgs& a, const ItemDesc& d, const StripUnit& u,
+                                                                     PolyEdge* stage, int lane, int& wlo) {
+  const uint32_t n = (uint32_t)d.nv;
+  const int w0 = max(0, (d.c0 >> 6) - (u.C0 >> 6));
+  if (NWORD > 1 && w0 < min(NWORD - 1, ((d.c1 - 1) >> 6) - (u.C0 >> 6))) {
+    wlo = 0;
+    return strip_coverage<NWORD, ROWS>(a.edges, d.vbeg, n, a.chunk_rows, u.Rw, u.strip_r1, u.C0, (double)u.ncols, stage, lane);
   }
-  return bits;
+  wlo = w0;
+  return strip_coverage<1, ROWS>(a.edges, d.vbeg, n, a.chunk_rows, u.Rw, u.strip_r1, u.C0 + 64 * w0, (double)u.ncols, stage,
+                                 lane);
 }
 
-// ... of any polygon item in tile word w, for a unit of 16 rows (k_tile_lp).
+// The rows that edge_words' words number w (from wlo on) cover in column lane
+// of it, as bits: each row's word goes to the lanes of its number (mod 16),
+// where a 16 x 16 transposition turns the 16 columns of a lane's quarter into
+// row bits (about 30 instructions, where reading the words back row by row
+// took 100).
+template <int ROWS>
+__device__ inline uint32_t word_bits(uint64_t words, int w, int lane) {
+  constexpr int LPR = 64 / ROWS;
+  const int from = (lane & (ROWS - 1)) * LPR + w;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * from, (int)(uint32_t)words);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * from, (int)(uint32_t)(words >> 32));
+  const uint32_t half = lane < 32 ? lo : hi;
+  uint32_t x = (lane & 16 ? half >> 16 : half) & 0xFFFFu;
+  if (ROWS < 16 && (lane & 15) >= ROWS) x = 0u;
+  return transpose16x2(x, lane) & 0xFFFFu;
+}
+
+// The rows any polygon item covers in column lane of tile word w, for a unit
+// of 16 rows (k_tile_lp, whose registers are all in use: an item without masks
+// has its edges read for each word, and word_bits would spill more).
 __device__ inline uint32_t column_bits(const TileArgs& a, const ItemDesc& d, const StripUnit& u, int w, PolyEdge* stage,
                                        int lane) {
   const int32_t wi = (u.C0 >> 6) + w - (d.c0 >> 6), nw = mask_row_words(d.c0, d.c1);
   if (wi < 0 || wi >= nw) return 0u;
-  if (!(d.flags & kItemMask)) return edge_bits(a, d, u, u.C0 + 64 * w, stage, lane);
+  if (!(d.flags & kItemMask)) {
+    const uint64_t cov = strip_coverage<1, WAVE_ROWS>(a.edges, d.vbeg, (uint32_t)d.nv, a.chunk_rows, u.Rw, u.strip_r1,
+                                                      u.C0 + 64 * w, (double)u.ncols, stage, lane);
+    uint32_t bits = 0;
+    for (int r = 0; r < WAVE_ROWS; ++r) {
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cov, 4 * r);
+      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cov >> 32), 4 * r);
+      bits |= ((lane < 32 ? lo : hi) >> (lane & 31) & 1u) << r;
+    }
+    return bits;
+  }
   const uint64_t* p = a.masks + ((uint64_t)d.mask + (uint64_t)((u.Rw >> 4) - (d.r0 >> 4)) * (uint64_t)nw + (uint64_t)wi) * 16u;
   return reinterpret_cast<const uint16_t*>(p)[mask_element(lane)];
 }
@@ -525,11 +556,30 @@ __device__ inline void load_bits(const TileArgs& a, const Visits& v, uint32_t k,
 // store it took about 80 instructions per item and strip before the folds,
 // and computing the coverage in the strip about 200.  Reading the masks as
 // execution masks through scalar loads needs half the vector instructions,
-// but the scalar cache's misses bound it.)  BARE: items without masks may be
-// among them.
-template <typename T, int FUN, int ROWS, bool BARE, int N, typename F>
+// but the scalar cache's misses bound it.)
+template <typename T, int FUN, int ROWS>
+__device__ __attribute__((always_inline)) inline void fold_visit(const TileArgs& a, const StripUnit& u, Pixels<T, ROWS>& p,
+                                                                 const Visits& v, uint32_t k, uint32_t y, uint32_t& burns) {
+  constexpr int NWORD = Pixels<T, ROWS>::NWORD;
+  const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
+  const uint32_t v0 = (uint32_t)__builtin_amdgcn_readlane((int)v.v0, (int)k);
+  const uint32_t v1 = sizeof(T) == 8 ? (uint32_t)__builtin_amdgcn_readlane((int)v.v1, (int)k) : 0u;
+  if (a.burns) burns += (uint32_t)__popc(y);
+  const int lo = (int)((info >> 8) & 31u), hi = (int)((info >> 16) & 31u);
+#pragma unroll
+  for (int w = 0; w < NWORD; ++w)
+    if (NWORD == 1 || (info & 3u) == (uint32_t)w) {  // (uniform)
+      p.template fold<FUN>(w, y, lo, hi, (uint64_t)v0 | ((uint64_t)v1 << 32), u.J->bg_bits);
+    }
+}
+// The unit's rows of a mask block's 16.
+template <int ROWS>
+__device__ inline uint32_t unit_rows(const StripUnit& u, uint32_t y) {
+  return ROWS < 16 ? (y >> (u.Rw & 15)) & ((1u << ROWS) - 1u) : y;
+}
+template <typename T, int FUN, int ROWS, int N>
 __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels<T, ROWS>& p, const Visits& v,
-                                   uint32_t (&bits)[N], PolyEdge* stage, int lane, uint32_t& burns, F&& desc_of) {
+                                   uint32_t (&bits)[N], int lane, uint32_t& burns) {
   constexpr int NWORD = Pixels<T, ROWS>::NWORD;
   const int shift = ROWS < 16 ? (u.Rw & 15) : 0;
   auto fold = [&](uint32_t k, uint32_t y) __attribute__((always_inline)) {
@@ -545,22 +595,6 @@ __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels
       }
   };
   auto rows = [&](uint32_t y) { return ROWS < 16 ? (y >> shift) & ((1u << ROWS) - 1u) : y; };
-  if (BARE && __any((uint32_t)lane < v.n && (v.info >> 31))) {
-    for (uint32_t k = 0; k < v.n; ++k) {
-      const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
-      uint32_t y;
-      if (info >> 31) {
-        y = edge_bits(a, desc_of(__builtin_amdgcn_readlane((int)v.item, (int)k)), u, u.C0 + 64 * (int32_t)(info & 3u), stage,
-                      lane);
-      } else {
-        uint32_t one[1];
-        load_bits(a, v, k, one, lane);
-        y = rows(one[0]);
-      }
-      fold(k, y);
-    }
-    return;
-  }
   for (uint32_t k = 0; k < v.n; k += (uint32_t)N) {
     uint32_t nxt[N] = {};
     const bool more = k + (uint32_t)N < v.n;
@@ -572,6 +606,36 @@ __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels
 #pragma unroll
       for (int g = 0; g < N; ++g) bits[g] = nxt[g];
     }
+  }
+}
+
+// Whether items without masks are among the visits.
+__device__ inline bool any_bare(const Visits& v, int lane) { return __any((uint32_t)lane < v.n && (v.info >> 31)); }
+// ... then fold(k, bits) for one visit after the other; desc_of: the
+// descriptor of the item in a lane of the batch.
+template <int NWORD, int ROWS, typename D, typename F>
+__device__ __attribute__((always_inline)) inline void bare_visits(const TileArgs& a, const StripUnit& u, const Visits& v,
+                                                                  PolyEdge* stage, int lane, D&& desc_of, F&& fold) {
+  uint64_t words = 0ull;  // the row words of the item in lane `at`
+  int at = -1, wlo = 0;
+  for (uint32_t k = 0; k < v.n; ++k) {
+    const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
+    // (what is computed of the lane alone is computed here each time: kept
+    // from before the loop it would take 20 registers of all calls)
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    uint32_t y;
+    if (info >> 31) {
+      const int item = __builtin_amdgcn_readlane((int)v.item, (int)k);
+      if (NWORD == 1 || item != at) words = edge_words<NWORD, ROWS>(a, desc_of(item), u, stage, l, wlo);
+      at = item;
+      y = word_bits<ROWS>(words, (int)(info & 3u) - wlo, l);
+    } else {
+      uint32_t one[1];
+      load_bits(a, v, k, one, l);
+      y = unit_rows<ROWS>(u, one[0]);
+    }
+    fold(k, y);
   }
 }
 
@@ -653,6 +717,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupan
     return visits_of<NWORD, WAVE_ROWS, WIDE>(q, x.u, x.have && x.g.ib + lane < x.g.ie, left, s_x[wave]);
   };
 
+  // (batch: the first of the items whose lanes v.item names)
+  auto fold = [&](const StripUnit& u, Pixels<T, WAVE_ROWS>& p, const Visits& v, uint32_t (&bits)[kAhead<T>],
+                  const ItemDesc* batch) __attribute__((always_inline)) {
+    if constexpr (BARE) {
+      if (any_bare(v, lane)) {
+        bare_visits<NWORD, WAVE_ROWS>(
+            a, u, v, s_edge[wave], lane, [&](int b) { return load_desc(as_const(batch) + b); },
+            [&](uint32_t k, uint32_t y) __attribute__((always_inline)) { fold_visit<T, FUN, WAVE_ROWS>(a, u, p, v, k, y, burns); });
+        return;
+      }
+    }
+    fold_visits<T, FUN, WAVE_ROWS>(a, u, p, v, bits, lane, burns);
+  };
+
   Unit A = pop_unit(tq.begin()), B{}, C{};
   if (A.have) B = pop_unit(tq.advance());
   if (B.have) C = pop_unit(tq.advance());
@@ -677,8 +755,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupan
     Pixels<T, WAVE_ROWS> p;
     p.fill(A.u);
     if (va.n)
-      fold_visits<T, FUN, WAVE_ROWS, BARE>(a, A.u, p, va, bits_a, s_edge[BARE ? wave : 0], lane, burns,
-                                           [&](int b) { return load_desc(as_const(A.g.list) + A.g.ib + b); });
+      fold(A.u, p, va, bits_a, A.g.list + A.g.ib);
     // the candidates past the first batch (64 items or visits), in order; scan
     // jobs of one band test the 8-byte boxes in strip and tile units first
     for (int64_t base = A.g.ib; left_a || base + 64 < A.g.ie;) {
@@ -697,8 +774,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupan
       if (!v.n) continue;
       uint32_t bits[kAhead<T>];
       load_bits(a, v, 0u, bits, lane);
-      fold_visits<T, FUN, WAVE_ROWS, BARE>(a, A.u, p, v, bits, s_edge[BARE ? wave : 0], lane, burns,
-                                           [&](int b) { return load_desc(as_const(A.g.list) + base + b); });
+      fold(A.u, p, v, bits, A.g.list + base);
     }
 
     // everything loaded has arrived
@@ -741,12 +817,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupan
 // waves 1,000 stars on 2048 x 2048 take 17.4 us, with 16 waves (4 rows each,
 // half the tiles at a time) 23.5, with 4 waves 16.5 but 52 on the 32 jobs.
 constexpr int kTileBlockWaves = 8;
-template <typename T>
+template <typename F>
+__device__ __attribute__((always_inline)) inline void with_fun(int32_t fun, F&& f) {
+  switch (fun) {
+    case 0: f(std::integral_constant<int, 0>{}); break;
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    default: f(std::integral_constant<int, 6>{}); break;
+  }
+}
+// BARE: compiled with the path for items without masks (its registers and LDS
+// cost the others 5 % on bytes: 170 us against 163 for 10,000 polygons on
+// 3989 x 4013 x 3).
+template <typename T, bool BARE>
 __global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a) {
   constexpr int TW = tile_w(sizeof(T));
   constexpr int NWORD = TW / 64;
   constexpr int ROWS = TILE_H / kTileBlockWaves;
-  __shared__ PolyEdge s_edge[kTileBlockWaves][64];
+  __shared__ PolyEdge s_edge[BARE ? kTileBlockWaves : 1][64];
   __shared__ __align__(16) uint32_t s_x[kTileBlockWaves][NWORD > 1 ? 256 : 1];
   __shared__ uint32_t s_list[64 * kTileBlockWaves], s_n[kTileBlockWaves];
   const int wave = wave_index(), lane = threadIdx.x & 63;
@@ -769,23 +860,30 @@ __global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a)
       if (!v.n) break;
       uint32_t bits[kAhead<T>];
       load_bits(a, v, 0u, bits, lane);
-      auto desc_of = [&](int b) {
-        const uint64_t at = (uint64_t)d;
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, b);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), b);
-        return load_desc((const RZ_CONST ItemDesc*)((uint64_t)lo | ((uint64_t)hi << 32)));
-      };
-      auto fold_fun = [&](auto fun) __attribute__((always_inline)) {
-        fold_visits<T, decltype(fun)::value, ROWS, true>(a, u, p, v, bits, s_edge[wave], lane, burns, desc_of);
-      };
+      if constexpr (BARE) {
+        if (any_bare(v, lane)) {
+          auto desc_of = [&](int b) {
+            const uint64_t at = (uint64_t)d;
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, b);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), b);
+            return load_desc((const RZ_CONST ItemDesc*)((uint64_t)lo | ((uint64_t)hi << 32)));
+          };
+          bare_visits<NWORD, ROWS>(a, u, v, s_edge[wave], lane, desc_of, [&](uint32_t k, uint32_t y) __attribute__((always_inline)) {
+            with_fun(J.fun, [&](auto fun) __attribute__((always_inline)) {
+              fold_visit<T, decltype(fun)::value, ROWS>(a, u, p, v, k, y, burns);
+            });
+          });
+          continue;
+        }
+      }
       switch (J.fun) {
-        case 0: fold_fun(std::integral_constant<int, 0>{}); break;
-        case 1: fold_fun(std::integral_constant<int, 1>{}); break;
-        case 2: fold_fun(std::integral_constant<int, 2>{}); break;
-        case 3: fold_fun(std::integral_constant<int, 3>{}); break;
-        case 4: fold_fun(std::integral_constant<int, 4>{}); break;
-        case 5: fold_fun(std::integral_constant<int, 5>{}); break;
-        default: fold_fun(std::integral_constant<int, 6>{}); break;
+        case 0: fold_visits<T, 0, ROWS>(a, u, p, v, bits, lane, burns); break;
+        case 1: fold_visits<T, 1, ROWS>(a, u, p, v, bits, lane, burns); break;
+        case 2: fold_visits<T, 2, ROWS>(a, u, p, v, bits, lane, burns); break;
+        case 3: fold_visits<T, 3, ROWS>(a, u, p, v, bits, lane, burns); break;
+        case 4: fold_visits<T, 4, ROWS>(a, u, p, v, bits, lane, burns); break;
+        case 5: fold_visits<T, 5, ROWS>(a, u, p, v, bits, lane, burns); break;
+        default: fold_visits<T, 6, ROWS>(a, u, p, v, bits, lane, burns); break;
       }
     }
   };
@@ -794,18 +892,19 @@ __global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a)
     for (uint32_t i = pb; i < pe; i += 64u) fold(a.pair_desc + i + lane, (uint32_t)lane < pe - i);
   } else {
     const bool compact = J.scan_compact && a.scan_box;
+    const int64_t ib = J.i_base;
     const int32_t T0 = u.Rw - wave * ROWS, T1 = min(T0 + TILE_H, u.nrows);  // the tile's rows
     for (int64_t base = 0; base < J.ni; base += 64 * kTileBlockWaves) {
       const int64_t i = base + wave * 64 + lane;
       bool meets = i < J.ni;
       if (meets) {
         if (compact) {
-          const uint2 bx = a.scan_box[J.i_base + i];
+          const uint2 bx = a.scan_box[ib + i];
           const uint32_t tx = (uint32_t)u.C0 / (uint32_t)TW, s0 = (uint32_t)T0 / WAVE_ROWS;
           meets = (bx.x & 0xFFFFu) <= s0 + TILE_H / WAVE_ROWS - 1 && s0 <= (bx.x >> 16) && (bx.y & 0xFFFFu) <= tx &&
                   tx <= (bx.y >> 16);
         } else {
-          const u32x4 q = *reinterpret_cast<const u32x4*>(a.desc + J.i_base + i);
+          const u32x4 q = *reinterpret_cast<const u32x4*>(a.desc + ib + i);
           meets = (int32_t)q[0] < T1 && (int32_t)q[1] > T0 && (int32_t)q[2] < u.tile_c1 && (int32_t)q[3] > u.C0;
         }
       }
@@ -821,7 +920,7 @@ __global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a)
       __syncthreads();
       for (uint32_t k = 0; k < n; k += 64u) {
         const bool cand = k + (uint32_t)lane < n;
-        fold(a.desc + J.i_base + base + (cand ? (int64_t)s_list[k + lane] : 0), cand);
+        fold(a.desc + ib + base + (cand ? (int64_t)s_list[k + lane] : 0), cand);
       }
       __syncthreads();  // the next boxes overwrite the list
     }

@@ -296,3 +296,32 @@ def test_long_rings_by_chunks(rows, cols, wide, monkeypatch):
             assert_same(job.result(), ref, f"batch {job.dtype} {job.fun}")
         for b in held:
             b.free()
+
+
+@pytest.mark.parametrize("binning", ["always", "never"])
+@pytest.mark.parametrize("dtype", ["uint8", "int16", "float32", "float64"])
+@pytest.mark.parametrize("rows,cols,n_layers", [(1, 1, 1), (15, 63, 1), (25, 65, 1), (65, 257, 1), (129, 1023, 2),
+                                                (67, 130, 2100)])
+def test_strips_without_masks(rows, cols, n_layers, dtype, binning, monkeypatch):
+    # every item's coverage from its edges: units of 8 rows (a workgroup per
+    # tile) and, with 2,100 layers, of 16; items in one, two and all of a
+    # tile's 64-column words, past the raster on every side, and lines beside
+    # them (the third kernel) in the last function
+    monkeypatch.setenv("RUSTERIZE_BINNING", binning)
+    monkeypatch.setenv("RUSTERIZE_WIDE", "never")
+    g = polygons(rows, cols)
+    info = _lib.raster_info(None, resolution=(1.0, 1.0), extent=(0, 0, cols, rows))
+    for fun, bg in (("sum", 0), ("count", 2), ("first", 1), ("min", 0)):
+        if fun == "min":
+            t = np.linspace(0, 1, 40)
+            line = np.stack([cols * t, rows * (0.5 + 0.4 * np.sin(9 * t))], 1)
+            g = Geometry(np.arange(g.n_geoms + 2), np.append(g.item_kind, 1).astype(np.int32),
+                         np.append(g.item_ring_offsets, g.item_ring_offsets[-1] + 1),
+                         np.append(g.ring_vertex_offsets, g.ring_vertex_offsets[-1] + 40),
+                         np.concatenate([g.xy, line]))
+        layers = (np.arange(g.n_geoms) * 37 % n_layers // (3 if n_layers > 1 else 1)).astype(np.uint32)
+        field = field_for(dtype, g.n_geoms, seed=rows + cols)
+        got = _lib.rasterize(g, info, dtype, fun, field, None, layers, n_layers, bg)
+        ref = oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, layer_of_geom=layers,
+                               n_layers=n_layers, background=bg)
+        assert_same(got, ref, f"{rows}x{cols}x{n_layers} {dtype} {fun} {binning}")
