@@ -375,17 +375,6 @@ __device__ inline uint32_t wave_prefix_sum(uint32_t x) {
   return x;
 }
 
-// Minimum over the wave, in its last lane (as wave_prefix_sum).
-__device__ inline int32_t wave_min_last(int32_t x) {
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x111, 0xF, 0xF, false));
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x112, 0xF, 0xF, false));
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x114, 0xF, 0xF, false));
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x118, 0xF, 0xF, false));
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x142, 0xA, 0xF, false));
-  x = min(x, __builtin_amdgcn_update_dpp(INT_MAX, x, 0x143, 0xC, 0xF, false));
-  return x;
-}
-
 // The chunks of 64 vertices of an item's rings whose edges may meet rows
 // [R0, R1), in order, those of numbers with a bit in `mine` (of number % 64):
 // `rows` holds the row range of each (null: all chunks are taken), 64 of which

@@ -108,7 +108,9 @@ __device__ inline void merge_box(int it, ItemBox& b) {
 // atomics per item segment.  Items own contiguous vertex ranges, so lanes of
 // one item are contiguous.  `stat` is a line lane's kept segment + 1 (v + 1; 0: none
 // kept, and for polygon and point lanes), whose maximum goes to item_last.
-__device__ inline void reduce_box(int64_t v, int64_t item, ItemBox b, uint64_t stat, ItemBox* out,
+// Returns, in lane 63, the rows that the wave's vertices meet if they are one
+// item's (all rows otherwise).
+__device__ inline int2 reduce_box(int64_t v, int64_t item, ItemBox b, uint64_t stat, ItemBox* out,
                                   unsigned long long* last_out, bool active) {
   const int lane = threadIdx.x & 63;
   // (items of one wave are neighbours, so their low halves tell them apart)
@@ -120,8 +122,11 @@ __device__ inline void reduce_box(int64_t v, int64_t item, ItemBox b, uint64_t s
   merge_box<0x118, 0xF>(it, b);
   merge_box<0x142, 0xA>(it, b);  // lane 15 of a row into the next one
   merge_box<0x143, 0xC>(it, b);  // lane 31 into the upper half
-  const bool head = lane == 0 || __builtin_amdgcn_update_dpp(0, it, 0x138, 0xF, 0xF, false) != it;  // wave_shr:1
-  const uint64_t heads = __ballot(head);
+  // the lane before: row_shr:1, into a row's first lane row_bcast:15 (wave_shr:1
+  // does not cross rows here: every 16 lanes wrote the box of a long ring)
+  int prev = __builtin_amdgcn_update_dpp(0, it, 0x142, 0xE, 0xF, false);
+  prev = __builtin_amdgcn_update_dpp(prev, it, 0x111, 0xF, 0xF, false);
+  const uint64_t heads = __ballot(lane == 0 || prev != it);
   const bool tail = lane == 63 || ((heads >> 1) >> lane & 1ull);
   if (kept && tail) {  // the item's last kept segment in this wave
     const uint64_t upto = ~0ull >> (63 - lane);
@@ -139,6 +144,7 @@ __device__ inline void reduce_box(int64_t v, int64_t item, ItemBox b, uint64_t s
     atomicMax(&out[item].c1, b.c1);
   }
   if (active && tail && stat) atomicMax(&last_out[item], (unsigned long long)stat);
+  return heads == 1ull ? make_int2(b.r0, b.r1) : make_int2(INT_MIN, INT_MAX);
 }
 
 // The edge (pixel coordinates x0, y0 to x1, y1) that starts at a polygon
@@ -301,11 +307,8 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
   } else if (active) {
     vertex(as_const(a.jobs)[find_job(a.job_vend, a.n_jobs, v)]);
   }
-  if (a.chunk_rows) {
-    const int32_t lo = wave_min_last(box.r0), hi = ~wave_min_last(~box.r1);
-    if ((threadIdx.x & 63u) == 63u && v0 < a.n_vertices) a.chunk_rows[v0 >> 6] = make_int2(lo, hi);
-  }
-  reduce_box(v, item, box, stat, a.item_box, a.item_last, active);
+  const int2 rows = reduce_box(v, item, box, stat, a.item_box, a.item_last, active);
+  if (a.chunk_rows && (threadIdx.x & 63u) == 63u && v0 < a.n_vertices) a.chunk_rows[v0 >> 6] = rows;
   if (odd) atomicOr(&a.item_last[item], kItemOddBit);
   if (far) atomicOr(&a.item_last[item], kItemFarBit);
 }
