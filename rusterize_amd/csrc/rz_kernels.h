@@ -502,6 +502,7 @@ struct TileArgs {
   const uint64_t* band_off;   // edge bands of banded line items
   const uint4* band_segs;
   const uint64_t* masks;      // coverage masks of kItemMask items
+  int any_mask;               // whether an item may have some (edges null: all polygons do)
   // scan jobs: every item of the job is tested against the tile
   const ItemDesc* desc;
   const PolyEdge* edges;    // read for polygon items without masks only

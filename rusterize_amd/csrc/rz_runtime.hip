@@ -1190,6 +1190,7 @@ static rz_status run_batch(rz_context* c, const rz_job* jobs_in, int64_t n_in,
     const uint64_t g = ((uint64_t)I + (read_totals ? c->last_units : 0)) / 4 + 1;
     hipLaunchKernelGGL(k_cover<false>, dim3((unsigned)std::min<uint64_t>(g, 1536)), dim3(256), 0, s, ca);
     ta.masks = (const uint64_t*)c->masks.p;
+    ta.any_mask = 1;
   } else {
     ta.masks = (const uint64_t*)c->misc.p;  // (read, never used: the tile kernels load ahead)
   }

@@ -88,8 +88,10 @@ void RZ_CAT(launch_tile_, RZ_TILE_NAME)(int fun, const TileArgs& a, bool lines, 
 
 void RZ_CAT(launch_blocks_, RZ_TILE_NAME)(const TileArgs& a, hipStream_t s) {
   const uint32_t g = (a.t_hi - a.t_lo + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
-  if (a.edges) hipLaunchKernelGGL((k_tile_block<T, true>), dim3(g), dim3(64 * kTileBlockWaves), 0, s, a);
-  else hipLaunchKernelGGL((k_tile_block<T, false>), dim3(g), dim3(64 * kTileBlockWaves), 0, s, a);
+  const dim3 block(64 * kTileBlockWaves);
+  if (!a.edges) hipLaunchKernelGGL((k_tile_block<T, 0>), dim3(g), block, 0, s, a);
+  else if (a.any_mask) hipLaunchKernelGGL((k_tile_block<T, 1>), dim3(g), block, 0, s, a);
+  else hipLaunchKernelGGL((k_tile_block<T, 2>), dim3(g), block, 0, s, a);
 }
 
 }  // namespace rzk

@@ -589,7 +589,7 @@ __device__ inline uint32_t unit_rows(const StripUnit& u, uint32_t y) {
 }
 template <typename T, int FUN, int ROWS, int N>
 __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels<T, ROWS>& p, const Visits& v,
-                                   uint32_t (&bits)[N], int lane, uint32_t& burns) {
+                                   uint32_t k0, uint32_t end, uint32_t (&bits)[N], int lane, uint32_t& burns) {
   constexpr int NWORD = Pixels<T, ROWS>::NWORD;
   const int shift = ROWS < 16 ? (u.Rw & 15) : 0;
   auto fold = [&](uint32_t k, uint32_t y) __attribute__((always_inline)) {
@@ -605,13 +605,13 @@ __device__ inline void fold_visits(const TileArgs& a, const StripUnit& u, Pixels
       }
   };
   auto rows = [&](uint32_t y) { return ROWS < 16 ? (y >> shift) & ((1u << ROWS) - 1u) : y; };
-  for (uint32_t k = 0; k < v.n; k += (uint32_t)N) {
+  for (uint32_t k = k0; k < end; k += (uint32_t)N) {
     uint32_t nxt[N] = {};
-    const bool more = k + (uint32_t)N < v.n;
+    const bool more = k + (uint32_t)N < end;
     if (more) load_bits(a, v, k + (uint32_t)N, nxt, lane);
 #pragma unroll
     for (int g = 0; g < N; ++g)
-      if (k + (uint32_t)g < v.n) fold(k + (uint32_t)g, rows(bits[g]));
+      if (k + (uint32_t)g < end) fold(k + (uint32_t)g, rows(bits[g]));
     if (more) {
 #pragma unroll
       for (int g = 0; g < N; ++g) bits[g] = nxt[g];
@@ -738,7 +738,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TileOccupan
         return;
       }
     }
-    fold_visits<T, FUN, WAVE_ROWS>(a, u, p, v, bits, lane, burns);
+    fold_visits<T, FUN, WAVE_ROWS>(a, u, p, v, 0u, v.n, bits, lane, burns);
   };
 
   Unit A = pop_unit(tq.begin()), B{}, C{};
@@ -839,11 +839,18 @@ __device__ __attribute__((always_inline)) inline void with_fun(int32_t fun, F&& 
     default: f(std::integral_constant<int, 6>{}); break;
   }
 }
-// BARE: compiled with the path for items without masks (its registers and LDS
-// cost the others 5 % on bytes: 170 us against 163 for 10,000 polygons on
-// 3989 x 4013 x 3).
-template <typename T, bool BARE>
-__global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a) {
+// BARE: whether items have no masks: 0 none, 1 some may, 2 all (calls too small
+// for masks, the allocation-free entry point).  A variant each, as that path's
+// registers and LDS cost the others 5 % on bytes (170 us against 163 for 10,000
+// polygons on 3989 x 4013 x 3).  1 folds both kinds through one copy of the
+// code, in at most 80 registers for 1-byte pixels, so that three workgroups
+// fit a CU (1,800 stars on 3417 x 2960 uint8: 37.6 us a call; with a second
+// copy of the folds 44.2); 2 needs no mask loads (95 stars on 827 x 1253
+// float64: 19.4 us, through 1 20.2).
+constexpr int kBlockMinWaves = 2;  // (what two waves of a workgroup per SIMD take anyway)
+template <typename T, int BARE>
+__global__ __launch_bounds__(64 * kTileBlockWaves)
+    __attribute__((amdgpu_waves_per_eu(BARE == 1 && sizeof(T) == 1 ? 6 : kBlockMinWaves))) void k_tile_block(TileArgs a) {
   constexpr int TW = tile_w(sizeof(T));
   constexpr int NWORD = TW / 64;
   constexpr int ROWS = TILE_H / kTileBlockWaves;
@@ -868,33 +875,48 @@ __global__ __launch_bounds__(64 * kTileBlockWaves) void k_tile_block(TileArgs a)
     while (left) {
       const Visits v = visits_of<NWORD, ROWS, sizeof(T) == 8>(q, u, (left >> lane) & 1ull, left, s_x[wave]);
       if (!v.n) break;
-      uint32_t bits[kAhead<T>];
-      load_bits(a, v, 0u, bits, lane);
-      if constexpr (BARE) {
-        if (any_bare(v, lane)) {
-          auto desc_of = [&](int b) {
-            const uint64_t at = (uint64_t)d;
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, b);
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), b);
-            return load_desc((const RZ_CONST ItemDesc*)((uint64_t)lo | ((uint64_t)hi << 32)));
-          };
-          bare_visits<NWORD, ROWS>(a, u, v, s_edge[wave], lane, desc_of, [&](uint32_t k, uint32_t y) __attribute__((always_inline)) {
-            with_fun(J.fun, [&](auto fun) __attribute__((always_inline)) {
-              fold_visit<T, decltype(fun)::value, ROWS>(a, u, p, v, k, y, burns);
-            });
-          });
-          continue;
+      uint32_t bits[BARE == 2 ? 1 : kAhead<T>];
+      if (BARE < 2) load_bits(a, v, 0u, bits, lane);
+      // items without masks are folded one visit after the other, through the
+      // same code (a second copy of it cost registers)
+      const bool bare = BARE == 2 || (BARE && any_bare(v, lane));
+      uint64_t words = 0ull;  // the row words of the item in lane `at`
+      int at = -1, wlo = 0;
+      uint32_t k = 0, end = v.n;
+      do {
+        if (bare) {
+          int l = lane;
+          asm volatile("" : "+v"(l));  // (what is computed of it is not kept in registers from before the loop)
+          const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)v.info, (int)k);
+          if (BARE == 2 || info >> 31) {
+            const int item = __builtin_amdgcn_readlane((int)v.item, (int)k);
+            if (NWORD == 1 || item != at) {
+              const uint64_t da = (uint64_t)d;
+              const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)da, item);
+              const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(da >> 32), item);
+              words = edge_words<NWORD, ROWS>(a, load_desc((const RZ_CONST ItemDesc*)((uint64_t)lo | ((uint64_t)hi << 32))), u,
+                                              s_edge[BARE ? wave : 0], l, wlo);
+              at = item;
+            }
+            bits[0] = word_bits<ROWS>(words, (int)(info & 3u) - wlo, l) << (u.Rw & 15);
+          } else {
+            uint32_t one[1];
+            load_bits(a, v, k, one, l);
+            bits[0] = one[0];
+          }
+          end = k + 1u;
         }
-      }
-      switch (J.fun) {
-        case 0: fold_visits<T, 0, ROWS>(a, u, p, v, bits, lane, burns); break;
-        case 1: fold_visits<T, 1, ROWS>(a, u, p, v, bits, lane, burns); break;
-        case 2: fold_visits<T, 2, ROWS>(a, u, p, v, bits, lane, burns); break;
-        case 3: fold_visits<T, 3, ROWS>(a, u, p, v, bits, lane, burns); break;
-        case 4: fold_visits<T, 4, ROWS>(a, u, p, v, bits, lane, burns); break;
-        case 5: fold_visits<T, 5, ROWS>(a, u, p, v, bits, lane, burns); break;
-        default: fold_visits<T, 6, ROWS>(a, u, p, v, bits, lane, burns); break;
-      }
+        switch (J.fun) {
+          case 0: fold_visits<T, 0, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          case 1: fold_visits<T, 1, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          case 2: fold_visits<T, 2, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          case 3: fold_visits<T, 3, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          case 4: fold_visits<T, 4, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          case 5: fold_visits<T, 5, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+          default: fold_visits<T, 6, ROWS>(a, u, p, v, k, end, bits, lane, burns); break;
+        }
+        k = end;
+      } while (k < v.n);
     }
   };
   if (!J.scan) {
