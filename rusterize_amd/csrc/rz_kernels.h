@@ -279,10 +279,9 @@ constexpr unsigned long long kItemFarBit = 1ull << 62;
 // Coverage masks of a kItemMask item: strip k (rows from (r0 / 16 + k) * 16)
 // and word w (columns (c0 / 64 + w) * 64 .. + 63) hold one block of 128 bytes
 // at masks[(mask + k * nw + w) * 16], nw = (c1 - 1) / 64 - c0 / 64 + 1: for
-// each column the bits of its 16 rows, column c at 16-bit element
-// mask_element(c).  A wave whose lanes stand for columns reads a block with
+// each column the bits of its 16 rows, column c at 16-bit element c.  A wave
+// whose lanes stand for columns reads a block with
 // one 2-byte load per lane.
-__host__ __device__ inline int32_t mask_element(int32_t c) { return (c & 15) * 4 + (c >> 4); }
 __host__ __device__ inline int32_t mask_row_words(int32_t c0, int32_t c1) { return ((c1 - 1) >> 6) - (c0 >> 6) + 1; }
 __host__ __device__ inline int32_t mask_strip_count(int32_t r0, int32_t r1) { return (r1 - 1) / 16 - r0 / 16 + 1; }
 
@@ -323,9 +322,12 @@ struct InitArgs {
   }
 };
 
-// k_cover's work, listed by k_item_desc.  A unit keeps the toggle words of
-// its rows in LDS (a row's words padded to an odd count against bank
-// conflicts, one more for the rightmost crossing of a kItemOddRows item):
+// k_cover's work, listed by k_item_desc.  A unit keeps toggles in LDS: those of
+// a wave in the order of the mask blocks, a word for four columns of a strip (a
+// strip's words padded by one against bank conflicts, 16 more for the rightmost
+// crossings and the parities of a kItemOddRows item's rows); those of a
+// workgroup row by row, a word for 64 columns (padded to an odd count, one more
+// for a row's rightmost crossing; see CoverWave::cross for why):
 //   small  items of at most 64 vertices whose words fit kCoverWave, as many
 //          to a wave as fit together;
 //   wave   items of at most kCoverBlockNv vertices (a few chunks of 64, so
@@ -343,28 +345,33 @@ constexpr int kCoverBlockNv = 320;
 // chunks of 64 vertices (see Chunks).  A ring of two chunks is read whole.
 constexpr int kChunkNv = 128;
 struct CoverWindows {
-  int32_t ww, stride, strips;  // mask words, padded words and strips of a window
+  int32_t ww, stride, strips;  // mask words across, LDS words per strip and strips of a window
   int32_t ncw, n;              // windows across, windows in all
 };
-__host__ __device__ inline CoverWindows cover_windows(int32_t ns, int32_t nw, bool odd, int32_t words) {
+// LDS words per strip (`rows`: row by row).
+__host__ __device__ constexpr int32_t cover_stride(int32_t ww, bool odd, bool rows) {
+  return rows ? 16 * ((ww + (odd ? 1 : 0)) | 1) : 16 * ww + (odd ? 17 : 1);
+}
+__host__ __device__ inline CoverWindows cover_windows(int32_t ns, int32_t nw, bool odd, bool block) {
+  const int32_t words = block ? kCoverBlock : kCoverWave;
   CoverWindows c;
   c.ww = nw < words / 16 - 2 ? nw : words / 16 - 2;
-  c.stride = (c.ww + (odd ? 1 : 0)) | 1;
-  if (c.ww == nw && (int64_t)16 * c.stride * ns <= words) {  // (no divisions)
+  c.stride = cover_stride(c.ww, odd, block);
+  if (c.ww == nw && (int64_t)c.stride * ns <= words) {  // (no divisions)
     c.strips = ns;
     c.ncw = c.n = 1;
     return c;
   }
-  c.strips = words / (16 * c.stride);
+  c.strips = words / c.stride;
   if (c.strips > ns) c.strips = ns;
   c.ncw = (nw + c.ww - 1) / c.ww;
   c.n = c.ncw * ((ns + c.strips - 1) / c.strips);
   return c;
 }
-// The LDS words of a unit whose raster row R0 is at word `first`: those of row
-// r start at cover_word(cover_origin(first, R0, stride), r, stride).  Unsigned,
-// since the products pass 2^31 on rasters of some million rows (a signed
-// overflow would not be a constant below).
+// The LDS words of a unit whose raster row (or strip) R0 is at word `first`:
+// those of row (strip) r start at cover_word(cover_origin(first, R0, stride), r,
+// stride).  Unsigned, since the products pass 2^31 on rasters of some million
+// rows (a signed overflow would not be a constant below).
 __host__ __device__ constexpr uint32_t cover_origin(uint32_t first, int32_t R0, int32_t stride) {
   return first - (uint32_t)R0 * (uint32_t)stride;
 }

@@ -346,9 +346,9 @@ __device__ inline bool assign_cover(const CoverLists& c, bool poly, const ItemDe
     const int32_t ns = mask_strip_count(d.r0, d.r1), nw = mask_row_words(d.c0, d.c1);
     const bool odd = (d.flags & kItemOddRows) != 0;
     mu = (uint64_t)ns * (uint64_t)nw;
-    if (d.nv <= 64 && !odd && (uint64_t)ns * 16u * (uint64_t)(nw | 1) <= (uint64_t)kCoverWave) small = true;
-    else if (d.nv <= kCoverBlockNv) n[1] = (uint32_t)cover_windows(ns, nw, odd, kCoverWave).n;
-    else n[2] = (uint32_t)cover_windows(ns, nw, odd, kCoverBlock).n;
+    if (d.nv <= 64 && !odd && (int64_t)ns * cover_stride(nw, false, false) <= kCoverWave) small = true;
+    else if (d.nv <= kCoverBlockNv) n[1] = (uint32_t)cover_windows(ns, nw, odd, false).n;
+    else n[2] = (uint32_t)cover_windows(ns, nw, odd, true).n;
   }
   if (LIST) n[0] = small ? 1u : 0u;
   own = !LIST && n[1] && n[1] <= (uint32_t)kCoverOwn;

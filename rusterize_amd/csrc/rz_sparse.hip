@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void k_sp_polys(SparseArgs a, uint64_t n_units
                         cw.cap <= ((uint64_t)1 << 34);
     const uint64_t* cbits = filter ? a.bits + a.bit_base[p] : nullptr;
     const uint16_t* m = reinterpret_cast<const uint16_t*>(a.masks + ((uint64_t)d.mask + (uint64_t)k * (uint64_t)nw) * 16u) +
-                        mask_element(lane);
+                        lane;
     const int32_t Rw = ((d.r0 >> 4) + k) * WAVE_ROWS, C = (d.c0 >> 6) * 64;
     uint64_t o = EMIT ? a.toff[u] : 0, n = 0;
     uint32_t block[kSpBlocks];

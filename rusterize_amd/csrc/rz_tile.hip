@@ -5,29 +5,72 @@
 
 namespace rzk {
 
-// A strip's row words, row i's 64 columns in lane i of each 16, to
-// mask_element's order: 16-bit element j of lane i gets the rows' bits of
-// column 16 j + i.
-__device__ inline uint64_t transpose16(uint64_t x, int lane) {
+// Inclusive prefix parity over the 64 columns of a mask block of toggles, its
+// word i (columns 4 i .. 4 i + 3, 16 rows' bits each) in lane i of 16: `carry`
+// holds the parities of the block's left neighbours (twice) and gets its own.
+__device__ inline uint2 block_parity(uint2 x, uint32_t& carry) {
+  x.x ^= x.x << 16;
+  x.y ^= x.y << 16;
+  x.y ^= __builtin_amdgcn_perm(x.x, x.x, 0x03020302u);  // (the high half, twice)
+  uint32_t t = __builtin_amdgcn_perm(x.y, x.y, 0x03020302u);
+  t ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x111, 0xF, 0xF, true);  // row_shr:1, 2, 4, 8
+  t ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x112, 0xF, 0xF, true);
+  t ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x114, 0xF, 0xF, true);
+  t ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x118, 0xF, 0xF, true);
+  const uint32_t left = carry ^ (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x111, 0xF, 0xF, true);
+  carry ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x15F, 0xF, 0xF, true);  // row_newbcast:15
+  return make_uint2(x.x ^ left, x.y ^ left);
+}
+
+// Row words keep column 4 i + j of 64 at bit 16 j + i, so that the transposition
+// of 16 rows' words (below) leaves a mask block's word i in lane i.
+// Inclusive prefix parity over a row word's columns, `carry` (0 or ~0) before
+// them: that of the sums of four columns, then column by column.
+__device__ inline uint64_t row_parity(uint64_t x, uint32_t& carry) {
+  uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
+  uint32_t t = lo ^ hi;
+  t = (t ^ (t >> 16)) & 0xFFFFu;
+  t ^= t << 1;
+  t ^= t << 2;
+  t ^= t << 4;
+  t ^= t << 8;
+  const uint32_t left = __builtin_amdgcn_perm(t << 1, t << 1, 0x01000100u) ^ carry;  // (the low half, twice)
+  carry ^= 0u - ((t >> 15) & 1u);
+  lo ^= lo << 16;
+  hi ^= hi << 16;
+  hi ^= __builtin_amdgcn_perm(lo, lo, 0x03020302u);
+  return (uint64_t)(lo ^ left) | ((uint64_t)(hi ^ left) << 32);
+}
+// The columns below n of a row word.
+__device__ inline uint64_t row_below(int64_t n) {
+  uint64_t m = 0ull;
+  for (int j = 0; j < 4; ++j) {
+    const int64_t k = (n - j + 3) >> 2;
+    m |= (uint64_t)(k <= 0 ? 0u : (k >= 16 ? 0xFFFFu : ((1u << k) - 1u))) << (16 * j);
+  }
+  return m;
+}
+// Row i's word in lane i of each 16: lane i gets word i of the mask block.
+__device__ inline uint64_t block_word(uint64_t x, int lane) {
   return (uint64_t)transpose16x2((uint32_t)x, lane) | ((uint64_t)transpose16x2((uint32_t)(x >> 32), lane) << 32);
 }
 
 // An item (or a window of one) whose toggle words are in LDS.
 struct __align__(16) CoverItem {
-  uint32_t A;         // the words of raster row r start at cover_word(A, r, stride)
+  uint32_t A;         // the words of strip (workgroups: row) r start at cover_word(A, r, stride)
   int32_t stride;
   int32_t W0, wid;    // first column and columns
   int32_t R0, R1;     // raster rows [R0, R1)
   int64_t lv;         // edge e of the unit starts at local vertex lv + e
   uint32_t mask;      // ItemDesc::mask
   uint32_t row0;      // rows of the unit's items before this one
-  uint32_t base, pad; // word of its first row
+  uint32_t base, pad; // word of its first strip
   // The windows of a whole item, its rows and LDS words.
   __device__ void set_box(int32_t r0, int32_t r1, int32_t c0, int32_t c1, uint32_t& rows, uint32_t& words) {
     const int32_t ww = mask_row_words(c0, c1);
     rows = (uint32_t)mask_strip_count(r0, r1) * 16u;
-    stride = ww | 1;
-    words = rows * (uint32_t)stride;
+    stride = cover_stride(ww, false, false);
+    words = (rows >> 4) * (uint32_t)stride;
     W0 = (c0 >> 6) * 64;
     wid = ww * 64;
     R0 = (r0 >> 4) * 16;
@@ -71,30 +114,46 @@ struct CoverWave {
     return at;
   }
 
-  // The toggles of edges [0, n_e) of the items in `items`, taken in
-  // chunks of 64.  `many`: the lane's item (own) has the edges from e0 of the
-  // one chunk; else all are item 0's.  AHEAD: those chunks of item 0 alone
-  // that `chunks` hands out, its first `skew` edges before the item's.
-  template <bool AHEAD>
-  __device__ __attribute__((always_inline)) void toggles(const RZ_CONST JobDev& J, bool many, bool own, uint32_t e0,
+  // The toggles of n_e edges, taken in chunks of 64.  MANY: of the items in
+  // `items`, the lane's (own) from edge e0 of the one chunk on; else of `one`
+  // (in scalar registers: a read of LDS less for every crossing).  AHEAD: those
+  // chunks of it that `chunks` hands out, its first `skew` edges before the
+  // item's.
+  template <bool AHEAD, bool MANY>
+  __device__ __attribute__((always_inline)) void toggles(const RZ_CONST JobDev& J, const CoverItem& one, bool own, uint32_t e0,
                                                          uint32_t n_e, Chunks<true>* chunks, uint32_t skew, bool odd) const {
     const double ncols_f = (double)J.ncols;
     const bool sx = J.xres != 1.0, sy = J.yres != 1.0;  // (v / 1.0 is v)
     auto px_x = [&](double X) { return isnan(X) ? X : (sx ? (X - J.xmin) / J.xres : X - J.xmin); };
     auto px_y = [&](double Y) { return isnan(Y) ? Y : (sy ? (J.ymax - Y) / J.yres : J.ymax - Y); };
     // the crossing of row r by the edge x0, y0, dxdy of an item
-    auto cross = [&](const CoverItem* it, int32_t r, double x0, double y0, double dxdy) __attribute__((always_inline)) {
-      const int32_t W0 = it->W0, wid = it->wid;
+    auto cross = [&](const CoverItem& it, int32_t r, double x0, double y0, double dxdy) __attribute__((always_inline)) {
+      const int32_t W0 = it.W0, wid = it.wid;
       const double x = x0 + (((double)r + 0.5) - y0) * dxdy;
       const int32_t col = span_col(x, ncols_f);
       const int32_t rel = max(col - W0, 0);
-      uint64_t* row = tog + cover_word(it->A, r, it->stride);
+      if constexpr (AHEAD) {
+        // (row by row: the many short edges of a long ring would otherwise
+        // flip bits of the same few words, one after the other: 24 jobs of
+        // rings of up to 4,096 vertices 1.13 ms, row by row 1.06)
+        uint32_t* row = reinterpret_cast<uint32_t*>(tog + cover_word(it.A, r, it.stride));
+        if (rel < wid)
+          __hip_atomic_fetch_xor(row + ((rel >> 6) * 2 + ((rel >> 1) & 1)), 1u << ((rel & 1) * 16 + ((rel >> 2) & 15)),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        // the rightmost crossing of a row matters only with an odd count
+        if (odd)
+          __hip_atomic_fetch_max(row + (wid >> 5), (uint32_t)col + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return;
+      }
+      uint32_t* strip = reinterpret_cast<uint32_t*>(tog + cover_word(it.A, r >> 4, it.stride));
       if (rel < wid)
-        __hip_atomic_fetch_xor(row + (rel >> 6), 1ull << (rel & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      // the rightmost crossing of a row matters only with an odd count
-      if (odd)
-        __hip_atomic_fetch_max(reinterpret_cast<uint32_t*>(row + (wid >> 6)), (uint32_t)col + 1u, __ATOMIC_RELAXED,
+        __hip_atomic_fetch_xor(strip + (rel >> 1), 1u << ((rel & 1) * 16 + (r & 15)), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (odd) {
+        uint32_t* end = strip + (wid >> 1) + (r & 15) * 2;
+        __hip_atomic_fetch_max(end, (uint32_t)col + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_xor(end + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
     };
     // (an item's next vertices are loaded while this chunk's edges are built)
     uint64_t vi = 0;
@@ -111,14 +170,15 @@ struct CoverWave {
       uint32_t c = 0;
       more = chunks->next(c);
       cb = c * 64u - skew;
-      if (more && cb + (uint32_t)lane < n_e) load(items->lv + (int64_t)(cb + (uint32_t)lane));
+      if (more && cb + (uint32_t)lane < n_e) load(one.lv + (int64_t)(cb + (uint32_t)lane));
     };
     if (AHEAD) advance();
     for (; AHEAD ? more : cb < n_e; cb += AHEAD ? 0u : 64u) {
       const uint32_t e = cb + (uint32_t)lane;
       uint32_t before = 0;
-      const uint32_t k = many ? owner(own, e0, 0u, before) : 0u;
-      if (!AHEAD && e < n_e) load(items[k].lv + (int64_t)e);
+      const uint32_t k = MANY ? owner(own, e0, 0u, before) : 0u;
+      const CoverItem& it = MANY ? items[k] : one;
+      if (!AHEAD && e < n_e) load(it.lv + (int64_t)e);
       const uint64_t vi0 = vi;
       const double2 p0 = p, q0 = q;
       if (AHEAD) advance();
@@ -126,12 +186,11 @@ struct CoverWave {
       int32_t a0 = 0;
       uint32_t span = 0;
       if (e < n_e) {
-        const CoverItem* it = &items[k];
         double xb, yb;
         bool o = false;
         if ((vi0 & VI_HAS_NEXT) && ring_edge(px_x(p0.x), px_y(p0.y), px_x(q0.x), px_y(q0.y), J.nrows, false, ee, xb, yb, o)) {
-          a0 = max(ee.ystart, it->R0);
-          span = (uint32_t)max(0, min(ee.yend, it->R1) - a0);
+          a0 = max(ee.ystart, it.R0);
+          span = (uint32_t)max(0, min(ee.yend, it.R1) - a0);
           // (an edge of an infinite or NaN end has its slope already: its
           // crossings are pinned or come from that slope)
           const double inf = __builtin_inf();
@@ -176,7 +235,7 @@ struct CoverWave {
             uint64_t rk;
             __builtin_memcpy(&rk, src + 3, 8);
             const int32_t r = (int32_t)(b0 + c + (uint32_t)lane) + (int32_t)(uint32_t)rk;
-            cross(&items[many ? (int)(rk >> 32) : 0], r, src[0], src[1], src[2]);
+            cross(MANY ? items[rk >> 32] : one, r, src[0], src[1], src[2]);
           }
         }
         wave_sync();
@@ -185,26 +244,48 @@ struct CoverWave {
     }
   }
 
+  // A strip's toggles (ww blocks of 16 words from `strip`, cleared as they are
+  // read) into mask blocks out, out + 16, ..., by 16 neighbouring lanes, a word
+  // of each block to a lane (k, of 16; out: the lane's word of a block).  odd:
+  // each row's rightmost crossing + 1 and parity lie after its words; a row of
+  // odd parity covers nothing from that crossing on, as if it were there twice
+  // (W0: the strip's first column).
+  __device__ __attribute__((always_inline)) void finish_strip(uint64_t* strip, int32_t k, int32_t ww, uint64_t* out,
+                                                              bool odd, int32_t W0) const {
+    if (odd) {
+      const uint64_t end = strip[16 * ww + k];
+      strip[16 * ww + k] = 0ull;
+      const int32_t rel = max((int32_t)((uint32_t)end - 1u) - W0, 0);
+      if ((end >> 32) && rel < 64 * ww)
+        __hip_atomic_fetch_xor(reinterpret_cast<uint32_t*>(strip) + (rel >> 1), 1u << ((rel & 1) * 16 + k),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      wave_sync();
+    }
+    uint2* p = reinterpret_cast<uint2*>(strip + k);
+    uint32_t carry = 0u;
+    for (int32_t w = 0; w < ww; ++w) {
+      const uint2 x = block_parity(p[16 * w], carry);
+      p[16 * w] = make_uint2(0u, 0u);
+      reinterpret_cast<uint2*>(out)[16 * w] = x;
+    }
+  }
+
   // One row's toggles (ww words from `row`, cleared as they are read), the
   // rows of a strip in 16 neighbouring lanes, into mask blocks out, out + 16,
-  // ... (out: the lane's word of a block); odd: the row's rightmost crossing
-  // + 1 lies after its words, W0 is its first column.
+  // ... (out: the lane's word of a block); odd: the row's rightmost crossing + 1
+  // lies after its words, W0 is its first column.
   __device__ __attribute__((always_inline)) void finish_row(uint64_t* row, int32_t ww, uint64_t* out, bool odd, int32_t W0) const {
     int64_t lim = INT_MAX;  // columns of the window left of the rightmost crossing
     if (odd) {
       lim = (int64_t)(uint32_t)row[ww] - 1 - (int64_t)W0;
       row[ww] = 0ull;
     }
-    uint64_t carry = 0ull;
+    uint32_t carry = 0u;
     for (int32_t w = 0; w < ww; ++w) {
-      uint64_t x = prefix_xor64(row[w]) ^ carry;
+      uint64_t x = row_parity(row[w], carry);
       row[w] = 0ull;
-      carry = 0ull - (x >> 63);
-      if (odd) {
-        const int64_t l = lim - 64 * (int64_t)w;
-        x &= l <= 0 ? 0ull : (l >= 64 ? ~0ull : ((1ull << l) - 1ull));
-      }
-      out[(uint64_t)w * 16u] = transpose16(x, lane);
+      if (odd) x &= row_below(lim - 64 * (int64_t)w);
+      out[(uint64_t)w * 16u] = block_word(x, lane);
     }
   }
 
@@ -232,23 +313,23 @@ struct CoverWave {
       if (own) {
         CoverItem x = it;
         x.base = base + wi - words;
-        x.A = cover_origin(x.base, x.R0, x.stride);
+        x.A = cover_origin(x.base, x.R0 >> 4, x.stride);
         x.R1 = min(x.R1, J.nrows);
         x.lv -= J.v_base + (int64_t)(ei - nv);
         x.row0 = ri - rows;
         items[__popcll(unit & ((1ull << lane) - 1ull))] = x;
       }
       wave_sync();
-      toggles<false>(J, true, own, ei - nv, n_e, nullptr, 0u, false);
+      toggles<false, true>(J, it, own, ei - nv, n_e, nullptr, 0u, false);
       uint32_t before = 0;
       for (uint32_t c = 0; c < n_rows; c += 64u) {
         const uint32_t at = owner(own, ri - rows, c, before);
         if (c + (uint32_t)lane < n_rows) {
           const CoverItem x = items[at];
           const uint32_t r = c + (uint32_t)lane - x.row0;
-          finish_row(tog + x.base + r * (uint32_t)x.stride, x.wid >> 6,
-                     masks + ((uint64_t)x.mask + (uint64_t)(r >> 4) * (uint64_t)(x.wid >> 6)) * 16u + (uint64_t)(r & 15u),
-                     false, 0);
+          finish_strip(tog + x.base + (r >> 4) * (uint32_t)x.stride, (int32_t)(r & 15u), x.wid >> 6,
+                       masks + ((uint64_t)x.mask + (uint64_t)(r >> 4) * (uint64_t)(x.wid >> 6)) * 16u + (uint64_t)(r & 15u),
+                       false, 0);
         }
       }
       wave_sync();
@@ -261,23 +342,19 @@ struct CoverWave {
                                                         int32_t c0, int32_t c1, int64_t vbeg, uint32_t nv, bool odd,
                                                         uint32_t mask, int32_t t) const {
     const int32_t ns = mask_strip_count(r0, r1), nw = mask_row_words(c0, c1);
-    const CoverWindows win = cover_windows(ns, nw, odd, BLOCK ? kCoverBlock : kCoverWave);
+    const CoverWindows win = cover_windows(ns, nw, odd, BLOCK);
     const int32_t row = win.n == 1 ? 0 : t / win.ncw;
     const int32_t s0 = row * win.strips, w0 = (t - row * win.ncw) * win.ww;
     const int32_t ww = min(win.ww, nw - w0), n_rows = min(win.strips, ns - s0) * 16;
     const int32_t first = BLOCK ? 0 : (int32_t)base, R0 = ((r0 >> 4) + s0) * 16, W0 = ((c0 >> 6) + w0) * 64;
-    if (lane == 0) {
-      CoverItem it{};
-      it.A = cover_origin((uint32_t)first, R0, win.stride);
-      it.stride = win.stride;
-      it.W0 = W0;
-      it.wid = ww * 64;
-      it.R0 = R0;
-      it.R1 = min(R0 + n_rows, J.nrows);
-      it.lv = vbeg - J.v_base;
-      items[0] = it;
-    }
-    wave_sync();
+    CoverItem it{};
+    it.stride = BLOCK ? win.stride >> 4 : win.stride;
+    it.A = cover_origin((uint32_t)first, BLOCK ? R0 : R0 >> 4, it.stride);
+    it.W0 = W0;
+    it.wid = ww * 64;
+    it.R0 = R0;
+    it.R1 = min(R0 + n_rows, J.nrows);
+    it.lv = vbeg - J.v_base;
     if constexpr (BLOCK) {  // the waves take the window's chunks in turn
       // (an item of one window needs them all, from its own first vertex on)
       const bool all = win.n == 1;
@@ -285,17 +362,17 @@ struct CoverWave {
       static_assert(kCoverBlockWaves == 4, "every fourth chunk is a wave's");
       Chunks<true> chunks(all ? nullptr : chunk_rows + (vbeg >> 6), (nv + skew + 63u) >> 6, R0, R0 + n_rows,
                     0x1111111111111111ull << wave_index(), lane);
-      toggles<true>(J, false, false, 0u, nv, &chunks, skew, odd);
+      toggles<true, false>(J, it, false, 0u, nv, &chunks, skew, odd);
     } else {
-      toggles<false>(J, false, false, 0u, nv, nullptr, 0u, odd);
+      toggles<false, false>(J, it, false, 0u, nv, nullptr, 0u, odd);
     }
     if (BLOCK) __syncthreads();
     else wave_sync();
-    for (int32_t r = BLOCK ? (int32_t)threadIdx.x : lane; r < n_rows; r += BLOCK ? 64 * kCoverBlockWaves : 64)
-      finish_row(tog + first + r * win.stride, ww,
-                 masks + ((uint64_t)mask + (uint64_t)(s0 + (r >> 4)) * (uint64_t)nw + (uint64_t)w0) * 16u +
-                     (uint64_t)(r & 15),
-                 odd, W0);
+    for (int32_t r = BLOCK ? (int32_t)threadIdx.x : lane; r < n_rows; r += BLOCK ? 64 * kCoverBlockWaves : 64) {
+      uint64_t* out = masks + ((uint64_t)mask + (uint64_t)(s0 + (r >> 4)) * (uint64_t)nw + (uint64_t)w0) * 16u + (uint64_t)(r & 15);
+      if (BLOCK) finish_row(tog + r * (win.stride >> 4), ww, out, odd, W0);
+      else finish_strip(tog + first + (r >> 4) * win.stride, r & 15, ww, out, odd, W0);
+    }
     if (BLOCK) __syncthreads();
     else wave_sync();
   }
@@ -308,12 +385,15 @@ struct CoverWave {
 // coordinates, 64 at a time; the (edge, row) crossings of those edges are
 // then laid out one per lane (an edge of a few rows and one of hundreds cost
 // what they cross, where a lane per edge would wait for the longest one);
-// every crossing flips its toggle bit in LDS (order-free), at bit 0 when it
-// lies left of the window; and a lane per row turns the toggles into
-// coverage (inclusive prefix parity across its words, see the note above
-// row_coverage_word), the 16 lanes of a strip transpose it to the order of
-// the mask blocks and store it.  Small items are packed: as many as
-// have at most 64 edges and a wave's LDS words together form one unit.
+// every crossing flips its toggle bit in LDS (order-free), in column 0 when it
+// lies left of the window; and the 16 lanes of a strip turn its toggles into
+// coverage (inclusive prefix parity across the columns, see the note above
+// row_coverage_word) and store it as mask blocks.  A wave's toggles are in the
+// blocks' own order, so a word of them (4 columns of 16 rows) takes about 20
+// instructions (row by row, with a transposition, 66: 1.1 M small polygons on
+// 40000 x 40000 took 0.83 ms, bound by vector issue, and take 0.65).  Small
+// items are packed: as many as have at most 64 edges and a wave's LDS words
+// together form one unit.
 // Bound by the latency of its dependent loads and LDS round trips (vector
 // issue is busy about half of the time), so LDS is sized for 6 waves per
 // SIMD, the block list's next edges are loaded ahead and its entries handed
@@ -331,7 +411,7 @@ __global__ __launch_bounds__(64 * (BLOCK ? kCoverBlockWaves : 4)) void k_cover(C
   __shared__ __align__(16) double s_edge[NW][64][4];  // x0, y0, dxdy, (row offset, item)
   __shared__ CoverItem s_item[NW][RUN];
   __shared__ uint64_t s_start[NW][kStartWords];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = wave_index(), lane = threadIdx.x & 63;
   const RZ_CONST JobDev* jobs_c = as_const(a.jobs);
   const RZ_CONST ItemDesc* desc_c = as_const(a.desc);
   const CoverWave cw{s_tog, s_edge[wave], s_item[wave], s_start[wave], (uint32_t)(wave * kCoverWave), lane, a.chunk_rows};
@@ -403,7 +483,7 @@ __global__ __launch_bounds__(64 * kItemsWaves) void k_items(ItemsArgs a) {
   __shared__ CoverItem s_item[kItemsWaves][1];
   __shared__ uint64_t s_start[kItemsWaves][kStartWords];
   __shared__ ItemBox s_box[kItemsWaves];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = wave_index(), lane = threadIdx.x & 63;
   const uint32_t base = (uint32_t)(wave * kCoverWave);
   const CoverWave cw{s_tog, s_edge[wave], s_item[wave], s_start[wave], base, lane, nullptr};
   const int64_t i = (int64_t)blockIdx.x * kItemsWaves + wave;
@@ -446,7 +526,7 @@ __global__ __launch_bounds__(64 * kItemsWaves) void k_items(ItemsArgs a) {
   if (lane == 0) a.d.desc[i] = d;
   if (!__any(ok && (small || own))) return;
   const bool odd = (d.flags & kItemOddRows) != 0;
-  const int32_t n_win = (int32_t)cover_windows(mask_strip_count(d.r0, d.r1), mask_row_words(d.c0, d.c1), odd, kCoverWave).n;
+  const int32_t n_win = (int32_t)cover_windows(mask_strip_count(d.r0, d.r1), mask_row_words(d.c0, d.c1), odd, false).n;
   const uint32_t mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.mask);
   for (int32_t t = 0; t < n_win; ++t)
     cw.window<false>(J, a.masks, d.r0, d.r1, d.c0, d.c1, d.vbeg, (uint32_t)d.nv, odd, mask, t);

@@ -191,7 +191,7 @@ __device__ inline uint32_t column_bits(const TileArgs& a, const ItemDesc& d, con
   if (!(d.flags & kItemMask))
     return edge_bits(a.edges, d.vbeg, d.nv, a.chunk_rows, u.Rw, u.strip_r1, u.C0 + 64 * w, u.ncols, (RZ_LDS PolyEdge*)stage, lane);
   const uint64_t* p = a.masks + ((uint64_t)d.mask + (uint64_t)((u.Rw >> 4) - (d.r0 >> 4)) * (uint64_t)nw + (uint64_t)wi) * 16u;
-  return reinterpret_cast<const uint16_t*>(p)[mask_element(lane)];
+  return reinterpret_cast<const uint16_t*>(p)[lane];
 }
 
 // Writes a strip once: lane l's chunk of PPC pixels in rows
@@ -551,7 +551,7 @@ constexpr int kAhead = sizeof(T) == 8 ? 3 : 2;
 // last one's again).
 template <int N>
 __device__ inline void load_bits(const TileArgs& a, const Visits& v, uint32_t k, uint32_t (&bits)[N], int lane) {
-  const uint16_t* base = reinterpret_cast<const uint16_t*>(a.masks) + mask_element(lane);
+  const uint16_t* base = reinterpret_cast<const uint16_t*>(a.masks) + lane;
 #pragma unroll
   for (int g = 0; g < N; ++g) {
     const uint32_t blk = (uint32_t)__builtin_amdgcn_readlane((int)v.blk, (int)min(k + (uint32_t)g, v.n - 1u));
