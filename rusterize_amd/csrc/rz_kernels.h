@@ -115,6 +115,7 @@ struct JobDev {
   const int64_t* item_vbeg;  // [ni + 1] local vertex range of every item
   int64_t v_base, i_base, nv, ni;
   double xmin, ymax, xres, yres;
+  double xinv, yinv;         // 1 / xres, 1 / yres where exact (powers of two), else 0 (to_pixel)
   int32_t nrows, ncols, ntx, nty;
   int32_t esz, tile_w;       // element size of the output dtype, tile width in pixels
   uint32_t tiles_per_layer, tile_base, n_tiles;

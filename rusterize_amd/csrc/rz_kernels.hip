@@ -205,9 +205,8 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a) {
     const bool closed = (vi & VI_CLOSED) != 0;
     const double rows = (double)J.nrows, cols = (double)J.ncols;
     // world -> pixel; a NaN coordinate stays that NaN (x86 semantics, x86_nan)
-    const bool sx = J.xres != 1.0, sy = J.yres != 1.0;  // (v / 1.0 is v; uniform)
-    auto px_x = [&](double X) { return isnan(X) ? X : (sx ? (X - J.xmin) / J.xres : X - J.xmin); };
-    auto px_y = [&](double Y) { return isnan(Y) ? Y : (sy ? (J.ymax - Y) / J.yres : J.ymax - Y); };
+    auto px_x = [&](double X) { return isnan(X) ? X : to_pixel(X - J.xmin, J.xres, J.xinv); };
+    auto px_y = [&](double Y) { return isnan(Y) ? Y : to_pixel(J.ymax - Y, J.yres, J.yinv); };
     const double x0 = px_x(X0);
     const double y0 = px_y(Y0);
     if (kind == 0) {  // polygon rings: extract_ring + PolyEdge::new

@@ -647,6 +647,12 @@ struct BatchCaps {
   uint64_t pairs, band_entries, band_edges, masks, units, at_words;
 };
 
+// 1 / r where that is a power of two far from the ends of the range, else 0.
+static double exact_reciprocal(double r) {
+  int e = 0;
+  return std::frexp(std::fabs(r), &e) == 0.5 && e > -1000 && e < 1000 ? 1.0 / r : 0.0;
+}
+
 // The device record of job j, whose vertex / item / tile ranges start at
 // v_base / i_base / t_base of its batch (J.scan is left 0); returns the
 // job's tile count (tiles per band x bands).
@@ -674,6 +680,8 @@ static uint64_t job_record(const rz_job& j, JobDev& J, int64_t v_base, int64_t i
   J.ymax = j.info.ymax;
   J.xres = j.info.xres;
   J.yres = j.info.yres;
+  J.xinv = exact_reciprocal(J.xres);
+  J.yinv = exact_reciprocal(J.yres);
   J.nrows = nrows;
   J.ncols = ncols;
   J.ntx = ntx;

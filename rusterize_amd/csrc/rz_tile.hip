@@ -123,9 +123,8 @@ struct CoverWave {
   __device__ __attribute__((always_inline)) void toggles(const RZ_CONST JobDev& J, const CoverItem& one, bool own, uint32_t e0,
                                                          uint32_t n_e, Chunks<true>* chunks, uint32_t skew, bool odd) const {
     const double ncols_f = (double)J.ncols;
-    const bool sx = J.xres != 1.0, sy = J.yres != 1.0;  // (v / 1.0 is v)
-    auto px_x = [&](double X) { return isnan(X) ? X : (sx ? (X - J.xmin) / J.xres : X - J.xmin); };
-    auto px_y = [&](double Y) { return isnan(Y) ? Y : (sy ? (J.ymax - Y) / J.yres : J.ymax - Y); };
+    auto px_x = [&](double X) { return isnan(X) ? X : to_pixel(X - J.xmin, J.xres, J.xinv); };
+    auto px_y = [&](double Y) { return isnan(Y) ? Y : to_pixel(J.ymax - Y, J.yres, J.yinv); };
     // the crossing of row r by the edge x0, y0, dxdy of an item
     auto cross = [&](const CoverItem& it, int32_t r, double x0, double y0, double dxdy) __attribute__((always_inline)) {
       const int32_t W0 = it.W0, wid = it.wid;
@@ -505,8 +504,8 @@ __global__ __launch_bounds__(64 * kItemsWaves) void k_items(ItemsArgs a) {
         const int64_t ln = min(lv + 1, J.nv - 1);
         const uint64_t vi = J.vert_info[lv];
         const double X0 = J.xy[2 * lv], Y0 = J.xy[2 * lv + 1], X1 = J.xy[2 * ln], Y1 = J.xy[2 * ln + 1];
-        auto px_x = [&](double X) { return isnan(X) ? X : (X - J.xmin) / J.xres; };
-        auto px_y = [&](double Y) { return isnan(Y) ? Y : (J.ymax - Y) / J.yres; };
+        auto px_x = [&](double X) { return isnan(X) ? X : to_pixel(X - J.xmin, J.xres, J.xinv); };
+        auto px_y = [&](double Y) { return isnan(Y) ? Y : to_pixel(J.ymax - Y, J.yres, J.yinv); };
         PolyEdge e;
         polygon_edge(vi, px_x(X0), px_y(Y0), px_x(X1), px_y(Y1), J, a.edges != nullptr, e, box, odd);
         if (a.edges) a.edges[J.v_base + lv] = e;

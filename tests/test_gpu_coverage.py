@@ -325,3 +325,57 @@ def test_strips_without_masks(rows, cols, n_layers, dtype, binning, monkeypatch)
         ref = oracle.rasterize(g, oracle.copy_info(info), dtype, fun, field=field, layer_of_geom=layers,
                                n_layers=n_layers, background=bg)
         assert_same(got, ref, f"{rows}x{cols}x{n_layers} {dtype} {fun} {binning}")
+
+
+def wide_rings(rows, cols, top):
+    """Rings of up to `top` vertices across the whole raster and past it, every
+    second one open, and small ones at the words' edges."""
+    rng = np.random.default_rng(cols)
+    rings = []
+    for k, nv in enumerate([4, 5, 63, 64, 300, 319, top, top]):
+        a = np.sort(rng.uniform(0, 2 * np.pi, nv))
+        r = rng.uniform(0.2, 1.0, nv)
+        p = np.stack([cols * (0.5 + 0.6 * r * np.cos(a)), rows * (0.5 + 0.8 * r * np.sin(a))], 1)
+        rings.append(p if k % 2 else np.concatenate([p, p[:1]]))
+    for w in range(0, cols, 320):
+        x, y = w + rng.uniform(-2, 2), rng.uniform(0, rows)
+        rings.append(np.array([[x, y], [x + 70, y + 3], [x + 9, y + 20.5], [x, y]]))
+    rvo = np.concatenate([[0], np.cumsum([len(r) for r in rings])])
+    n = len(rings)
+    return Geometry(np.arange(n + 1), np.zeros(n, np.int32), np.arange(n + 1), rvo, np.concatenate(rings))
+
+
+@pytest.mark.parametrize("binning,top", [("never", 319), ("never", 900), ("always", 319), ("always", 900)])
+@pytest.mark.parametrize("rows,cols", [(50, 26 * 64), (50, 26 * 64 + 1), (430, 64), (33, 238 * 64), (33, 238 * 64 + 1)])
+def test_windows_across_wide_items(rows, cols, binning, top, monkeypatch):
+    # items as wide as a wave's window (26 words of 64 columns; by rows 26
+    # strips of one word) or a workgroup's (238), and one word wider: carries
+    # from block to block, and the columns past a row's rightmost crossing
+    # where open rings leave an odd count
+    monkeypatch.setenv("RUSTERIZE_BINNING", binning)
+    monkeypatch.setenv("RUSTERIZE_WIDE", "always")
+    g = wide_rings(rows, cols, top)
+    info = _lib.raster_info(None, resolution=(1.0, 1.0), extent=(0, 0, cols, rows))
+    field = field_for("int32", g.n_geoms, seed=rows)
+    for fun in ("sum", "last"):
+        got = _lib.rasterize(g, info, "int32", fun, field, None, None, 1, 0)
+        ref = oracle.rasterize(g, oracle.copy_info(info), "int32", fun, field=field, background=0)
+        assert_same(got, ref, f"{rows}x{cols} {fun} {binning} {top}")
+
+
+@pytest.mark.parametrize("res", [(0.25, 0.25), (32.0, 0.5), (2.0 ** -1005, 2.0 ** -1005), (0.3, 30.0), (1.0, 0.1)])
+@pytest.mark.parametrize("binning", ["always", "never"])
+def test_resolutions(res, binning, monkeypatch):
+    # powers of two multiply by their exact reciprocal (far from the ends of
+    # the range), all others divide; the third has coordinates near the
+    # smallest normal numbers
+    monkeypatch.setenv("RUSTERIZE_BINNING", binning)
+    monkeypatch.setenv("RUSTERIZE_WIDE", "always")
+    rows, cols = 130, 321
+    g = polygons(rows, cols)
+    scaled = Geometry(g.geom_item_offsets, g.item_kind, g.item_ring_offsets, g.ring_vertex_offsets, g.xy * np.array(res))
+    info = _lib.raster_info(None, resolution=res, extent=(0, 0, cols * res[0], rows * res[1]))
+    field = field_for("float64", g.n_geoms, seed=5)
+    got = _lib.rasterize(scaled, info, "float64", "sum", field, None, None, 1, float("nan"))
+    ref = oracle.rasterize(scaled, oracle.copy_info(info), "float64", "sum", field=field, background=float("nan"))
+    assert_same(got, ref, f"{res} {binning}")
