@@ -355,7 +355,9 @@ rz_status rz_batch_graph_destroy(rz_batch_graph* graph);
  * is set and has no effect: all polygon coverage is precomputed).  rz_autotune
  * times every candidate on each job (reps timed runs each) and stores the
  * fastest for that job's class in a process-wide table that every later call
- * and batch uses; run it while no other rasterisation runs in the process.
+ * and batch uses; run it while no other rasterisation runs in the process.  A
+ * job whose launch has no work queue (polygons on few tiles) is not timed; its
+ * entry is in a class of its own (bit 9) that no launch reads.
  * rz_autotune_table lists the table (returns the entry count, fills up to
  * cap); rz_autotune_set adds or (0, 0) removes an entry. */
 rz_status rz_autotune(rz_context* ctx, const rz_job* jobs, int64_t n_jobs, int reps,

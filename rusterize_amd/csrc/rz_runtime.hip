@@ -567,7 +567,9 @@ inline int floor_log2_u64(uint64_t v) {
 }
 
 // Size class: bit 8 tile width (0: 64 px, 1: 256 px), bits 4-7 log4 of the
-// launch's tiles, bits 0-3 log2 of (items per tile + 1).
+// launch's tiles, bits 0-3 log2 of (items per tile + 1); bit 9: a launch
+// without a queue (k_tile_block), whose entry nothing reads.
+constexpr uint32_t kClassNoQueue = 1u << 9;
 uint32_t size_class(int tile_w, uint64_t tiles, uint64_t pairs) {
   const uint64_t t = std::max<uint64_t>(tiles, 1);
   const uint32_t tb = (uint32_t)std::min(15, floor_log2_u64(t) / 2);
@@ -1352,6 +1354,15 @@ extern "C" rz_status rz_autotune(rz_context* c, const rz_job* jobs, int64_t n_jo
       }
       st = run_batch(c, jobs + k, 1);  // warm-up (workspace)
       if (st == RZ_OK) st = rz_context_synchronize(c);
+      cls = size_class(tile_w((int)rz_dtype_size(jobs[k].dtype)), c->last_tiles, c->last_pairs);
+      // a workgroup per tile: all candidates are the same launch, and the
+      // fastest of them would be noise, set for larger launches of the class
+      const rz_device_geometry* dg = jobs[k].geometry;
+      if (st == RZ_OK && !dg->has_line && !dg->has_point && !jobs[k].all_touched && c->last_tiles <= kBlockTiles) {
+        cls |= kClassNoQueue;
+        best = Tuning{ch, kHeavy};
+        break;
+      }
       float ms = 0.f;
       if (st == RZ_OK && hipEventRecord(e0, c->stream) != hipSuccess) st = RZ_DEVICE_ERROR;
       for (int r = 0; r < reps && st == RZ_OK; ++r) st = run_batch(c, jobs + k, 1);
@@ -1363,7 +1374,6 @@ extern "C" rz_status rz_autotune(rz_context* c, const rz_job* jobs, int64_t n_jo
         best_ms = ms;
         best = Tuning{ch, kHeavy};
       }
-      cls = size_class(tile_w((int)rz_dtype_size(jobs[k].dtype)), c->last_tiles, c->last_pairs);
     }
     if (st == RZ_OK) {
       std::lock_guard<std::mutex> lk(ts.mu);

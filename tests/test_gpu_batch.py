@@ -411,3 +411,27 @@ def test_graph_replay_past_band_and_mask_capacities(ctx, wide, monkeypatch):
         d_field.free()
         out.free()
         dg.free()
+
+
+def test_autotuner_keeps_launches_without_a_queue_apart(ctx):
+    # polygons on at most 12,288 tiles take a workgroup per tile whatever the
+    # candidate, so the fastest of them would be noise: their entries are in
+    # classes (bit 9) that no launch reads; lines take their tiles from the queue
+    from rusterize_amd.device import autotune, autotune_clear, autotune_table
+    polys = Geometry.synth(1, 41, 300, 1000.0, 700.0, 3.0, 40.0)
+    xy = np.stack([np.linspace(0, 1000, 50), np.linspace(0, 700, 50)], 1)
+    line = Geometry([0, 1], np.array([1], np.int32), [0, 1], [0, 50], xy)
+    held = []
+    try:
+        for g, apart in ((polys, 1), (line, 0)):
+            autotune_clear()
+            dg, out = DeviceGeometry(ctx, g), DeviceBuffer(ctx, 700 * 1000 * 4)
+            d_field = DeviceBuffer.from_array(ctx, field_for("int32", g.n_geoms, seed=2))
+            held += [d_field, out, dg]
+            job = Job(dg, grid(1000, 700, 0, 0), "int32", "last", out, field=d_field, background=0)
+            assert autotune(ctx, [job], reps=1) == 1
+            assert [cls >> 9 for cls in autotune_table()] == [apart]
+    finally:
+        autotune_clear()
+        for h in held:
+            h.free()
