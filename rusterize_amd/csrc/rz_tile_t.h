@@ -653,10 +653,11 @@ __device__ __attribute__((always_inline)) inline void bare_visits(const TileArgs
 // pixels (a million polygons on 40000^2 float32 in 2 bands: 5.17 ms a call,
 // in 8 bands, about one item to a tile, 12.1; with 5 waves and 6 visits ahead
 // 5.24 and 14.3), 5 for 8-byte ones (24 uneven jobs 3.85 ms, with 4 waves
-// 4.04); 4 where more would spill.
+// 4.04), 3 for 2-byte ones (LineWriter's rows take the LDS of more); 4 where
+// more would spill.
 template <typename T, bool BARE>
 struct TileOccupancy {
-  static constexpr int value = sizeof(T) <= 2 || BARE ? 4 : (sizeof(T) == 4 ? 7 : 5);
+  static constexpr int value = sizeof(T) == 2 ? 3 : (sizeof(T) == 1 || BARE ? 4 : (sizeof(T) == 4 ? 7 : 5));
 };
 
 // Tile kernel of polygon-only groups, one launch per pixel-function group of
