@@ -349,9 +349,28 @@ __device__ inline void store_rows(const StripUnit& u, const Pixels<T, ROWS>& p, 
   T* out = (T*)u.J->out + ((uint64_t)u.layer * (uint64_t)u.nrows + (uint64_t)u.Rw) * (uint64_t)u.ncols;
   if constexpr (sizeof(T) >= 4) {
     if (u.C0 + lane < u.ncols) {
+      // the address moves down a row in vector registers (the asm keeps it
+      // there), and rows are only counted in a strip that ends the raster:
+      // written as offsets from the first row, a row took up to 11 scalar
+      // instructions, half of those of a strip that nothing meets
+      T* at = out + u.C0 + lane;
+      const uint64_t ncols = (uint64_t)u.ncols;
+      const int n = u.nrows - u.Rw;
+      if (n >= ROWS) {
 #pragma unroll
-      for (int r = 0; r < ROWS; ++r)
-        if (u.Rw + r < u.nrows) __builtin_nontemporal_store(p.px[r], out + (uint64_t)r * (uint64_t)u.ncols + u.C0 + lane);
+        for (int r = 0; r < ROWS; ++r) {
+          __builtin_nontemporal_store(p.px[r], at);
+          at += ncols;
+          asm volatile("" : "+v"(at));
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+          if (r < n) __builtin_nontemporal_store(p.px[r], at);
+          at += ncols;
+          asm volatile("" : "+v"(at));
+        }
+      }
     }
   } else {
     const bool part = u.C0 + tile_w(sizeof(T)) > u.ncols;
