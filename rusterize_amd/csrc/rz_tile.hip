@@ -393,9 +393,9 @@ struct CoverWave {
 // 40000 x 40000 took 0.83 ms, bound by vector issue, and take 0.65).  Small
 // items are packed: as many as have at most 64 edges and a wave's LDS words
 // together form one unit.
-// Bound by the latency of its dependent loads and LDS round trips (vector
-// issue is busy about half of the time), so LDS is sized for 6 waves per
-// SIMD, the block list's next edges are loaded ahead and its entries handed
+// Windows are bound by the latency of their dependent loads and LDS round
+// trips (vector issue is busy about half of the time), so LDS is sized for 6
+// waves per SIMD (4 of workgroups), the block list's next edges are loaded ahead and its entries handed
 // out as workgroups finish (82 M vertices in rings of up to 4,096: 1.63 ms
 // before, with the edges of crossings found through LDS, and 1.06 ms now).
 // A window of the block list reads the chunks of its item's vertices that may

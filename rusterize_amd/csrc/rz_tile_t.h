@@ -669,11 +669,11 @@ __device__ __attribute__((always_inline)) inline void bare_visits(const TileArgs
 }
 
 // Waves per SIMD the register allocation of k_tile targets: 7 for 4-byte
-// pixels (a million polygons on 40000^2 float32 in 2 bands: 5.17 ms a call,
-// in 8 bands, about one item to a tile, 12.1; with 5 waves and 6 visits ahead
-// 5.24 and 14.3), 5 for 8-byte ones (24 uneven jobs 3.85 ms, with 4 waves
-// 4.04), 3 for 2-byte ones (LineWriter's rows take the LDS of more); 4 where
-// more would spill.
+// pixels (a million polygons on 40000^2 float32 in 8 bands, about one item to
+// a tile: 10.9 ms a call, with 8 waves 11.5; with 5 waves and 6 visits ahead it
+// was 14.3 where 7 took 12.1), 5 for 8-byte ones (24 uneven jobs 3.85 ms, with
+// 4 waves 4.04), 3 for 2-byte ones (LineWriter's rows take the LDS of more); 4
+// where more would spill.
 template <typename T, bool BARE>
 struct TileOccupancy {
   static constexpr int value = sizeof(T) == 2 ? 3 : (sizeof(T) == 1 || BARE ? 4 : (sizeof(T) == 4 ? 7 : 5));
